@@ -1,0 +1,44 @@
+"""The contraction engine (``ccx_contract`` / ``ccx_contract_f32``, pycc/device.py:64-86) at the sizes where its
+kernels change path: tile edges and remainders, extents of one, odd strides, long K with small outputs
+(split K), three summed indices that do not fuse.
+
+The reference is torch's einsum in FP64 on the CPU. Tolerance: a sum of K products in any order is
+within (K + 4) u sum |a||b| of the exact one (u the unit roundoff), and so is the reference.
+"""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def contract():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import pycc_amd
+    return pycc_amd.DeviceManager('GPU', 'DP').contract
+
+
+def _check(contract, sub, ext, dtype, beta=0.0, seed=0):
+    lhs, out = sub.split("->")
+    la, lb = lhs.split(",")
+    g = torch.Generator().manual_seed(seed)
+    A, B, C = (torch.randn([ext[c] for c in l], dtype=torch.float64, generator=g).to(dtype) for l in (la, lb, out))
+    K = 1
+    for c in set(la) & set(lb) - set(out):
+        K *= ext[c]
+    ref = 0.75 * torch.einsum(sub, A.double(), B.double()) + beta * C.double()
+    mag = 0.75 * torch.einsum(sub, A.double().abs(), B.double().abs()) + abs(beta) * C.double().abs()
+    u = torch.finfo(dtype).eps
+    got = C.cuda() if beta else None
+    got = contract(sub, A.cuda(), B.cuda(), alpha=0.75, out=got, beta=beta)
+    over = ((got.cpu().double() - ref).abs() - 2 * (K + 4) * u * mag).max()
+    assert float(over) <= 0.0, (sub, ext, float(over))
+
+
+# outputs of 1 .. 200 values with long K: the split-K sums and every grouping of the reduction
+@pytest.mark.parametrize("m,n,k", [(1, 1, 9000), (13, 13, 30011), (5, 19, 4099), (67, 61, 2053), (1, 200, 777), (129, 65, 1500)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("beta", [0.0, -0.5])
+def test_split_k(contract, m, n, k, dtype, beta):
+    _check(contract, "ak,bk->ab", {"a": m, "b": n, "k": k}, dtype, beta)
