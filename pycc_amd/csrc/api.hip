@@ -119,6 +119,7 @@ int ccx_create(int no, int nv, int mode, ccx_ctx** out) {
     h->c.v = nv;
     h->c.nmo = no + nv;
     h->c.mode = mode;
+    h->c.ws.fixed_k = mode != CCX_MODE_DP;
     *out = h;
   });
 }

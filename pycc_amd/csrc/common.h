@@ -42,14 +42,15 @@ struct Idx2 {
   int64_t s1 = 0, s2 = 0;
 };
 
-// C[b][m][n] = alpha * sum_k A[b][m][k] * B[b][k][n] + beta * C[b][m][n], every operand addressed
-// through 2-level indices. Split-K partials go to `work` and are reduced by a second kernel.
+// C[b][m][n] = alpha * sum_(x,k) A[b][m][x,k] * B[b][x,k][n] + beta * C[b][m][n], every operand addressed
+// through 2-level indices and an outer third level x of K. Split-K partials go to `work` and are reduced by a second kernel.
 template <typename T>
 struct GemmParams {
   int64_t M = 0, N = 0, K = 0;
   int64_t batch = 1;
   Idx2 am, ak, bk, bn, cm, cn;
   int64_t a_b = 0, b_b = 0, c_b = 0;   // batch strides
+  int64_t kx = 1, a_x = 0, b_x = 0;    // outer third level of K: extent and strides
   T alpha = 1, beta = 0;
   const T* A = nullptr;
   const T* B = nullptr;

@@ -4,7 +4,7 @@
 // device counterpart of pycc's ContractionBackend.__call__(subscripts, *operands)
 // (pycc/device.py:64-86). Indices are classified as batch (in A, B and C), M (A and C), N (B and C)
 // or K (A and B). Indices of one class whose strides nest in every operand are fused; a class left
-// with more than two indices (more than one for batch) is looped on the host.
+// with more than two indices (three for K, one for batch) is looped on the host.
 #pragma once
 #include "common.h"
 #include "gemm.h"

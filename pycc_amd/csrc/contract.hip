@@ -210,6 +210,22 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
                  (gb.size() > 1 || gk.size() > 2 || gm.size() > 2 || gn.size() > 2) ? "  HOST-LOOP" : "");
   }
   if (gb.size() > 1) { loop_over(smallest(ob)); return; }
+  // Three K classes: the third is the GEMM's outer K level -- the one of the smallest extent that is not
+  // contiguous in an operand. (The sliced form stays where a slice alone is an FP16x3 product.)
+  Lab kx{0, 1, {0, 0, 0}};
+  if (gk.size() == 3) {
+    size_t x = 3;
+    for (int pass = 0; pass < 2 && x == 3; ++pass)
+      for (size_t y = 0; y < 3; ++y)
+        if ((pass == 1 || (gk[y].s[0] != 1 && gk[y].s[1] != 1)) && (x == 3 || gk[y].ext < gk[x].ext)) x = y;
+    std::vector<Lab> in = gk;
+    in.erase(in.begin() + x);
+    const double slice = 2.0 * (double)extent(gm) * (double)extent(gn) * (double)extent(in);
+    if (!(std::is_same<T, double>::value && split16 && slice >= X3_ROUTE_FLOPS)) {
+      kx = gk[x];
+      gk = in;
+    }
+  }
   if (gk.size() > 2) {
     // a K index is sliced by accumulating: the first slice applies beta, the rest add
     char c = smallest(ok);
@@ -233,6 +249,9 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   p.cn = make_idx(gn, in, 2);
   p.ak = make_idx(gk, ik, 0);
   p.bk = make_idx(gk, ik, 1);
+  p.kx = kx.ext;
+  p.a_x = kx.s[0];
+  p.b_x = kx.s[1];
   if (!gb.empty()) { p.a_b = gb[0].s[0]; p.b_b = gb[0].s[1]; p.c_b = gb[0].s[2]; }
   p.alpha = alpha;
   p.beta = beta;
@@ -240,7 +259,7 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   p.B = (const T*)B.p;
   p.C = (T*)C.p;
   if constexpr (std::is_same<T, double>::value) {
-    if (split16 && p.batch == 1 && 2.0 * p.M * p.N * p.K >= X3_ROUTE_FLOPS && x3_contract(p, ws, s)) return;
+    if (split16 && p.batch == 1 && p.kx == 1 && 2.0 * p.M * p.N * p.K >= X3_ROUTE_FLOPS && x3_contract(p, ws, s)) return;
   }
   tc_gemm<T>(p, ws, s);
 }

@@ -9,11 +9,16 @@ namespace ccx {
 // Grow-only device scratch owned by a context; `limit` bounds what split-K may request. A fixed
 // workspace wraps memory it does not own (size = limit): it never allocates or frees, and a request
 // beyond its size is an error.
+constexpr int FIXED_K_SPLITS = 8;
 struct Workspace {
   void* ptr = nullptr;
   size_t size = 0;
   size_t limit = size_t(1) << 30;
   bool fixed = false;
+  // FP64 sums over K in up to FIXED_K_SPLITS parts are partitioned by the shape alone, and the parts added in order: a
+  // context whose FP64 results become FP32 or split FP16 operands then rounds the same operands however a
+  // launch is planned.
+  bool fixed_k = false;
   static Workspace wrap(void* p, size_t bytes) {
     Workspace w;
     w.ptr = p;

@@ -48,213 +48,360 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t w, int64_t ntiles) {
   return x * q + (x < r ? x : r) + j;
 }
 
-// LDS tile of one operand: stored [rows][BK + 1] when the operand is loaded along k (k-fast) and
-// [BK][rows + 1] when it is loaded along m / n. The +1 shifts consecutive rows by two 4-byte banks,
-// so neither the stores nor the MFMA fragment reads conflict.
-template <typename T, int R, int BK, bool KFAST>
-struct LdsTile {
-  T d[KFAST ? R : BK][(KFAST ? BK : R) + 1];
-  __device__ __forceinline__ T& at(int r, int k) { return KFAST ? d[r][k] : d[k][r]; }
+// ---- the tile kernel -------------------------------------------------------------------------------
+// C[b][m][n] = alpha sum_(x, k) A[b][m][x, k] B[b][x, k][n] + beta C: M, N and K are 2-level indices, x an
+// outer third level of K (its strides a_x, b_x), b the batch.
+//
+// What bounds it: a 16x16x4 FP64 MFMA holds a SIMD for 64 cycles, so a k-tile of a 128 x 128 tile is 8192
+// matrix cycles per CU against 16 8-byte loads per thread: the matrix cores, as long as some wave always has
+// one to issue. Hence 8 waves of 64 x 32 per work-group and two work-groups per CU (4 waves per SIMD, 128
+// registers), where 4 waves of 64 x 64 (2 per SIMD) stand still at every barrier; and hence plain 8-byte
+// loads whose addresses come from a multiply-high division per k index: any strides, odd extents and
+// remainders run the same loop. Rows past M or N read row M - 1 or N - 1 (their outputs are not stored); k past
+// its end reads the last k and is zeroed on its way into LDS.
+//
+// LDS: a k-fast tile is [rows][BK + 2] (FP32: BK + 1) and a row-fast one [BK][rows + 16]: the two k rows of a half wave's
+// fragment read start 4 (k-fast: rows start 36 banks) or 32 banks apart, so reads are free of conflicts.
+
+// i / d for 0 <= i < 2^31 by multiply-high (d >= 1).
+struct FastIdx {
+  uint32_t n2, mul, sh;
+  int64_t s1, s2;
+};
+static FastIdx fast_idx(const Idx2& x) {
+  FastIdx f;
+  CCX_CHECK(x.n2 >= 1 && x.n2 < (1ll << 31), ERR_INTERNAL, "index extent");
+  f.n2 = (uint32_t)x.n2;
+  f.sh = 0;
+  while ((1ull << f.sh) < f.n2) ++f.sh;
+  f.mul = (uint32_t)((((1ull << f.sh) - f.n2) << 32) / f.n2 + 1);
+  f.s1 = x.s1;
+  f.s2 = x.s2;
+  return f;
+}
+__device__ __forceinline__ int64_t off2(const FastIdx& d, uint32_t i) {
+  const uint32_t q = (__umulhi(i, d.mul) + i) >> d.sh;
+  const uint32_t r = i - q * d.n2;
+  return (int64_t)q * d.s1 + (int64_t)r * d.s2;
+}
+
+template <typename T>
+struct TileGemm {
+  int M, N, K, kx, splits, chunk;   // chunk: k-tiles per split, counted over x and k
+  FastIdx am, ak, bk, bn, cm, cn;
+  int64_t a_x, b_x, a_b, b_b, c_b;
+  T alpha, beta;
+  const T* A;
+  const T* B;
+  T* C;
+  T* work;   // [split][batch][M][N] partial sums when splits > 1
 };
 
-// Loader of one operand tile (R rows x BK k's) from a 2-level-indexed global array. Each thread
-// owns NE = R * BK / 256 elements: k-fast -> one k column and NE rows; otherwise one row, NE k's.
-template <typename T, int R, int BK, bool KFAST>
-struct TileLoader {
-  static constexpr int NT = 256;
-  static constexpr int NE = R * BK / NT;
-  int kl, rl;                      // local coordinates of the thread's first element
-  int64_t roff[KFAST ? NE : 1];    // global offsets of the thread's rows
-  bool rok[KFAST ? NE : 1];
-  T v[NE];
+// two doubles in LDS
+struct alignas(16) Two {
+  double x, y;
+};
+// two neighbouring doubles in memory: 8-byte aligned, read by one 16-byte load
+struct __attribute__((packed, aligned(8))) TwoIn {
+  double x, y;
+};
 
-  __device__ __forceinline__ void init(const Idx2& rix, int64_t row0, int64_t nrows, int tid) {
-    if (KFAST) {
-      kl = tid % BK; rl = tid / BK;
+// One operand's tile, and its fragments: MFMA step s of a 16-wide k-tile holds k = 4 s + lane / 16, so every sum runs
+// over k upwards whatever the tile.
+template <typename T, int R, int BK, bool KF>
+struct GTile {
+  alignas(16) T d[KF ? R : BK][KF ? BK + (sizeof(T) == 8 ? 2 : 1) : R + 16];
+  __device__ __forceinline__ T& at(int r, int k) { return KF ? d[r][k] : d[k][r]; }
+  // f[h][b]: row r0 + 16 b + fc, MFMA step k8 / 4 + h
+  template <int NB>
+  __device__ __forceinline__ void frags(T (&f)[2][NB], int r0, int k8, int fr, int fc) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) f[h][b] = at(r0 + 16 * b + fc, k8 + 4 * h + fr);
+  }
+};
+
+// One operand's loader: a thread owns NE pieces of V values of the R x BK tile, V along k (k-fast) or along the
+// rows; k-fast: one k and NE rows, else one row piece and NE k's. Addresses are a uniform base plus a lane
+// offset in bytes (Off: 32 bits where the operand spans less than 4 GiB), k by an odometer over its (n2, s1, s2):
+// a k-tile costs a lane one step of it and an add per load. Where a whole wave holds one k (row-fast, V R >= 64
+// lanes) that k stays in scalar registers.
+// V = 2 reads 16 bytes at a time. It needs the inner index contiguous and pairs that do not straddle its blocks: an
+// even n2 or a single level. An odd extent ends in a pair that starts one early (`late`: its second half counts).
+template <typename T, int R, int BK, bool KF, int NT, typename Off, int V>
+struct GLoader {
+  static constexpr int LANES = (KF ? BK : R) / V;   // pieces along the contiguous index
+  static constexpr int NE = R * BK / V / NT, STEP = NT / LANES;
+  static constexpr bool UK = !KF && LANES >= 64;    // k uniform in a wave
+  static constexpr int NO = KF || UK ? 1 : NE;      // odometers
+  int kl, rl;
+  Off roff[KF ? NE : 1], koff[NO];
+  uint32_t kr[NO];
+  bool row_late;
+  // one k-tile's values on their way to LDS
+  struct Load {
+    T v[NE][V];
+    uint32_t ok;   // bit i: piece i's k is inside
+    bool late, whole;
+  };
+  __device__ __forceinline__ void init(const FastIdx& rix, int row0, int nrows, int tid) {
+    const int along = tid % LANES * V, across = tid / LANES;
+    kl = KF ? along : UK ? __builtin_amdgcn_readfirstlane(across) : across;
+    rl = KF ? across : along;
+    row_late = false;
+#pragma unroll
+    for (int i = 0; i < (KF ? NE : 1); ++i) {
+      int r = row0 + rl + i * STEP;
+      if (!KF && V == 2) row_late = r == nrows - 1;
+      r = r < nrows - (KF ? 1 : V) ? r : nrows - (KF ? 1 : V);
+      roff[i] = (Off)(off2(rix, (uint32_t)r) * (int64_t)sizeof(T));
+    }
+  }
+  __device__ __forceinline__ void seek(const FastIdx& kix, int k0) {
+    if (UK) return;
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      const uint32_t k = (uint32_t)(k0 + kl + i * STEP), q = (__umulhi(k, kix.mul) + k) >> kix.sh;
+      kr[i] = k - q * kix.n2;
+      koff[i] = (Off)(((int64_t)q * kix.s1 + (int64_t)kr[i] * kix.s2) * (int64_t)sizeof(T));
+    }
+  }
+  __device__ __forceinline__ void step(const FastIdx& kix, int k0) {   // BK further, to the tile at k0
+    if (UK) return;
+    if (kix.n2 < (uint32_t)BK) {
+      seek(kix, k0);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      kr[i] += BK;
+      koff[i] += (Off)(BK * kix.s2 * (int64_t)sizeof(T));
+      if (kr[i] >= kix.n2) {
+        kr[i] -= kix.n2;
+        koff[i] += (Off)((kix.s1 - (int64_t)kix.n2 * kix.s2) * (int64_t)sizeof(T));
+      }
+    }
+  }
+  static __device__ __forceinline__ void get(T (&v)[V], const char* p) {
+    if constexpr (V == 2) {
+      const TwoIn q = *(const TwoIn*)p;
+      v[0] = q.x;
+      v[1] = q.y;
+    } else {
+      v[0] = *(const T*)p;
+    }
+  }
+  // rows_in: every row of the tile is inside
+  __device__ __forceinline__ void load(Load& l, const T* __restrict__ base, const FastIdx& kix, int k0, int K,
+                                       bool rows_in) {
+    l.ok = 0;
+    l.late = row_late;
+    l.whole = rows_in && k0 + BK <= K;
+    if constexpr (KF) {
+      const int k = k0 + kl;
+      Off ko = koff[0];
+      if (V == 2) l.late = k == K - 1;
+      if (k > K - V) ko = V == 2 && k < K ? ko - (Off)sizeof(T) : 0;
+      if (k < K) l.ok = ~0u;
+#pragma unroll
+      for (int i = 0; i < NE; ++i) get(l.v[i], (const char*)base + (Off)(roff[i] + ko));
+    } else {
 #pragma unroll
       for (int i = 0; i < NE; ++i) {
-        int64_t r = row0 + rl + i * (NT / BK);
-        rok[i] = r < nrows;
-        roff[i] = rok[i] ? off2(rix, r) : 0;
+        const int k = k0 + kl + i * STEP;
+        if (k < K) l.ok |= 1u << i;
+        if constexpr (UK) get(l.v[i], (const char*)(base + off2(kix, (uint32_t)(k < K ? k : K - 1))) + roff[0]);
+        else get(l.v[i], (const char*)base + (Off)(roff[0] + (k < K ? koff[i] : (Off)0)));
       }
-    } else {
-      rl = tid % R; kl = tid / R;
-      int64_t r = row0 + rl;
-      rok[0] = r < nrows;
-      roff[0] = rok[0] ? off2(rix, r) : 0;
     }
   }
-  // Unguarded load of a k-tile that lies inside one k1 block (kix.n2 % BK == 0) and whose rows are
-  // all valid: one offset computation per tile, then constant strides.
-  __device__ __forceinline__ void load_fast(const T* __restrict__ base, const Idx2& kix, int64_t k0) {
-    const int64_t kb = off2(kix, k0);
-    if (KFAST) {
-      const int64_t ko = kb + (int64_t)kl * kix.s2;
-#pragma unroll
-      for (int i = 0; i < NE; ++i) v[i] = base[roff[i] + ko];
-    } else {
-#pragma unroll
-      for (int i = 0; i < NE; ++i) v[i] = base[roff[0] + kb + (int64_t)(kl + i * (NT / R)) * kix.s2];
-    }
+  __device__ __forceinline__ void put(const T (&x)[V], int i, GTile<T, R, BK, KF>& t) {
+    T* dst = KF ? &t.at(rl + i * STEP, kl) : &t.at(rl, kl + i * STEP);
+    if constexpr (V == 2) *(Two*)dst = Two{x[0], x[1]};
+    else *dst = x[0];
   }
-  // Guarded load for edge tiles / k-tiles that straddle a k1 block.
-  __device__ __forceinline__ void load_safe(const T* __restrict__ base, const Idx2& kix, int64_t k0, int64_t kend) {
-    if (KFAST) {
-      int64_t k = k0 + kl;
-      bool kok = k < kend;
-      int64_t ko = kok ? off2(kix, k) : 0;
+  __device__ __forceinline__ void store(const Load& l, GTile<T, R, BK, KF>& t) {
+    if (l.whole) {
 #pragma unroll
-      for (int i = 0; i < NE; ++i) v[i] = (kok && rok[i]) ? base[roff[i] + ko] : T(0);
+      for (int i = 0; i < NE; ++i) put(l.v[i], i, t);
     } else {
+      asm volatile("");   // keeps this a branch (it is uniform): as selects it would cost every k-tile
 #pragma unroll
       for (int i = 0; i < NE; ++i) {
-        int64_t k = k0 + kl + i * (NT / R);
-        v[i] = (rok[0] && k < kend) ? base[roff[0] + off2(kix, k)] : T(0);
+        const bool in = (l.ok >> i) & 1u, late = V == 2 && l.late;
+        T x[V];
+        x[0] = in ? (late ? l.v[i][V - 1] : l.v[i][0]) : T(0);
+        if (V == 2) x[V - 1] = in && !late ? l.v[i][V - 1] : T(0);
+        put(x, i, t);
       }
-    }
-  }
-  __device__ __forceinline__ void store(LdsTile<T, R, BK, KFAST>& t) {
-    if (KFAST) {
-#pragma unroll
-      for (int i = 0; i < NE; ++i) t.at(rl + i * (NT / BK), kl) = v[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < NE; ++i) t.at(rl, kl + i * (NT / R)) = v[i];
     }
   }
 };
 
-template <typename T, int BM, int BN, int BK, bool A_KFAST, bool B_KFAST>
-__global__ __launch_bounds__(256, 2) void tc_gemm_kernel(GemmParams<T> p, T* __restrict__ work,
-                                                         int splits, int64_t kchunk) {
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int NBI = WM / 16, NBJ = WN / 16;
+template <typename T, int BM, int BN, int WM, int WN, int BK, bool AKF, bool BKF, typename Off, int V>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kernel(TileGemm<T> p) {
+  constexpr int NWN = BN / WN, NT = 64 * (BM / WM) * NWN, NBI = WM / 16, NBJ = WN / 16;
   typedef typename AccT<T>::type acc_t;
+  __shared__ GTile<T, BM, BK, AKF> As[2];
+  __shared__ GTile<T, BN, BK, BKF> Bs[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / NWN, wn = wave % NWN;
 
-  __shared__ LdsTile<T, BM, BK, A_KFAST> As[2];
-  __shared__ LdsTile<T, BN, BK, B_KFAST> Bs[2];
+  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
+  const int64_t t = xcd_remap(blockIdx.x, (int64_t)tiles_m * tiles_n);
+  // 8 tile-rows together, so that concurrently running tiles share A and B panels
+  const int64_t group = t / (8 * tiles_n);
+  const int first_m = (int)group * 8, gsize = tiles_m - first_m < 8 ? tiles_m - first_m : 8;
+  const int within = (int)(t - group * 8 * tiles_n);
+  const int m0 = (first_m + within % gsize) * BM, n0 = within / gsize * BN;
+  const int bidx = blockIdx.y / p.splits, sidx = blockIdx.y % p.splits;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int ntk = (p.K + BK - 1) / BK;   // k-tiles of one x
+  int kt = sidx * p.chunk;               // first and end k-tile of this split, over x and k
+  const int kt_end = kt + p.chunk < ntk * p.kx ? kt + p.chunk : ntk * p.kx;
+  const int x0 = ntk ? kt / ntk : 0;
+  int k0 = (kt - x0 * ntk) * BK;
+  const T* __restrict__ A = p.A + bidx * p.a_b + x0 * p.a_x;
+  const T* __restrict__ B = p.B + bidx * p.b_b + x0 * p.b_x;
 
-  const int64_t tiles_m = ceil_div(p.M, BM), tiles_n = ceil_div(p.N, BN);
-  const int64_t ntiles = tiles_m * tiles_n;
-  int64_t t = xcd_remap(blockIdx.x, ntiles);
-  // group 8 tile-rows together so that concurrently running tiles share A and B panels
-  const int64_t GM = 8;
-  int64_t group = t / (GM * tiles_n);
-  int64_t first_m = group * GM;
-  int64_t gsize = tiles_m - first_m < GM ? tiles_m - first_m : GM;
-  int64_t within = t - group * GM * tiles_n;
-  const int64_t tm = first_m + within % gsize;
-  const int64_t tn = within / gsize;
-
-  const int64_t bz = blockIdx.y;
-  const int64_t bidx = bz / splits, sidx = bz - bidx * splits;
-  const int64_t k_begin = sidx * kchunk;
-  const int64_t k_end = (k_begin + kchunk < p.K) ? k_begin + kchunk : p.K;
-
-  const T* __restrict__ Ab = p.A + bidx * p.a_b;
-  const T* __restrict__ Bb = p.B + bidx * p.b_b;
-
-  TileLoader<T, BM, BK, A_KFAST> la;
-  TileLoader<T, BN, BK, B_KFAST> lb;
-  la.init(p.am, tm * BM, p.M, tid);
-  lb.init(p.bn, tn * BN, p.N, tid);
-  // interior tile whose k-tiles never straddle a k1 block: unguarded loads
-  const bool fast = (tm + 1) * BM <= p.M && (tn + 1) * BN <= p.N && (p.ak.n2 % BK == 0) &&
-                    (k_begin % BK == 0);
+  GLoader<T, BM, BK, AKF, NT, Off, V> la;
+  GLoader<T, BN, BK, BKF, NT, Off, V> lb;
+  la.init(p.am, m0, p.M, tid);
+  lb.init(p.bn, n0, p.N, tid);
 
   acc_t acc[NBI][NBJ];
 #pragma unroll
   for (int i = 0; i < NBI; ++i)
 #pragma unroll
     for (int j = 0; j < NBJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  const int fr = lane >> 4, fc = lane & 15;
+  const bool m_in = m0 + BM <= p.M, n_in = n0 + BN <= p.N;
 
-  const int fr = lane >> 4;   // k row within an MFMA step
-  const int fc = lane & 15;   // m / n column within a 16-wide block
-  // output row of register r within a 16x16 block (see the layout note at the top)
-  auto orow = [&](int r) { return sizeof(T) == 8 ? 4 * r + fr : 4 * fr + r; };
-
-  auto load = [&](int64_t k0) {
-    if (fast && k0 + BK <= k_end) {
-      la.load_fast(Ab, p.ak, k0);
-      lb.load_fast(Bb, p.bk, k0);
-    } else {
-      la.load_safe(Ab, p.ak, k0, k_end);
-      lb.load_safe(Bb, p.bk, k0, k_end);
-    }
-  };
-
-  if (k_begin < k_end) {
-    load(k_begin);
-    la.store(As[0]);
-    lb.store(Bs[0]);
+  if (kt < kt_end) {
+    typename decltype(la)::Load va;
+    typename decltype(lb)::Load vb;
+    la.seek(p.ak, k0);
+    lb.seek(p.bk, k0);
+    auto load = [&] {
+      la.load(va, A, p.ak, k0, p.K, m_in);
+      lb.load(vb, B, p.bk, k0, p.K, n_in);
+    };
+    // to the next k-tile; past the last one the last is loaded again (no branch around the loads)
+    auto next = [&] {
+      if (kt + 1 >= kt_end) return;
+      k0 += BK;
+      if (k0 >= p.K) {
+        k0 = 0;
+        A += p.a_x;
+        B += p.b_x;
+        la.seek(p.ak, 0);
+        lb.seek(p.bk, 0);
+      } else {
+        la.step(p.ak, k0);
+        lb.step(p.bk, k0);
+      }
+    };
+    load();
+    la.store(va, As[0]);
+    lb.store(vb, Bs[0]);
     __syncthreads();
-    int buf = 0;
-    for (int64_t k0 = k_begin; k0 < k_end; k0 += BK) {
-      const bool has_next = k0 + BK < k_end;
-      if (has_next) load(k0 + BK);
+    // one k-tile, from LDS buffer `buf` (a constant where it is called: LDS addresses stay immediate offsets)
+    auto body = [&](int buf) {
+      next();
+      load();
+      // small wave tiles read the whole k-tile's fragments first; large ones have no registers for that, and more
+      // waves to fill the gaps
+      constexpr int KG = WM * WN <= 1024 ? BK : 8;
 #pragma unroll
-      for (int ks = 0; ks < BK; ks += 4) {
-        T a[NBI], b[NBJ];
+      for (int kg = 0; kg < BK; kg += KG) {
+        T a[KG / 8][2][NBI], b[KG / 8][2][NBJ];
 #pragma unroll
-        for (int i = 0; i < NBI; ++i) a[i] = As[buf].at(wm * WM + i * 16 + fc, ks + fr);
+        for (int g = 0; g < KG / 8; ++g) {
+          As[buf].frags(a[g], wm * WM, kg + 8 * g, fr, fc);
+          Bs[buf].frags(b[g], wn * WN, kg + 8 * g, fr, fc);
+        }
+        if (KG == BK) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NBJ; ++j) b[j] = Bs[buf].at(wn * WN + j * 16 + fc, ks + fr);
+        for (int g = 0; g < KG / 8; ++g)
 #pragma unroll
-        for (int i = 0; i < NBI; ++i)
+          for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int j = 0; j < NBJ; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+            for (int i = 0; i < NBI; ++i)
+#pragma unroll
+              for (int j = 0; j < NBJ; ++j) acc[i][j] = mfma16(a[g][h][i], b[g][h][j], acc[i][j]);
       }
-      if (has_next) {
-        la.store(As[buf ^ 1]);
-        lb.store(Bs[buf ^ 1]);
-      }
+      la.store(va, As[buf ^ 1]);
+      lb.store(vb, Bs[buf ^ 1]);
       __syncthreads();
-      buf ^= 1;
+      ++kt;
+    };
+    while (kt + 1 < kt_end) {
+      body(0);
+      body(1);
     }
+    if (kt < kt_end) body(0);
   }
 
-  // ---- epilogue ----
-  if (splits == 1) {
-    T* Cb = p.C + bidx * p.c_b;
+  // output row of register r within a 16x16 block (see the layout note at the top)
+  auto row = [&](int i, int r) { return m0 + wm * WM + i * 16 + (sizeof(T) == 8 ? 4 * r + fr : 4 * fr + r); };
+  if (p.splits == 1) {
+    T* C = p.C + bidx * p.c_b;
 #pragma unroll
-    for (int j = 0; j < NBJ; ++j) {
-      int64_t n = tn * BN + wn * WN + j * 16 + fc;
-      if (n >= p.N) continue;
-      int64_t no = off2(p.cn, n);
+    for (int i = 0; i < NBI; ++i)
 #pragma unroll
-      for (int i = 0; i < NBI; ++i) {
+      for (int r = 0; r < 4; ++r) {
+        const int m = row(i, r);
+        if (m >= p.M) continue;
+        T* Cm = C + off2(p.cm, (uint32_t)m);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int64_t m = tm * BM + wm * WM + i * 16 + orow(r);
-          if (m >= p.M) continue;
-          T* dst = Cb + off2(p.cm, m) + no;
+        for (int j = 0; j < NBJ; ++j) {
+          const int n = n0 + wn * WN + j * 16 + fc;
+          if (n >= p.N) continue;
+          T* dst = Cm + off2(p.cn, (uint32_t)n);
           T v = p.alpha * acc[i][j][r];
           if (p.beta != T(0)) v += p.beta * *dst;
           *dst = v;
         }
       }
-    }
   } else {
-    // dense partial tile: work[s][b][m][n]
-    T* Wb = work + (sidx * p.batch + bidx) * p.M * p.N;
+    T* W = p.work + ((int64_t)sidx * (gridDim.y / p.splits) + bidx) * p.M * p.N;
 #pragma unroll
-    for (int j = 0; j < NBJ; ++j) {
-      int64_t n = tn * BN + wn * WN + j * 16 + fc;
-      if (n >= p.N) continue;
+    for (int i = 0; i < NBI; ++i)
 #pragma unroll
-      for (int i = 0; i < NBI; ++i)
+      for (int r = 0; r < 4; ++r) {
+        const int m = row(i, r);
+        if (m >= p.M) continue;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int64_t m = tm * BM + wm * WM + i * 16 + orow(r);
-          if (m < p.M) Wb[m * p.N + n] = acc[i][j][r];
+        for (int j = 0; j < NBJ; ++j) {
+          const int n = n0 + wn * WN + j * 16 + fc;
+          if (n < p.N) W[(int64_t)m * p.N + n] = acc[i][j][r];
         }
-    }
+      }
   }
+}
+
+template <typename T, int BM, int BN, int WM, int WN, typename Off, int V>
+static void launch_tile(const TileGemm<T>& p, int64_t batch, bool akf, bool bkf, hipStream_t s) {
+  constexpr int BK = 16, NT = 64 * (BM / WM) * (BN / WN);
+  const dim3 grid((unsigned)(ceil_div(p.M, BM) * ceil_div(p.N, BN)), (unsigned)(batch * p.splits));
+  if (akf && bkf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, true, true, Off, V><<<grid, NT, 0, s>>>(p);
+  else if (akf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, true, false, Off, V><<<grid, NT, 0, s>>>(p);
+  else if (bkf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, false, true, Off, V><<<grid, NT, 0, s>>>(p);
+  else tile_gemm_kernel<T, BM, BN, WM, WN, BK, false, false, Off, V><<<grid, NT, 0, s>>>(p);
+  CCX_HIP(hipGetLastError());
+}
+
+template <typename T, typename Off, int V>
+static void launch_tile(int tile, const TileGemm<T>& p, int64_t batch, bool akf, bool bkf, hipStream_t s) {
+  if (tile == 64) launch_tile<T, 64, 64, 32, 32, Off, V>(p, batch, akf, bkf, s);
+  else launch_tile<T, 128, 128, 64, 32, Off, V>(p, batch, akf, bkf, s);
+}
+
+// Largest element offset of a 2-level index over `extent` values; negative when a stride is.
+static int64_t span(const Idx2& d, int64_t extent) {
+  if (d.s1 < 0 || d.s2 < 0) return -1;
+  const int64_t q = (extent - 1) / d.n2;
+  return q * d.s1 + (std::min(extent, d.n2) - 1) * d.s2;
 }
 
 // C = alpha * sum_s work[s] + beta * C, in a fixed summation order (deterministic).
@@ -314,7 +461,7 @@ static void splitk_reduce(const GemmParams<T>& p, const T* work, int splits, hip
   const int64_t waves = ceil_div(total, 64);
   if (sizeof(T) == 8 && waves < 256 && splits >= 32)
     splitk_reduce_kernel<T, 16><<<(unsigned)waves, 1024, 0, s>>>(p, work, splits);
-  else if (sizeof(T) == 8 && waves < 1024 && splits >= 8)
+  else if (sizeof(T) == 8 && waves < 1024 && splits > FIXED_K_SPLITS)
     splitk_reduce_kernel<T, 4><<<(unsigned)waves, 256, 0, s>>>(p, work, splits);
   else
     splitk_reduce_kernel<T, 1><<<(unsigned)ceil_div(total, 256), 256, 0, s>>>(p, work, splits);
@@ -368,18 +515,6 @@ static void plain_dispatch(const PlainGemm<T>& q, Workspace& ws, hipStream_t s) 
   splitk_reduce<T>(r, work, (int)splits, s);
 }
 
-template <typename T, int BM, int BN, int BK>
-static void launch_tiles(const GemmParams<T>& p, bool akf, bool bkf, T* work, int splits,
-                         int64_t kchunk, hipStream_t s) {
-  int64_t ntiles = ceil_div(p.M, BM) * ceil_div(p.N, BN);
-  dim3 grid((unsigned)ntiles, (unsigned)(p.batch * splits));
-  if (akf && bkf) tc_gemm_kernel<T, BM, BN, BK, true, true><<<grid, 256, 0, s>>>(p, work, splits, kchunk);
-  else if (akf) tc_gemm_kernel<T, BM, BN, BK, true, false><<<grid, 256, 0, s>>>(p, work, splits, kchunk);
-  else if (bkf) tc_gemm_kernel<T, BM, BN, BK, false, true><<<grid, 256, 0, s>>>(p, work, splits, kchunk);
-  else tc_gemm_kernel<T, BM, BN, BK, false, false><<<grid, 256, 0, s>>>(p, work, splits, kchunk);
-  CCX_HIP(hipGetLastError());
-}
-
 // Single stride of a 2-level index over `extent` values, or -1 when it is not a plain stride.
 static int64_t plain_stride(const Idx2& d, int64_t extent) {
   if (extent <= 1) return 0;
@@ -420,57 +555,149 @@ static bool as_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
   return plain_gemm_ok(q);
 }
 
+// Tile and split count of an FP64 contraction: the cheapest of both tiles and a few split counts under a model of
+// the launch fitted to M x N x 1313 products of 1, 2 and 3 tiles per CU (64 x 64: 68, 115, 158 us) and to 8192^3
+// (128 x 128: 18 ms): a k-tile costs 0.25 us a round of resident work-groups plus its flops at 0.24 TF a CU,
+// a launch 6 us; partial sums move at 4 TB/s behind a launch of 5 us. At o=13 v=101 an ov x ov x ov product
+// takes 121 tiles of 128 x 128 split in 9 171 us, 441 tiles of 64 x 64 unsplit 122.
+struct Plan {
+  int tile = 128, splits = 1, chunk = 0;
+};
+static Plan plan_f64(const GemmParams<double>& p, size_t limit) {
+  static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128, 192, 256};
+  const int64_t ntk = std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx);
+  Plan best;
+  double t_best = 0.0;
+  for (int tile : {128, 64}) {
+    const int64_t tiles = ceil_div(p.M, tile) * ceil_div(p.N, tile) * p.batch;
+    const double t_ktile = 2.0 * tile * tile * 16 / 0.24e6;
+    const int per_cu = tile == 128 ? 2 : 4;   // resident work-groups (LDS)
+    for (int want : counts) {
+      const int64_t chunk = ceil_div(ntk, want), splits = ceil_div(ntk, chunk);
+      if (want > 1 && (chunk < 4 || splits * p.batch > 65535)) break;
+      const double bytes = 8.0 * (double)splits * (double)p.batch * (double)p.M * (double)p.N;
+      if (want > 1 && bytes > (double)limit) break;
+      const int64_t on_cu = ceil_div(tiles * splits, 256);
+      double t = 6.0 + (double)chunk * (0.25 * (double)ceil_div(on_cu, per_cu) + (double)on_cu * t_ktile);
+      if (splits > 1) t += 5.0 + 2.0 * bytes / 4.0e6;
+      if (t_best == 0.0 || t < t_best) {
+        t_best = t;
+        best.tile = tile;
+        best.splits = (int)splits;
+        best.chunk = (int)chunk;
+      }
+    }
+  }
+  return best;
+}
+
+// The K partition by the shape alone, where it is part of the result: FP32 sums, and FP64 sums that are rounded to FP32
+// or split FP16 operands. About 1024 work-groups, at least 8 k-tiles per split, at most 256 splits.
+template <typename T>
+static Plan plan_fixed(const GemmParams<T>& p, size_t limit) {
+  Plan r;
+  r.tile = p.M <= 64 || p.N <= 64 ? 64 : 128;
+  const int64_t ntk = ceil_div(p.K, 16) * p.kx;
+  const int64_t tiles = ceil_div(p.M, r.tile) * ceil_div(p.N, r.tile) * p.batch;
+  int64_t splits = 1, kchunk = p.K;
+  if (p.K > 0 && tiles < 1024) {
+    splits = std::max<int64_t>(1, std::min<int64_t>(ceil_div(1024, tiles), std::min<int64_t>(p.K * p.kx / 128, 256)));
+    splits = std::max<int64_t>(1, std::min<int64_t>(splits, 65535 / p.batch));
+  }
+  if (splits > 1) {
+    kchunk = ceil_div(ntk, splits);
+    splits = ceil_div(ntk, kchunk);
+    const size_t one = (size_t)p.batch * p.M * p.N * sizeof(T);
+    if ((size_t)splits * one > limit) {   // keep the workspace bounded; fall back to fewer splits
+      splits = (int64_t)std::max<size_t>(1, limit / one);
+      kchunk = ceil_div(ntk, splits);
+      splits = ceil_div(ntk, kchunk);
+    }
+  }
+  if (splits <= 1) kchunk = ntk;
+  r.splits = (int)std::max<int64_t>(splits, 1);
+  r.chunk = (int)kchunk;
+  return r;
+}
+static Plan plan(const GemmParams<float>& p, const Workspace& ws) { return plan_fixed(p, ws.limit); }
+static Plan plan(const GemmParams<double>& p, const Workspace& ws) {
+  if (ws.fixed_k) {
+    Plan f = plan_fixed(p, ws.limit);
+    if (f.splits <= FIXED_K_SPLITS) {   // the tile is free
+      if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch * f.splits < 512) f.tile = 64;
+      return f;
+    }
+  }
+  return plan_f64(p, ws.limit);
+}
+
 template <typename T>
 void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
   {
     // enough 128 x 128 tiles to fill the 256 CUs: the plain-matrix kernel
     PlainGemm<T> q;
-    if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q)) {
+    if (p.kx == 1 && ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q)) {
       plain_dispatch<T>(q, ws, s);
       return;
     }
   }
-  CCX_CHECK(p.M < (1ll << 31) && p.N < (1ll << 31) && p.K < (1ll << 31), ERR_ARG, "gemm extent too large");
+  CCX_CHECK(p.M < (1ll << 31) && p.N < (1ll << 31) && p.K < (1ll << 31) && p.K * p.kx < (1ll << 31), ERR_ARG,
+            "gemm extent too large");
   CCX_CHECK(p.batch < 65536, ERR_ARG, "gemm batch too large");
   // A is "k-fast" when its inner k index is contiguous (coalesced loads along k); otherwise the
   // loader walks along m. Same for B with n.
   const bool akf = !(p.am.s2 == 1 && p.ak.s2 != 1);
   const bool bkf = !(p.bn.s2 == 1 && p.bk.s2 != 1);
-  const bool small = p.M <= 64 || p.N <= 64;
-  const int BM = small ? 64 : 128, BN = small ? 64 : 128, BKt = 16;
-  int64_t tiles = ceil_div(p.M, BM) * ceil_div(p.N, BN) * p.batch;
-  CCX_CHECK(tiles < (1ll << 31), ERR_ARG, "gemm grid too large");
-  // split K when the tile grid cannot fill the 256 CUs and K is long
-  int splits = 1;
-  if (p.K > 0 && tiles < 1024) {
-    // fill ~4 workgroups per CU; every split keeps at least 8 k-tiles
-    int64_t want = ceil_div(1024, tiles);
-    int64_t maxs = p.K / (BKt * 8);
-    splits = (int)std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(maxs, 256)));
-    splits = (int)std::max<int64_t>(1, std::min<int64_t>(splits, 65535 / p.batch));   // grid.y limit
-  }
-  int64_t kchunk = p.K;
-  T* work = nullptr;
-  if (splits > 1) {
-    kchunk = ceil_div(ceil_div(p.K, splits), BKt) * BKt;
-    splits = (int)ceil_div(p.K, kchunk);
-    size_t bytes = (size_t)splits * p.batch * p.M * p.N * sizeof(T);
-    if (bytes > ws.limit) {       // keep the workspace bounded; fall back to fewer splits
-      splits = (int)std::max<int64_t>(1, ws.limit / ((size_t)p.batch * p.M * p.N * sizeof(T)));
-      kchunk = ceil_div(ceil_div(p.K, splits), BKt) * BKt;
-      splits = (int)ceil_div(p.K, kchunk);
-    }
-    if (splits > 1) work = (T*)ws.get((size_t)splits * p.batch * p.M * p.N * sizeof(T));
-    else kchunk = p.K;
-  }
-  if (p.K == 0) kchunk = 0;
+  const Plan pl = plan(p, ws);
+  CCX_CHECK(ceil_div(p.M, pl.tile) * ceil_div(p.N, pl.tile) < (1ll << 31), ERR_ARG, "gemm grid too large");
+  TileGemm<T> g;
+  g.M = (int)p.M;
+  g.N = (int)p.N;
+  g.K = (int)p.K;
+  g.kx = (int)p.kx;
+  g.splits = pl.splits;
+  g.chunk = pl.chunk;
+  g.am = fast_idx(p.am);
+  g.ak = fast_idx(p.ak);
+  g.bk = fast_idx(p.bk);
+  g.bn = fast_idx(p.bn);
+  g.cm = fast_idx(p.cm);
+  g.cn = fast_idx(p.cn);
+  g.a_x = p.a_x;
+  g.b_x = p.b_x;
+  g.a_b = p.a_b;
+  g.b_b = p.b_b;
+  g.c_b = p.c_b;
+  g.alpha = p.alpha;
+  g.beta = p.beta;
+  g.A = p.A;
+  g.B = p.B;
+  g.C = p.C;
+  g.work = pl.splits > 1 ? (T*)ws.get((size_t)pl.splits * p.batch * p.M * p.N * sizeof(T)) : nullptr;
   if (std::getenv("CCX_TRACE"))
-    std::fprintf(stderr, "[ccx]   -> generic %s tile%s%s batch %lld splits %d\n", small ? "64" : "128", akf ? " Ak" : " Am",
-                 bkf ? " Bk" : " Bn", (long long)p.batch, splits);
-  if (small) launch_tiles<T, 64, 64, 16>(p, akf, bkf, work, splits, kchunk, s);
-  else launch_tiles<T, 128, 128, 16>(p, akf, bkf, work, splits, kchunk, s);
-  if (splits > 1) splitk_reduce<T>(p, work, splits, s);
+    std::fprintf(stderr, "[ccx]   -> tile %d%s%s batch %lld splits %d\n", pl.tile, akf ? " Ak" : " Am",
+                 bkf ? " Bk" : " Bn", (long long)p.batch, pl.splits);
+  // lane offsets in 32 bits: what a lane adds to the uniform base stays under 4 GiB -- the rows, and k where it is
+  // not the same in a whole wave (k-fast, and pairs of rows in a 64-wide tile)
+  auto narrow = [&](const Idx2& r, int64_t nr, const Idx2& k, bool with_k) {
+    const int64_t a = span(r, nr), b = with_k ? span(k, std::max<int64_t>(p.K, 1)) : 0;
+    return a >= 0 && b >= 0 && (a + b + 1) * (int64_t)sizeof(T) <= (1ll << 32);
+  };
+  const bool off32 = narrow(p.am, p.M, p.ak, akf) && narrow(p.bn, p.N, p.bk, bkf);
+  // pairs along the contiguous index of both operands
+  auto pairs = [](const Idx2& d, int64_t n) { return d.s2 == 1 && n >= 2 && (d.n2 % 2 == 0 || n <= d.n2); };
+  const bool two = off32 && (pl.tile == 128 || (narrow(p.am, p.M, p.ak, true) && narrow(p.bn, p.N, p.bk, true))) &&
+                   pairs(akf ? p.ak : p.am, akf ? p.K : p.M) && pairs(bkf ? p.bk : p.bn, bkf ? p.K : p.N);
+  if constexpr (sizeof(T) == 8) {
+    if (two) launch_tile<T, uint32_t, 2>(pl.tile, g, p.batch, akf, bkf, s);
+    else if (off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+  } else {
+    if (off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+  }
+  if (pl.splits > 1) splitk_reduce<T>(p, g.work, pl.splits, s);
 }
 
 template void tc_gemm<double>(const GemmParams<double>&, Workspace&, hipStream_t);

@@ -42,3 +42,36 @@ def _check(contract, sub, ext, dtype, beta=0.0, seed=0):
 @pytest.mark.parametrize("beta", [0.0, -0.5])
 def test_split_k(contract, m, n, k, dtype, beta):
     _check(contract, "ak,bk->ab", {"a": m, "b": n, "k": k}, dtype, beta)
+
+
+# tile edges (64 and 128) and remainders, odd and even extents: 16-byte loads with and without a late pair, every
+# combination of contiguous index in A and B
+@pytest.mark.parametrize("sub", ["ak,bk->ab", "ak,kb->ab", "ka,bk->ab", "ka,kb->ab", "ak,kb->ba"])
+@pytest.mark.parametrize("m,n,k", [(64, 128, 32), (65, 129, 33), (127, 63, 17), (128, 191, 15), (257, 130, 2), (300, 301, 1),
+                                   (1025, 1023, 47)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_tiles(contract, sub, m, n, k, dtype):
+    _check(contract, sub, {"a": m, "b": n, "k": k}, dtype, beta=0.5)
+
+
+# two-level rows and columns, two and three summed indices that do not fuse, inner extents under and over a k-tile
+@pytest.mark.parametrize("sub", ["kaub,ukcd->abcd", "iumef,umefa->ia", "imef,efam->ia", "imef,fmea->ia", "mnab,nmba->a",
+                                 "xmey,mfxe->fy", "mief,meaf->ia", "jnfb,mnef->mbej"])
+@pytest.mark.parametrize("occ,vir", [(3, 17), (5, 16), (17, 31), (2, 40)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_compound_indices(contract, sub, occ, vir, dtype):
+    ext = {c: (vir if c in "abcdefg" else occ) for c in sub if c.isalpha()}
+    _check(contract, sub, ext, dtype)
+
+
+def test_rows_more_than_4_gib_apart(contract):
+    """Rows of A 2 GiB apart: lane offsets past 32 bits."""
+    step, rows, k, n = 1 << 28, 3, 37, 21
+    buf = torch.empty((rows - 1) * step + k, dtype=torch.float64, device="cuda")
+    A = torch.as_strided(buf, (rows, k), (step, 1))
+    g = torch.Generator().manual_seed(1)
+    a, b = torch.randn(rows, k, dtype=torch.float64, generator=g), torch.randn(k, n, dtype=torch.float64, generator=g)
+    A.copy_(a)
+    for sub, B in (("ak,kb->ab", b), ("ak,bk->ab", b.t().contiguous())):
+        out = contract(sub, A, B.cuda()).cpu()
+        assert float((out - a @ b).abs().max()) <= 2 * (k + 4) * 2.2e-16 * float((a.abs() @ b.abs()).max())
