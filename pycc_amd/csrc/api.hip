@@ -242,7 +242,7 @@ int ccx_vjp(ccx_ctx* ctx, const double* fock, const double* t1, const double* t2
     else
       ccx::hbar_build(c, fock, t1, t2, (flags & CCX_HBAR_STORED) != 0, s);
     // l1 = c1, l2 = c2 + c2^T (r2 is pair-symmetric, so only the symmetric part of c2 acts)
-    ccx::pair_symmetrize(c.o, c.v, 1.0, c2, c.Lsym, s);
+    ccx::pair_symmetrize(c.o, c.v, 1.0, 1, c2, c.Lsym, s);
     ccx::lambda_residual(c, c1, c.Lsym, g1, g2, false, 0.5, s);
   });
 }
@@ -259,7 +259,7 @@ int ccx_jvp(ccx_ctx* ctx, const double* fock, const double* t1, const double* t2
     else
       ccx::hbar_build(c, fock, t1, t2, (flags & CCX_HBAR_STORED) != 0, s);
     // the pair-symmetric part of x2 (t2_ijab and t2_jiba are one parameter)
-    ccx::pair_symmetrize(c.o, c.v, 0.5, x2, c.Lsym, s);
+    ccx::pair_symmetrize(c.o, c.v, 0.5, 1, x2, c.Lsym, s);
     ccx::jacobian(c, x1, c.Lsym, j1, j2, s);
   });
 }

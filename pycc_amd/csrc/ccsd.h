@@ -11,6 +11,29 @@ namespace ccx {
 
 enum Mode : int { MODE_DP = 0, MODE_MIXED = 1, MODE_MIXED_BF16X3 = 2, MODE_MIXED_F16X3 = 3 };
 
+// A sum of many contractions as `count` partial sums, taken in turn: contractions into different ones are independent, so a
+// queue gathers them into one launch. An array's first term has beta = 0.
+struct PartSum {
+  double* base;
+  int64_t n;
+  int count, used = 0, next = 0;
+  PartSum(double* b, int64_t size, int cnt) : base(b), n(size), count(cnt) {}
+  double* take(double& beta) {
+    const int k = next;
+    next = next + 1 == count ? 0 : next + 1;
+    beta = k < used ? 1.0 : 0.0;
+    used = used > k + 1 ? used : k + 1;
+    return base + k * n;
+  }
+};
+constexpr int SINGLES_PARTS = 16;                           // r_L1 and the Jacobian's singles
+constexpr int PR1 = 8, PAE = 4, PMI = 3, PMNIJ = 3;         // r1, Fae, Fmi, Wmnij
+// o^2 v^2 partial sums of r2, r_L2 and the Jacobian's doubles: while launches and small grids are what the terms cost (a
+// 4 M element array of o=16 v=128 is 34 MB, read once more in 8 us)
+inline int doubles_parts(int64_t n) { return n <= (int64_t(1) << 19) ? 8 : n <= (int64_t(1) << 22) ? 4 : 1; }
+constexpr int64_t W_PARTS = int64_t(1) << 20;               // (ov)^2 up to which W is summed from partial sums
+constexpr int64_t GEMV_OV = 1024;                           // ov from which o^2 v^2 matrix-vector terms have launches of their own
+
 struct Ctx {
   int64_t o = 0, v = 0, nmo = 0;
   int mode = MODE_DP;
@@ -81,6 +104,10 @@ struct Ctx {
   // beside the rest of the residual (fork after the amplitude scales, join before zt_add)
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // partial sums (PartSum) of r1, Fae, Fmi and Wmnij; at small sizes also of Zt (two) and W (DP: three and K.A1), and a tau~
+  // beside tau (else taut == tau)
+  double *pr1 = nullptr, *pae = nullptr, *pmi = nullptr, *pmnij = nullptr, *pZt = nullptr, *pW = nullptr, *taut = nullptr;
+  bool parts() const { return doubles_parts(ov() * ov()) > 1; }
   double* red = nullptr;             // reduction partials
   double* scal = nullptr;            // small device scalars
 
@@ -125,6 +152,7 @@ struct Ctx {
   double *Ltmp = nullptr, *Goo = nullptr, *Gvv = nullptr, *Lh = nullptr, *Lsym = nullptr;
   double *LY = nullptr, *LVf = nullptr, *LVg = nullptr, *LU = nullptr, *LQ = nullptr, *Lsm = nullptr;
   double* Jsm = nullptr;
+  double *Lr = nullptr, *Ltmp2 = nullptr, *Ltmp3 = nullptr;   // partial sums of r_L1; more temporaries
   double* Jv3 = nullptr;   // density energy: two v^3 slices and the term values
 
   // ---- DIIS (pycc utils.helper_diis) ----
@@ -174,8 +202,8 @@ void hbar_block(Ctx& c, int block, double* out, hipStream_t s);
 // vector-Jacobian product of the CCSD residual.
 void lambda_residual(Ctx& c, const double* l1, const double* l2, double* r1, double* r2, bool with_source,
                      double alpha, hipStream_t s);
-// out[i][j][a][b] = alpha * (h[i][j][a][b] + h[j][i][b][a])
-void pair_symmetrize(int64_t o, int64_t v, double alpha, const double* h, double* out, hipStream_t s);
+// out[i][j][a][b] = alpha * (h[i][j][a][b] + h[j][i][b][a]), h the sum of `parts` arrays one after the other
+void pair_symmetrize(int64_t o, int64_t v, double alpha, int parts, const double* h, double* out, hipStream_t s);
 void pseudoenergy(Ctx& c, const double* l2, double* e_dev, hipStream_t s);
 // dL/dF (full [nmo][nmo] D) and the two-particle densities of the Lagrangian at (t, l)
 void densities(Ctx& c, const double* t1, const double* t2, const double* l1, const double* l2, double* D,

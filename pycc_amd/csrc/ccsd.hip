@@ -237,8 +237,16 @@ void alloc_work(Ctx& c) {
   c.Hm = c.alloc<double>(o * o);
   c.tau = c.alloc<double>(ov * ov);
   c.Wmnij = c.alloc<double>(o * o * o * o);
-  c.Hh = c.alloc<double>(ov * ov);
+  const int hp = c.mode == MODE_MIXED_F16X3 ? 1 : doubles_parts(ov * ov);
+  c.Hh = c.alloc<double>((size_t)hp * ov * ov);
   c.Zt = c.alloc<double>(ov * o * o);
+  c.pr1 = c.alloc<double>(PR1 * ov);
+  c.pae = c.alloc<double>(PAE * v * v);
+  c.pmi = c.alloc<double>(PMI * o * o);
+  c.pmnij = c.alloc<double>(PMNIJ * o * o * o * o);
+  c.taut = c.parts() ? c.alloc<double>(ov * ov) : c.tau;
+  if (c.parts()) c.pZt = c.alloc<double>(2 * ov * o * o);
+  if (c.mode == MODE_DP && ov * ov <= W_PARTS) c.pW = c.alloc<double>(7 * ov * ov);   // three of 2 (ov)^2, one of (ov)^2
   if (c.mode != MODE_MIXED_F16X3) c.Wd = c.alloc<double>(2 * ov * ov);   // FP16x3 builds W directly
   c.Ud = c.alloc<double>(ov * ov);
   const size_t es = c.mode == MODE_DP ? sizeof(double) : sizeof(float);
@@ -320,6 +328,12 @@ void ladder_bf16x3(Ctx& c, const double* t1, const double* t2, hipStream_t s);  
 void ladder_x3(Ctx& c, const double* t1, const double* t2, hipStream_t s);       // split16.hip
 
 // The ring and ladder GEMMs run in T (double for DP, float for the mixed modes).
+//
+// Small FP64 terms go through a queue (gemm.h) that runs independent ones in one launch. Its order of terms follows what
+// they read -- amplitudes and integrals, then the intermediates, then G and Hm -- and sums of several terms are taken as
+// partial sums (PartSum), which are independent of each other. One by one the terms of o=5 v=19 are 67 launches of 5 to
+// 10 us; together they are about 25. Where a sum is rounded to FP32 or FP16 operands afterwards (Wmnij and W in the mixed
+// modes, Fae in MIXED_F16X3) its terms are added in the same order in every form.
 template <typename T>
 static void residual_t(Ctx& c, const double* F, const double* t1, const double* t2, double* r1,
                        double* r2, hipStream_t s) {
@@ -329,17 +343,29 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
   const std::vector<int64_t> OOOV{o, o, o, v}, OVVV{o, v, v, v}, OOOO{o, o, o, o};
   // Fock blocks, row-major (nmo x nmo)
   const TV Fov = tvs(F + o, "me", OV, {nmo, 1});
-  const TV Fvv = tvs(F + o * nmo + o, "ae", VV, {nmo, 1});
-  const TV Foo = tvs(F, "mi", OO, {nmo, 1});
-  const TV Fvo = tvs(F + o * nmo, "ai", {v, o}, {nmo, 1});
 
   auto T1 = [&](const char* l) { return tv(t1, l, OV); };
   auto T2 = [&](const char* l) { return tv(t2, l, OOVV); };
-  auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C) {
-    contract<double>(a, A, B, b, C, ws, s);
+  GemmQueue q(ws, s);
+  auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C, int part = 0) {
+    contract<double>(a, A, B, b, C, ws, s, false, &q, part);
   };
+  auto copy = [&](double a, const TV& A, const TV& C) { axpby<double>(a, A, 0.0, C, s, &q); };
 
+  constexpr bool dp = std::is_same<T, double>::value;
   const bool x3 = c.mode == MODE_MIXED_F16X3;
+  const bool parts = c.parts();   // sizes at which partial sums pay (doubles_parts)
+  // partial sums of r1, Fae, Fmi, Wmnij, and of the half residual Hh
+  PartSum pr1(c.pr1, ov, PR1), pae(c.pae, v * v, PAE), pmi(c.pmi, o * o, PMI), pw(c.pmnij, o * o * o * o, PMNIJ);
+  PartSum ph(c.Hh, ov * ov, x3 ? 1 : doubles_parts(ov * ov));
+  auto into = [&](PartSum& ps, const char* l, const std::vector<int64_t>& ext, double a, const TV& A, const TV& B) {
+    double beta;
+    double* p = ps.take(beta);
+    cd(a, A, B, beta, tv(p, l, ext));
+  };
+  auto R1 = [&](double a, const TV& A, const TV& B) { into(pr1, "ia", OV, a, A, B); };
+  auto H = [&](double a, const TV& A, const TV& B) { into(ph, "ijab", OOVV, a, A, B); };
+
   if (x3) x3_amp_scales(c, t1, t2, s);   // every amplitude-derived FP16x3 operand scale
   // ---- ladder + Z: ccwfn.py:931 (1/2 tau_ijef <ab|ef>) and :715 (Z_mbij = <mb|ef> tau_ijef) ----
   // In the split-GEMM modes it needs only t1, t2 (and the scales above): it runs on the side stream
@@ -353,42 +379,146 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
   }
   if (x3) covvv_x3_products(c, t1, s);   // the <ov|vv> products of t1 (Fae, W, Hh terms below)
 
-  // ---- Fme: ccwfn.py:563-564 -------------------------------------------------------------
-  const TV Fme = tv(c.Fme, "me", OV);
-  axpby<double>(1.0, Fov, 0.0, Fme, s);
-  // + t_nf L_mnef: Fme[m][e] += sum_(n,f) t[n][f] Loovv[m][n][e][f]
-  wsum(o, v, o, v, 1.0, t1, v, c.Loovv, o * v * v, v, v * v, 1.0, c.Fme, v, s);
+  // ---- operands from t1, t2: tau~ = t2 + 1/2 t1 t1 (c.taut; :494-497), tau (:603, :455), the ring operands ----
+  T* S1 = (T*)c.S1;
+  T* A1 = (T*)c.A1;
+  T* S2 = (T*)c.S2;
+  T* Tx = (T*)c.Tx;
+  T* W = (T*)c.W;
+  const bool two_tau = c.taut != c.tau;   // else tau~ is used before tau is formed in its place
+  build_tau(o, v, 1.0, 0.5, t1, t2, c.taut, s, two_tau ? c.tau : nullptr, 1.0);
+  if (!x3) ring_prep<T>(o, v, t1, t2, S1, A1, S2, Tx, c.Ud, s);
 
-  // ---- Fae: ccwfn.py:494-497 (tau~ = t2 + 1/2 t1 t1) ----------------------------------------
-  build_tau(o, v, 1.0, 0.5, t1, t2, c.tau, s);
-  const TV Fae = tv(c.Fae, "ae", VV);
-  axpby<double>(1.0, Fvv, 0.0, Fae, s);
-  cd(-0.5, Fov, T1("ma"), 1.0, Fae);
-  if (x3) {
-    covvv_x3_fae(c, c.Fae, s);
-  } else {
-    cd(2.0, T1("mf"), tv(c.Covvv, "mfae", OVVV), 1.0, Fae);   // L_mafe = 2(mf|ae) - (me|af)
-    cd(-1.0, T1("mf"), tv(c.Covvv, "meaf", OVVV), 1.0, Fae);
+  // ---- the terms without amplitudes --------------------------------------------------------------
+  // W[(m,e)][x][(j,b)]: x = 0 Wmbej, x = 1 Wmbje (built in FP64 Wd and cast, or in MIXED_F16X3
+  // written in FP32 by one kernel)
+  const std::vector<int64_t> WSTR{v * 2 * ov, 2 * ov, v, 1};   // [(me)][x][(jb)]
+  auto Wh = [&](double* w, int x) { return tvs(w + x * ov, "mejb", OVOV, WSTR); };   // half x of a W array
+  const bool g_split = x3 && c.T2h;   // :925 as an FP16x3 GEMM: <ij|ab> (:922) is then added by assemble_r2
+  if (!x3) {
+    copy(1.0, tv(c.Covov, "mejb", OVOV), Wh(c.Wd, 0));              // <mb|ej> = (me|jb)        :641
+    copy(-1.0, tv(c.Coovv, "mjbe", OOVV), Wh(c.Wd, 1));             // -<mb|je> = -(mj|be)       :680
   }
-  if (!x3) cd(-1.0, tv(c.tau, "mnaf", OOVV), tv(c.Loovv, "mnef", OOVV), 1.0, Fae);   // FP16x3: below
+  if (!g_split) {
+    double beta;
+    copy(0.5, tv(c.Ioovv, "ijab", OOVV), tv(ph.take(beta), "ijab", OOVV));   // 1/2 <ab|ij> = 1/2 <ij|ab> :922
+  }
+  copy(1.0, Fov, tv(c.Fme, "me", OV));
+  copy(1.0, tv(c.Coooo, "minj", OOOO), tv(c.Wmnij, "mnij", OOOO));  // <mn|ij> = (mi|nj)
+  copy(1.0, tv(c.Cooov, "mijb", OOOV), tv(c.Zt, "mijb", {o, o, o, v}));   // <mb|ij> = (mi|jb)
 
-  // ---- Fmi: ccwfn.py:530-533 --------------------------------------------------------------
-  const TV Fmi = tv(c.Fmi, "mi", OO);
-  axpby<double>(1.0, Foo, 0.0, Fmi, s);
-  cd(0.5, T1("ie"), Fov, 1.0, Fmi);
-  cd(1.0, T1("ne"), tv(c.Looov, "imne", OOOV), 1.0, Fmi);     // L_mnie = 2(mi|ne) - (ni|me)
-  cd(1.0, tv(c.tau, "inef", OOVV), tv(c.Loovv, "mnef", OOVV), 1.0, Fmi);
-  if (x3) fae_tauL_x3(c, c.Fae, s);   // :497 as an FP16x3 GEMM (tau~ still in c.tau)
+  // ---- Fme: ccwfn.py:563-564; Fae: :494-497; Fmi: :530-533 ----------------------------------
+  const TV Fme = tv(c.Fme, "me", OV), Fae = tv(c.Fae, "ae", VV), Fmi = tv(c.Fmi, "mi", OO);
+  const TV Fvv = tvs(F + o * nmo + o, "ae", VV, {nmo, 1});
+  auto AE = [&](double a, const TV& A, const TV& B) { into(pae, "ae", VV, a, A, B); };
+  auto MI = [&](double a, const TV& A, const TV& B) { into(pmi, "mi", OO, a, A, B); };
+  MI(1.0, tv(c.taut, "inef", OOVV), tv(c.Loovv, "mnef", OOVV));
+  MI(0.5, T1("ie"), Fov);
+  MI(1.0, T1("ne"), tv(c.Looov, "imne", OOOV));     // L_mnie = 2(mi|ne) - (ni|me)
+  if (x3) {
+    axpby<double>(1.0, Fvv, 0.0, Fae, s);
+    contract<double>(-0.5, Fov, T1("ma"), 1.0, Fae, ws, s);
+    covvv_x3_fae(c, c.Fae, s);
+    q.flush();                    // Fmi's tau~ term, before tau takes its place
+    fae_tauL_x3(c, c.Fae, s);     // :497 as an FP16x3 GEMM
+  } else {
+    AE(-1.0, tv(c.taut, "mnaf", OOVV), tv(c.Loovv, "mnef", OOVV));
+    AE(2.0, T1("mf"), tv(c.Covvv, "mfae", OVVV));   // L_mafe = 2(mf|ae) - (me|af)
+    AE(-1.0, T1("mf"), tv(c.Covvv, "meaf", OVVV));
+    AE(-0.5, Fov, T1("ma"));
+  }
+  if (!two_tau) {
+    q.flush();
+    build_tau(o, v, 1.0, 1.0, t1, t2, c.tau, s);
+  }
+  // + t_nf L_mnef: Fme[m][e] += sum_(n,f) t[n][f] Loovv[m][n][e][f]; r1 (:758): 2 sum_(nf) t_nf Covov[(nf)][(ia)] -
+  // sum_(n,f) t_nf Coovv[n][i][a][f], each as one wave per output (wsum) or column sums where a launch is small beside
+  // the block it streams, else with the other small terms
+  const bool gemv = ov >= GEMV_OV;
+  if (!gemv) {
+    cd(1.0, T1("nf"), tv(c.Loovv, "mnef", OOVV), 1.0, Fme);
+    R1(2.0, T1("nf"), tv(c.Covov, "nfia", OVOV));
+    R1(-1.0, T1("nf"), tv(c.Coovv, "niaf", OOVV));
+  }
 
   // ---- Wmnij: ccwfn.py:596-603 (tau = t2 + t1 t1) -------------------------------------------
-  build_tau(o, v, 1.0, 1.0, t1, t2, c.tau, s);
   const TV Wmnij = tv(c.Wmnij, "mnij", OOOO);
-  axpby<double>(1.0, tv(c.Coooo, "minj", OOOO), 0.0, Wmnij, s);   // <mn|ij> = (mi|nj)
-  cd(1.0, T1("je"), tv(c.Cooov, "mine", OOOV), 1.0, Wmnij);        // <mn|ie> = (mi|ne)
-  cd(1.0, T1("ie"), tv(c.Cooov, "njme", OOOV), 1.0, Wmnij);        // <mn|ej> = (nj|me)
-  if (std::is_same<T, double>::value) {
-    cd(1.0, tv(c.tau, "ijef", OOVV), tv(c.Ioovv, "mnef", OOVV), 1.0, Wmnij);  // <mn|ef>
-  } else if (c.mode == MODE_MIXED_F16X3) {
+  auto MNIJ = [&](double a, const TV& A, const TV& B) { into(pw, "mnij", OOOO, a, A, B); };
+  MNIJ(1.0, T1("je"), tv(c.Cooov, "mine", OOOV));                   // <mn|ie> = (mi|ne)
+  MNIJ(1.0, T1("ie"), tv(c.Cooov, "njme", OOOV));                   // <mn|ej> = (nj|me)
+  if (dp) MNIJ(1.0, tv(c.tau, "ijef", OOVV), tv(c.Ioovv, "mnef", OOVV));   // <mn|ef>
+
+  // ---- the W intermediates: ccwfn.py:641-645 (Wmbej), :680-683 (Wmbje) ----
+  // At small sizes (pW) the FP64 terms are partial sums too: 0 the t1 (me|bf) terms, 1 the t1 (nj|me) ones, 2 J.S1, and the
+  // half-sized K.A1 behind them.
+  const std::vector<int64_t> OVXOV{o, v, 2, o, v};
+  const T* Kt = dp ? (const T*)c.Covov : (const T*)c.K32;
+  const T* Jt = dp ? (const T*)c.J : (const T*)c.J32;
+  const bool wparts = dp && c.pW && !c.timing;
+  const int64_t wn = 2 * ov * ov;
+  if (!x3) {
+    double* w0 = wparts ? c.pW : c.Wd;
+    double* w1 = wparts ? c.pW + wn : c.Wd;
+    const double b = wparts ? 0.0 : 1.0;
+    cd(1.0, T1("jf"), tv(c.Covvv, "mebf", OVVV), b, Wh(w0, 0), 1);         // t_jf <mb|ef>, (me|bf)     :642
+    cd(-1.0, T1("jf"), tv(c.Covvv, "mfbe", OVVV), b, Wh(w0, 1), 2);        // t_jf <mb|fe>, (mf|be)     :681
+    cd(-1.0, T1("nb"), tv(c.Cooov, "njme", OOOV), b, Wh(w1, 0), 1);        // t_nb <mn|ej>, (nj|me)     :643
+    cd(1.0, T1("nb"), tv(c.Cooov, "mjne", OOOV), b, Wh(w1, 1), 2);         // t_nb <mn|je>, (mj|ne)     :682
+  }
+  // :644 -tau'_jnfb <mn|ef> (tau' = t2/2 + t1 t1), :645 +1/2 t_njfb L_mnef, :683 +tau'_jnfb <mn|fe>:
+  //   Wej += K.(T - Tx/2 - P1) - 1/2 J.T ;  Wje += J.tau'
+  if (wparts) {
+    cd(1.0, tv(c.J, "menf", OVOV), tv(c.S1, "nfxjb", OVXOV), 0.0, tv(c.pW + 2 * wn, "mexjb", OVXOV));
+    cd(1.0, tv(c.Covov, "menf", OVOV), tv(c.A1, "nfjb", OVOV), 0.0, tv(c.pW + 3 * wn, "mejb", OVOV));
+  }
+
+  // ---- more terms that read amplitudes and integrals only: Zt, Hh, r1 -----------------------------
+  // Zt_mbij = Z_mbij + <mb|ij> + t_ie <mb|ej> + t_je <mb|ie>: :932 -t_ma Z_mbij, :940 -t_ma <mb|ij>, :937 -t_ie t_ma
+  // <mb|ej>, and :938 -t_ie t_mb <ma|je> taken in its (ij)(ab)-swapped form -t_ma (t_je <mb|ie>) (same symmetrised
+  // r2, :790).
+  double* z1 = parts ? c.pZt : c.Zt;
+  double* z2 = parts ? c.pZt + o * o * ov : c.Zt;
+  cd(1.0, T1("ie"), tv(c.Covov, "mejb", OVOV), parts ? 0.0 : 1.0, tv(z1, "mijb", {o, o, o, v}));   // <mb|ej> = (me|jb)
+  cd(1.0, T1("je"), tv(c.Coovv, "mibe", OOVV), parts ? 0.0 : 1.0, tv(z2, "mijb", {o, o, o, v}));   // <mb|ie> = (mi|be)
+  if (!x3) {
+    H(1.0, T1("ie"), tv(c.Covvv, "jbae", OVVV));                    // t_ie <ab|ej> = t_ie (jb|ae) :939
+    R1(1.0, tv(c.Ud, "meif", OVOV), tv(c.Covvv, "meaf", OVVV));     // <ma|ef> = (me|af)    :759
+  }
+  R1(-1.0, T2("mnae"), tv(c.Looov, "imne", OOOV));                  // L_nmei = 2(mi|ne) - (ni|me) :760
+
+  // ---- ladder + Z in the FP64 / FP32 modes ----
+  const int64_t npP = c.npP(), npM = c.npM(), noP = c.noP(), noM = c.noM();
+  const double f_lad_P = 2.0 * noP * (npP + ov) * npP, f_lad_M = 2.0 * noM * (npM + ov) * npM;
+  const bool queue_ladder = dp && parts && !c.timing;
+  auto ladder = [&] {
+    int k = c.tbegin(s, Ctx::PH_LADDER, f_lad_P);
+    const TV tp = tv(c.Tp, "xk", {noP, npP}), lp = tv(c.LP, "ky", {npP, npP + ov}), cp = tv(c.CP, "xy", {noP, npP + ov});
+    contract<T>(T(1), tp, lp, T(0), cp, ws, s, false, queue_ladder ? &q : nullptr);
+    c.tend(s, k);
+    if (noM > 0) {
+      k = c.tbegin(s, Ctx::PH_LADDER, f_lad_M);
+      const TV tm = tv(c.Tm, "xk", {noM, npM}), lm = tv(c.LM, "ky", {npM, npM + ov}), cm = tv(c.CM, "xy", {noM, npM + ov});
+      contract<T>(T(1), tm, lm, T(0), cm, ws, s, false, queue_ladder ? &q : nullptr);
+      c.tend(s, k);
+    }
+  };
+  if (queue_ladder) {
+    tau_pack<T>(o, v, t1, t2, (T*)c.Tp, (T*)c.Tm, s);   // meets nothing queued
+    ladder();
+  }
+  q.flush();
+
+  // ---- sums: Fae, Fmi, Wmnij, W ------------------------------------------------------------------
+  {
+    SumJobs j;
+    if (!x3) j.add(v * v, v, nmo, 1, (const double*)Fvv.p, pae, c.Fae, c.G);
+    else j.add(v * v, v, v, 1, c.Fae, pae, c.Fae, c.G);
+    j.add(o * o, o, nmo, 1, F, pmi, c.Fmi, c.Hm);
+    j.add(o * o * o * o, o * o, o * o, 1, c.Wmnij, pw, c.Wmnij, nullptr);
+    sum_jobs(j, s);
+  }
+  if (gemv) wsum(o, v, o, v, 1.0, t1, v, c.Loovv, o * v * v, v, v * v, 1.0, c.Fme, v, s);
+  if (x3) {
     // the two o^4 v^2 hole-hole contractions (:603 and :930) as FP16x3 GEMMs; tau is split once in
     // both orientations ([(ij)][(ef)] here, [(ab)][(mn)] for :930) with one scale
     x3_split_rows<double>(c.tau, o * o, v * v, v * v, c.xs + 5, c.TAh, c.TAl, c.v2p(), s);
@@ -398,47 +528,21 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.Ah = c.Ioh; g.Al = c.Iol; g.Bh = c.TAh; g.Bl = c.TAl; g.C64 = c.Wmnij; g.beta = 1.f;
     g.sa = c.xs + 6; g.sb = c.xs + 5;
     x3_gemm<_Float16>(g, s, &ws);   // into Wmnij (FP64), through split K
-  } else {
+    // every ring operand is bounded by 3 max|t2| + max|t1|^2 (scale xs[0])
+    ring_prep_x3(o, v, c.ovp(), t1, t2, c.xs, c.BJh, c.BJl, c.BKh, c.BKl, c.APh, c.APl, c.AQh, c.AQl, c.Ud, s);
+    w_build_x3(c, t1, (float*)W, s);   // :641-643, :680-682 in one pass, straight to FP32
+  } else if (!dp) {
     // mixed modes: the two o^4 v^2 hole-hole ladder contractions (:603 and :930) run in FP32
     cast<double, float>(ov * ov, c.tau, c.tau32, s);
     contract<float>(1.0f, tv(c.tau32, "ijef", OOVV), tv(c.Io32, "mnef", OOVV), 0.0f, tv(c.W32, "mnij", OOOO),
                     ws, s);
     accumulate(o * o * o * o, 1.0, c.W32, c.Wmnij, s);
+    cast<double, T>(wn, c.Wd, W, s);
+  } else if (wparts) {
+    w_sum(ov, c.pW, c.Wd, s);
   }
 
-  // ---- ring operands and the W intermediates: ccwfn.py:641-645 (Wmbej), :680-683 (Wmbje) ----
-  // W[(m,e)][x][(j,b)]: x = 0 Wmbej, x = 1 Wmbje (built in FP64 Wd and cast, or in MIXED_F16X3
-  // written in FP32 by one kernel).
-  T* S1 = (T*)c.S1;
-  T* A1 = (T*)c.A1;
-  T* S2 = (T*)c.S2;
-  T* Tx = (T*)c.Tx;
-  T* W = (T*)c.W;
-  if (x3) {
-    // every ring operand is bounded by 3 max|t2| + max|t1|^2 (scale xs[0])
-    ring_prep_x3(o, v, c.ovp(), t1, t2, c.xs, c.BJh, c.BJl, c.BKh, c.BKl, c.APh, c.APl, c.AQh, c.AQl, c.Ud, s);
-  } else {
-    ring_prep<T>(o, v, t1, t2, S1, A1, S2, Tx, c.Ud, s);
-  }
-  // W[(me)][x][(jb)]: x = 0 holds Wmbej, x = 1 holds Wmbje
-  const std::vector<int64_t> WSTR{v * 2 * ov, 2 * ov, v, 1};
-  if (x3) {
-    w_build_x3(c, t1, (float*)W, s);   // :641-643, :680-682 in one pass, straight to FP32
-  } else {
-    const TV Wej = tvs(c.Wd, "mejb", OVOV, WSTR), Wje = tvs(c.Wd + ov, "mejb", OVOV, WSTR);
-    axpby<double>(1.0, tv(c.Covov, "mejb", OVOV), 0.0, Wej, s);    // <mb|ej> = (me|jb)        :641
-    cd(1.0, T1("jf"), tv(c.Covvv, "mebf", OVVV), 1.0, Wej);        // t_jf <mb|ef>, (me|bf)     :642
-    axpby<double>(-1.0, tv(c.Coovv, "mjbe", OOVV), 0.0, Wje, s);   // -<mb|je> = -(mj|be)       :680
-    cd(-1.0, T1("jf"), tv(c.Covvv, "mfbe", OVVV), 1.0, Wje);       // t_jf <mb|fe>, (mf|be)     :681
-    cd(-1.0, T1("nb"), tv(c.Cooov, "njme", OOOV), 1.0, Wej);       // t_nb <mn|ej>, (nj|me)     :643
-    cd(1.0, T1("nb"), tv(c.Cooov, "mjne", OOOV), 1.0, Wje);        // t_nb <mn|je>, (mj|ne)     :682
-    if (!std::is_same<T, double>::value) cast<double, T>(2 * ov * ov, c.Wd, W, s);
-  }
-  const T* Kt = std::is_same<T, double>::value ? (const T*)c.Covov : (const T*)c.K32;
-  const T* Jt = std::is_same<T, double>::value ? (const T*)c.J : (const T*)c.J32;
-  const std::vector<int64_t> OVXOV{o, v, 2, o, v};
-  // :644 -tau'_jnfb <mn|ef> (tau' = t2/2 + t1 t1), :645 +1/2 t_njfb L_mnef, :683 +tau'_jnfb <mn|fe>:
-  //   Wej += K.(T - Tx/2 - P1) - 1/2 J.T ;  Wje += J.tau'
+  // ---- ring GEMMs of W ---------------------------------------------------------------------------
   const double unit = 2.0 * (double)ov * ov * ov;   // one ov x ov x ov GEMM
   const int64_t ovp = c.ovp();
   int kr = c.tbegin(s, Ctx::PH_RING, 2 * unit);
@@ -449,7 +553,7 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.Ah = c.Jh; g.Al = c.Jl; g.Bh = c.BJh; g.Bl = c.BJl; g.C = (float*)W;
     g.sa = c.xs + 1; g.sb = c.xs; g.beta = 1.f;
     x3_gemm<_Float16>(g, s);
-  } else {
+  } else if (!wparts) {
     contract<T>(T(1), tv(Jt, "menf", OVOV), tv(S1, "nfxjb", OVXOV), T(1), tv(W, "mexjb", OVXOV), ws, s);
   }
   c.tend(s, kr);
@@ -462,29 +566,16 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.sa = c.xs + 2; g.sb = c.xs; g.beta = 1.f;
     x3_gemm<_Float16>(g, s);
     // W (FP32 [me][x][jb]) -> split BP[jb][x][me] with its own scale xs[3]
-    x3_absmax<float>((const float*)W, 2 * ov * ov, c.xpart, s);
+    x3_absmax<float>((const float*)W, wn, c.xpart, s);
     x3_scale(c.xpart, 1.f, nullptr, 0.f, c.xs + 3, s);
     x3_split_t((const float*)W, ov, ov, 2, 2 * ov, c.xs + 3, c.BPh, c.BPl, ovp, 2 * ovp, s, true);
-  } else {
+  } else if (!wparts) {
     contract<T>(T(1), tv(Kt, "menf", OVOV), tv(A1, "nfjb", OVOV), T(1), tvs(W, "mejb", OVOV, WSTR), ws, s);
   }
   c.tend(s, kr);
-
-  // ---- ladder + Z in the FP64 / FP32 modes (through the contraction planner and its workspace) ----
-  const int64_t npP = c.npP(), npM = c.npM(), noP = c.noP(), noM = c.noM();
-  const double f_lad_P = 2.0 * noP * (npP + ov) * npP, f_lad_M = 2.0 * noM * (npM + ov) * npM;
-  if (!c.split_ladder()) {
+  if (!c.split_ladder() && !queue_ladder) {
     tau_pack<T>(o, v, t1, t2, (T*)c.Tp, (T*)c.Tm, s);
-    int k = c.tbegin(s, Ctx::PH_LADDER, f_lad_P);
-    contract<T>(T(1), tv(c.Tp, "xk", {noP, npP}), tv(c.LP, "ky", {npP, npP + ov}), T(0),
-                tv(c.CP, "xy", {noP, npP + ov}), ws, s);
-    c.tend(s, k);
-    if (noM > 0) {
-      k = c.tbegin(s, Ctx::PH_LADDER, f_lad_M);
-      contract<T>(T(1), tv(c.Tm, "xk", {noM, npM}), tv(c.LM, "ky", {npM, npM + ov}), T(0),
-                  tv(c.CM, "xy", {noM, npM + ov}), ws, s);
-      c.tend(s, k);
-    }
+    ladder();
   }
 
   // ---- ring GEMMs: ccwfn.py:933-935 ------------------------------------------------------------
@@ -492,6 +583,7 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
   // Q[(ja),(ib)] = t2_mjae Wmbie                                (:935)
   T* P = A1;   // A1 is dead after the K GEMM
   T* Q = S1;   // S1 is dead after the J GEMM
+  GemmQueue* rq = dp && parts && !c.timing ? &q : nullptr;
   kr = c.tbegin(s, Ctx::PH_RING, 2 * unit);
   if (x3) {
     X3Gemm g;
@@ -501,7 +593,7 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.sa = c.xs; g.sb = c.xs + 3;
     x3_gemm<_Float16>(g, s);
   } else {
-    contract<T>(T(1), tv(S2, "iamex", {o, v, o, v, 2}), tv(W, "mexjb", OVXOV), T(0), tv(P, "iajb", OVOV), ws, s);
+    contract<T>(T(1), tv(S2, "iamex", {o, v, o, v, 2}), tv(W, "mexjb", OVXOV), T(0), tv(P, "iajb", OVOV), ws, s, false, rq);
   }
   c.tend(s, kr);
   kr = c.tbegin(s, Ctx::PH_RING, unit);
@@ -513,48 +605,32 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.sa = c.xs; g.sb = c.xs + 3;
     x3_gemm<_Float16>(g, s);
   } else {
-    contract<T>(T(1), tv(Tx, "jame", OVOV), tvs(W + ov, "meib", OVOV, WSTR), T(0), tv(Q, "jaib", OVOV), ws, s);
+    contract<T>(T(1), tv(Tx, "jame", OVOV), tvs(W + ov, "meib", OVOV, WSTR), T(0), tv(Q, "jaib", OVOV), ws, s, false, rq);
   }
   c.tend(s, kr);
 
-  // ---- Zt_mbij = Z_mbij + <mb|ij> + t_ie <mb|ej> + t_je <mb|ie> -----------------------------------
-  // :932 -t_ma Z_mbij, :940 -t_ma <mb|ij>, :937 -t_ie t_ma <mb|ej>, and :938 -t_ie t_mb <ma|je>
-  // taken in its (ij)(ab)-swapped form -t_ma (t_je <mb|ie>) (same symmetrised r2, :790).
-  const TV Zt = tv(c.Zt, "mijb", {o, o, o, v});                     // Z-like terms, [m][i][j][b]
-  axpby<double>(1.0, tv(c.Cooov, "mijb", OOOV), 0.0, Zt, s);        // <mb|ij> = (mi|jb)
-  cd(1.0, T1("ie"), tv(c.Covov, "mejb", OVOV), 1.0, Zt);            // <mb|ej> = (me|jb)
-  cd(1.0, T1("je"), tv(c.Coovv, "mibe", OOVV), 1.0, Zt);            // <mb|ie> = (mi|be)
-  if (c.split_ladder()) CCX_HIP(hipStreamWaitEvent(s, c.ev_join, 0));   // CP, CM from the side stream
-  if (c.mode == MODE_DP) zt_add<double>(o, v, (const double*)c.CP, (const double*)c.CM, c.Zt, s);
-  else zt_add<float>(o, v, (const float*)c.CP, (const float*)c.CM, c.Zt, s);
-
-  // ---- half residual Hh (before P(ij,ab)): ccwfn.py:922-940 ------------------------------------
-  const TV Hh = tv(c.Hh, "ijab", OOVV);
-  // :923-925  t2_ijae (Fae_be - 1/2 t_mb Fme_me)
-  const TV G = tv(c.G, "be", VV);
-  axpby<double>(1.0, tv(c.Fae, "be", VV), 0.0, G, s);
+  // ---- from the intermediates: G, Hm, Hh, r1 -------------------------------------------------------
+  // :923-925  G_be = Fae_be - 1/2 t_mb Fme_me;  :926-928  Hm_mj = Fmi_mj + 1/2 t_je Fme_me (the copies are there)
+  const TV G = tv(c.G, "be", VV), Hm = tv(c.Hm, "mj", OO);
   cd(-0.5, T1("mb"), Fme, 1.0, G);
+  cd(0.5, T1("je"), Fme, 1.0, Hm);
+  R1(1.0, T1("ie"), Fae);                                            //                      :755
+  R1(-1.0, Fmi, T1("ma"));                                           //                      :756
+  // U = 2 t2 - t2^T in ring layout: Ud[i][a][m][e] = 2 t2_imae - t2_imea: (2t2 - t2^T) Fme :757
+  if (!gemv) R1(1.0, Fme, tv(c.Ud, "iame", OVOV));
+  // :930  1/2 tau_mnab Wmnij: in the mixed modes an FP32 product that assemble_r2 adds
+  if (dp) H(0.5, tv(c.tau, "mnab", OOVV), Wmnij);
+  q.flush();
   // In MIXED_F16X3 the FP32 terms :925 (off-diagonal G) and :930 go to Xr (the ring W buffer, dead
   // after the ring GEMMs), and <ij|ab> (:922) and the diagonal t2_ijab G_bb are added in FP64 by
   // assemble_r2; Hh then holds the -t2 Hm term only.
   float* Xr = x3 ? (float*)c.W : nullptr;
-  const bool g_split = x3 && c.T2h;
-  if (g_split) {
-    hh_g_x3(c, t2, Xr, s);   // Xr = off-diagonal t2 G (:925) in FP32; Gd = G's diagonal
-  } else {
-    axpby<double>(0.5, tv(c.Ioovv, "ijab", OOVV), 0.0, Hh, s);      // 1/2 <ab|ij> = 1/2 <ij|ab> :922
-    cd(1.0, T2("ijae"), G, 1.0, Hh);
-  }
-  // :926-928  -t2_imab (Fmi_mj + 1/2 t_je Fme_me)
-  const TV Hm = tv(c.Hm, "mj", OO);
-  axpby<double>(1.0, tv(c.Fmi, "mj", OO), 0.0, Hm, s);
-  cd(0.5, T1("je"), Fme, 1.0, Hm);
-  cd(-1.0, T2("imab"), Hm, g_split ? 0.0 : 1.0, Hh);
-  // :930  1/2 tau_mnab Wmnij
+  if (g_split) hh_g_x3(c, t2, Xr, s);   // Xr = off-diagonal t2 G (:925) in FP32; Gd = G's diagonal
+  else H(1.0, T2("ijae"), G);
+  H(-1.0, T2("imab"), Hm);
+  q.flush();
   const float* X930 = nullptr;
-  if (std::is_same<T, double>::value) {
-    cd(0.5, tv(c.tau, "mnab", OOVV), Wmnij, 1.0, Hh);
-  } else if (c.mode == MODE_MIXED_F16X3) {
+  if (x3) {
     cast<double, float>(o * o * o * o, c.Wmnij, c.W32, s);
     x3_absmax<float>(c.W32, o * o * o * o, c.xpart, s);
     x3_scale(c.xpart, 1.f, nullptr, 0.f, c.xs + 7, s);
@@ -565,40 +641,42 @@ static void residual_t(Ctx& c, const double* F, const double* t1, const double* 
     g.sa = c.xs + 7; g.sb = c.xs + 5; g.alpha = 0.5f;
     x3_gemm<_Float16>(g, s, &ws);
     X930 = Xr;
-  } else {
+  } else if (!dp) {
     float* X32 = (float*)c.S2;   // S2 is dead after the P ring GEMM
     cast<double, float>(o * o * o * o, c.Wmnij, c.W32, s);
     contract<float>(0.5f, tv(c.tau32, "mnab", OOVV), tv(c.W32, "mnij", OOOO), 0.0f, tv(X32, "ijab", OOVV), ws, s);
     X930 = X32;
   }
+  if (c.split_ladder()) CCX_HIP(hipStreamWaitEvent(s, c.ev_join, 0));   // CP, CM from the side stream
+  const double* zp = parts ? c.pZt : nullptr;
+  if (dp) zt_add<double>(o, v, (const double*)c.CP, (const double*)c.CM, zp, c.Zt, s);
+  else zt_add<float>(o, v, (const float*)c.CP, (const float*)c.CM, zp, c.Zt, s);
   // :932, :937, :938, :940 through Zt: -t_ma Zt_mijb, summed inside assemble_r2
   // :939  t_ie <ab|ej> = t_ie (jb|ae): in MIXED_F16X3 the FP32 products PT[i][(j,b,a)], added inside
   // assemble_r2 (with X930, the FP32 :930 term of the mixed modes)
-  if (!x3) cd(1.0, T1("ie"), tv(c.Covvv, "jbae", OVVV), 1.0, Hh);
 
   // ---- r2 = Hh + Hh^T + ladder + rings (ccwfn.py:790) --------------------------------------------
-  if (c.mode == MODE_DP)
-    assemble_r2<double>(o, v, c.Hh, (const double*)c.CP, (const double*)c.CM, (const double*)P,
+  if (dp)
+    assemble_r2<double>(o, v, ph.used, c.Hh, (const double*)c.CP, (const double*)c.CM, (const double*)P,
                         (const double*)Q, t1, c.Zt, nullptr, nullptr, nullptr, nullptr, nullptr, r2, s);
   else
-    assemble_r2<float>(o, v, c.Hh, (const float*)c.CP, (const float*)c.CM, (const float*)P,
+    assemble_r2<float>(o, v, ph.used, c.Hh, (const float*)c.CP, (const float*)c.CM, (const float*)P,
                        (const float*)Q, t1, c.Zt, x3 ? c.PT : nullptr, X930, g_split ? c.Ioovv : nullptr,
                        g_split ? t2 : nullptr, g_split ? c.Gd : nullptr, r2, s);
 
   // ---- r1: ccwfn.py:754-760 ------------------------------------------------------------------
-  const TV R1 = tv(r1, "ia", OV);
-  axpby<double>(1.0, Fvo, 0.0, R1, s);                               // f_ai                 :754
-  cd(1.0, T1("ie"), Fae, 1.0, R1);                                   //                      :755
-  cd(-1.0, Fmi, T1("ma"), 1.0, R1);                                  //                      :756
-  // U = 2 t2 - t2^T in ring layout: Ud[i][a][m][e] = 2 t2_imae - t2_imea
-  // (2t2 - t2^T) Fme :757: r1[i][a] += sum_(m,e) Ud[i][a][m][e] Fme[m][e]
-  wsum(o, v, o, v, 1.0, c.Fme, v, c.Ud, v * ov, ov, v, 1.0, r1, v, s);
-  // L_nafi = 2(nf|ia) - (ni|af) :758: 2 sum_(nf) t_nf Covov[(nf)][(ia)] - sum_(n,f) t_nf Coovv[n][i][a][f]
-  colsum(ov, ov, 2.0, t1, c.Covov, ov, 1.0, r1, (double*)ws.get((size_t)colsum_chunks(ov) * ov * sizeof(double)), s);
-  wsum(o, v, o, v, -1.0, t1, v, c.Coovv, v * v, v, o * v * v, 1.0, r1, v, s);
+  {
+    SumJobs j;
+    j.add(ov, v, 1, nmo, F + o * nmo, pr1, r1, nullptr);              // f_ai                 :754
+    sum_jobs(j, s);
+  }
+  if (gemv) {
+    // r1[i][a] += sum_(m,e) Ud[i][a][m][e] Fme[m][e] (:757) and the :758 terms
+    wsum(o, v, o, v, 1.0, c.Fme, v, c.Ud, v * ov, ov, v, 1.0, r1, v, s);
+    colsum(ov, ov, 2.0, t1, c.Covov, ov, 1.0, r1, (double*)ws.get((size_t)colsum_chunks(ov) * ov * sizeof(double)), s);
+    wsum(o, v, o, v, -1.0, t1, v, c.Coovv, v * v, v, o * v * v, 1.0, r1, v, s);
+  }
   if (x3) covvv_x3_r1(c, c.Ud, r1, s);                              // <ma|ef> = (me|af)    :759
-  else cd(1.0, tv(c.Ud, "meif", OVOV), tv(c.Covvv, "meaf", OVVV), 1.0, R1);
-  cd(-1.0, T2("mnae"), tv(c.Looov, "imne", OOOV), 1.0, R1);         // L_nmei = 2(mi|ne) - (ni|me) :760
 }
 
 void residual(Ctx& c, const double* fock, const double* t1, const double* t2, double* r1, double* r2,

@@ -37,16 +37,19 @@ inline TV relabel(TV v, const char* lab) { v.lab = lab; return v; }
 // and a full tile grid) runs as an FP16x3 split product (FP32 accumulation, about 2^-22 relative
 // error per product) instead of in FP64; smaller ones, and every FP32 one, stay as they are.
 constexpr double X3_ROUTE_FLOPS = 1e11;
+// q (FP64): the operation goes through a queue of small ones (gemm.h; `part` as there). An elementwise operation of more
+// than ELT_QUEUE elements (8 MB) is launched by itself.
+constexpr int64_t ELT_QUEUE = 1 << 20;
 template <typename T>
 void contract(T alpha, const TV& A, const TV& B, T beta, const TV& C, Workspace& ws, hipStream_t s,
-              bool split16 = false);
+              bool split16 = false, GemmQueue* q = nullptr, int part = 0);
 
 // C = alpha * A + beta * C elementwise, with A's labels a permutation of C's (up to rank 6).
 template <typename T>
-void axpby(T alpha, const TV& A, T beta, const TV& C, hipStream_t s);
+void axpby(T alpha, const TV& A, T beta, const TV& C, hipStream_t s, GemmQueue* q = nullptr);
 
 // C = beta * C (beta = 0 writes zeros).
 template <typename T>
-void scale(T beta, const TV& C, hipStream_t s);
+void scale(T beta, const TV& C, hipStream_t s, GemmQueue* q = nullptr);
 
 }  // namespace ccx

@@ -117,7 +117,8 @@ TV slice(const TV& v, char c, int64_t i) {
 }  // namespace
 
 template <typename T>
-void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspace& ws, hipStream_t s, bool split16) {
+void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspace& ws, hipStream_t s, bool split16,
+              GemmQueue* q, int part) {
   // Keep C's contiguous index in the N class (B operand): the epilogue stores 16 consecutive n
   // per MFMA row, so this makes the stores coalesced.
   bool swap = false;
@@ -175,7 +176,7 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   auto loop_over = [&](char c) {
     int64_t e = ext_of(c);
     for (int64_t i = 0; i < e; ++i)
-      contract<T>(alpha, slice<T>(A, c, i), slice<T>(B, c, i), beta, slice<T>(C, c, i), ws, s, split16);
+      contract<T>(alpha, slice<T>(A, c, i), slice<T>(B, c, i), beta, slice<T>(C, c, i), ws, s, split16, q, part);
   };
   // An M (N) class with a third index and no batch index: that index becomes the batch, with
   // stride 0 in B (A), which lacks it. Pick the index whose removal leaves a fusable class.
@@ -231,7 +232,7 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
     char c = smallest(ok);
     int64_t e = ext_of(c);
     for (int64_t i = 0; i < e; ++i)
-      contract<T>(alpha, slice<T>(A, c, i), slice<T>(B, c, i), i == 0 ? beta : T(1), C, ws, s, split16);
+      contract<T>(alpha, slice<T>(A, c, i), slice<T>(B, c, i), i == 0 ? beta : T(1), C, ws, s, split16, q, part);
     return;
   }
   if (gm.size() > 2) { loop_over(smallest(om)); return; }
@@ -259,7 +260,14 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   p.B = (const T*)B.p;
   p.C = (T*)C.p;
   if constexpr (std::is_same<T, double>::value) {
-    if (split16 && p.batch == 1 && p.kx == 1 && 2.0 * p.M * p.N * p.K >= X3_ROUTE_FLOPS && x3_contract(p, ws, s)) return;
+    if (split16 && p.batch == 1 && p.kx == 1 && 2.0 * p.M * p.N * p.K >= X3_ROUTE_FLOPS) {
+      if (q) q->flush();
+      if (x3_contract(p, ws, s)) return;
+    }
+    if (q) {
+      q->gemm(p, part);
+      return;
+    }
   }
   tc_gemm<T>(p, ws, s);
 }
@@ -271,6 +279,51 @@ struct Perm6 {
   int64_t sa[6], sc[6];
   int64_t total;
 };
+
+// Several elementwise operations in one launch: block b belongs to the one with first[i] <= b < first[i + 1] and takes 1024
+// of its elements.
+constexpr int ELTS = 14;
+struct EltGroup {
+  int n;
+  int first[ELTS + 1];
+  EltOp e[ELTS];
+};
+__global__ __launch_bounds__(256) void elt_group_kernel(const EltGroup a) {
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+  const EltOp& d = a.e[i];
+  const int64_t e0 = (int64_t)(blockIdx.x - a.first[i]) * 1024 + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t e = e0 + u * 256;
+    if (e >= d.total) return;
+    uint32_t r = (uint32_t)e;
+    int64_t oa = 0, oc = 0;
+    for (int k = d.rank - 1; k >= 0; --k) {
+      const uint32_t q = r / (uint32_t)d.ext[k], x = r - q * (uint32_t)d.ext[k];
+      r = q;
+      oa += x * d.sa[k];
+      oc += x * d.sc[k];
+    }
+    double v = d.A ? d.alpha * d.A[oa] : 0.0;
+    if (d.beta != 0.0) v += d.beta * d.C[oc];
+    d.C[oc] = v;
+  }
+}
+
+void elementwise(const std::vector<EltOp>& e, hipStream_t s) {
+  for (size_t at = 0; at < e.size();) {
+    EltGroup g{};
+    for (; at < e.size() && g.n < ELTS; ++at) {
+      CCX_CHECK(e[at].total < (1ll << 31), ERR_INTERNAL, "queued elementwise operation too large");
+      g.e[g.n] = e[at];
+      g.first[g.n + 1] = g.first[g.n] + (int)ceil_div(e[at].total, 1024);
+      ++g.n;
+    }
+    elt_group_kernel<<<(unsigned)g.first[g.n], 256, 0, s>>>(g);
+    CCX_HIP(hipGetLastError());
+  }
+}
 
 template <typename T>
 __global__ void axpby_kernel(Perm6 d, T alpha, const T* __restrict__ A, T beta, T* __restrict__ C) {
@@ -298,8 +351,34 @@ static void launch_perm(const Perm6& d, T alpha, const T* A, T beta, T* C, hipSt
   CCX_HIP(hipGetLastError());
 }
 
+// into the queue while a launch is what it costs; a large one is launched, behind what it may meet
+static void launch_perm(const Perm6& d, double alpha, const double* A, double beta, double* C, hipStream_t s, GemmQueue* q) {
+  if (!q) {
+    launch_perm<double>(d, alpha, A, beta, C, s);
+    return;
+  }
+  if (d.total > ELT_QUEUE) {
+    q->flush();
+    launch_perm<double>(d, alpha, A, beta, C, s);
+    return;
+  }
+  EltOp e{};
+  e.rank = d.rank;
+  for (int k = 0; k < d.rank; ++k) {
+    e.ext[k] = d.ext[k];
+    e.sa[k] = d.sa[k];
+    e.sc[k] = d.sc[k];
+  }
+  e.total = d.total;
+  e.alpha = alpha;
+  e.beta = beta;
+  e.A = A;
+  e.C = C;
+  q->axpby(e, d.total);
+}
+
 template <typename T>
-void axpby(T alpha, const TV& A, T beta, const TV& C, hipStream_t s) {
+void axpby(T alpha, const TV& A, T beta, const TV& C, hipStream_t s, GemmQueue* q) {
   CCX_CHECK(A.rank() == C.rank() && C.rank() <= 6, ERR_ARG, "axpby rank");
   Perm6 d{};
   d.rank = C.rank();
@@ -312,11 +391,12 @@ void axpby(T alpha, const TV& A, T beta, const TV& C, hipStream_t s) {
     d.sa[k] = A.str[a];
     d.total *= C.ext[k];
   }
-  launch_perm<T>(d, alpha, (const T*)A.p, beta, (T*)C.p, s);
+  if constexpr (std::is_same<T, double>::value) launch_perm(d, alpha, (const T*)A.p, beta, (T*)C.p, s, q);
+  else launch_perm<T>(d, alpha, (const T*)A.p, beta, (T*)C.p, s);
 }
 
 template <typename T>
-void scale(T beta, const TV& C, hipStream_t s) {
+void scale(T beta, const TV& C, hipStream_t s, GemmQueue* q) {
   Perm6 d{};
   d.rank = C.rank();
   d.total = 1;
@@ -326,14 +406,16 @@ void scale(T beta, const TV& C, hipStream_t s) {
     d.sa[k] = 0;
     d.total *= C.ext[k];
   }
-  launch_perm<T>(d, T(0), (const T*)nullptr, beta, (T*)C.p, s);
+  if constexpr (std::is_same<T, double>::value) launch_perm(d, T(0), (const T*)nullptr, beta, (T*)C.p, s, q);
+  else launch_perm<T>(d, T(0), (const T*)nullptr, beta, (T*)C.p, s);
 }
 
-template void contract<double>(double, const TV&, const TV&, double, const TV&, Workspace&, hipStream_t, bool);
-template void contract<float>(float, const TV&, const TV&, float, const TV&, Workspace&, hipStream_t, bool);
-template void axpby<double>(double, const TV&, double, const TV&, hipStream_t);
-template void axpby<float>(float, const TV&, float, const TV&, hipStream_t);
-template void scale<double>(double, const TV&, hipStream_t);
-template void scale<float>(float, const TV&, hipStream_t);
+template void contract<double>(double, const TV&, const TV&, double, const TV&, Workspace&, hipStream_t, bool, GemmQueue*,
+                               int);
+template void contract<float>(float, const TV&, const TV&, float, const TV&, Workspace&, hipStream_t, bool, GemmQueue*, int);
+template void axpby<double>(double, const TV&, double, const TV&, hipStream_t, GemmQueue*);
+template void axpby<float>(float, const TV&, float, const TV&, hipStream_t, GemmQueue*);
+template void scale<double>(double, const TV&, hipStream_t, GemmQueue*);
+template void scale<float>(float, const TV&, hipStream_t, GemmQueue*);
 
 }  // namespace ccx

@@ -2,6 +2,7 @@
 #pragma once
 #include "common.h"
 #include <algorithm>
+#include <string>
 #include <vector>
 
 namespace ccx {
@@ -47,6 +48,45 @@ struct Workspace {
 
 template <typename T>
 void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s);
+
+// One elementwise operation of a queue: C = alpha A + beta C over rank <= 6 dimensions (A null: no term).
+struct EltOp {
+  int rank;
+  int64_t ext[6], sa[6], sc[6], total;
+  double alpha, beta;
+  const double* A;
+  double* C;
+};
+// Independent elementwise operations in as few launches as they fit (contract.hip).
+void elementwise(const std::vector<EltOp>& e, hipStream_t s);
+
+// Small FP64 contractions and elementwise operations gathered into few launches. An operation is queued while it does
+// not meet a queued one (none reads or writes what another writes; ranges of addresses decide) and flush() runs
+// first when it does, so the results are those of the calls in program order. A contraction over GROUP_TILES 64 x 64
+// tiles or GROUP_FLOPS flops fills the chip by itself and is launched when it is added. `part`: two operations with
+// different nonzero parts write disjoint elements even where their ranges overlap. Whoever launches a kernel of another
+// kind that meets a queued operation flushes first; a queue ends with flush().
+constexpr int64_t GROUP_TILES = 8192;
+constexpr double GROUP_FLOPS = 4e10;
+class GemmQueue {
+ public:
+  GemmQueue(Workspace& ws, hipStream_t s);
+  ~GemmQueue();
+  GemmQueue(const GemmQueue&) = delete;
+  GemmQueue& operator=(const GemmQueue&) = delete;
+  void gemm(const GemmParams<double>& p, int part = 0);
+  void axpby(const EltOp& e, int64_t n);
+  void flush();
+  bool empty() const;
+
+ private:
+  struct Op;
+  struct Elt;
+  Workspace& ws;
+  hipStream_t s;
+  std::vector<Op> ops;
+  std::vector<Elt> elts;
+};
 
 // Plain strided matrices (gemm_plain.hip): C[b][m * ldc + n] = alpha op(A) op(B) + beta C.
 template <typename T>

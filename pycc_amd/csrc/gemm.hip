@@ -52,13 +52,14 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t w, int64_t ntiles) {
 // C[b][m][n] = alpha sum_(x, k) A[b][m][x, k] B[b][x, k][n] + beta C: M, N and K are 2-level indices, x an
 // outer third level of K (its strides a_x, b_x), b the batch.
 //
-// What bounds it: a 16x16x4 FP64 MFMA holds a SIMD for 64 cycles, so a k-tile of a 128 x 128 tile is 8192
-// matrix cycles per CU against 16 8-byte loads per thread: the matrix cores, as long as some wave always has
-// one to issue. Hence 8 waves of 64 x 32 per work-group and two work-groups per CU (4 waves per SIMD, 128
-// registers), where 4 waves of 64 x 64 (2 per SIMD) stand still at every barrier; and hence plain 8-byte
-// loads whose addresses come from a multiply-high division per k index: any strides, odd extents and
-// remainders run the same loop. Rows past M or N read row M - 1 or N - 1 (their outputs are not stored); k past
-// its end reads the last k and is zeroed on its way into LDS.
+// What bounds it: a 16x16x4 FP64 MFMA holds a SIMD for 64 cycles, so the matrix cores, as long as some wave always has
+// one to issue: 8 waves of 64 x 32 per 128 x 128 work-group, two work-groups per CU (4 waves per SIMD, 128 registers).
+// Measured at 8192^3: 59-62 TF; 70-74 TF with the global loads and LDS writes left out, each of which costs the
+// matrix cores about 10% however early it is issued (a third LDS stage, two k-tiles in flight and 32-wide k-tiles
+// changed nothing), so loads and LDS writes are 16 bytes wherever pairs are contiguous (57 TF with 8-byte ones). Addresses
+// come from an odometer per k-tile, so any strides, odd extents and remainders run the same loop: 2793^3 with odd
+// leading dimensions takes 0.76 ms (0.99 with guarded 8-byte loads). Rows past M or N read row M - 1 or N - 1
+// (their outputs are not stored); k past its end reads a valid k and is zeroed on its way into LDS.
 //
 // LDS: a k-fast tile is [rows][BK + 2] (FP32: BK + 1) and a row-fast one [BK][rows + 16]: the two k rows of a half wave's
 // fragment read start 4 (k-fast: rows start 36 banks) or 32 banks apart, so reads are free of conflicts.
@@ -239,22 +240,20 @@ struct GLoader {
   }
 };
 
+// One work-group's tile `t` (of tiles_m x tiles_n), batch entry and split.
 template <typename T, int BM, int BN, int WM, int WN, int BK, bool AKF, bool BKF, typename Off, int V>
-__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kernel(TileGemm<T> p) {
+__device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int bidx, int sidx, int64_t nbatch,
+                                          GTile<T, BM, BK, AKF>* As, GTile<T, BN, BK, BKF>* Bs) {
   constexpr int NWN = BN / WN, NT = 64 * (BM / WM) * NWN, NBI = WM / 16, NBJ = WN / 16;
   typedef typename AccT<T>::type acc_t;
-  __shared__ GTile<T, BM, BK, AKF> As[2];
-  __shared__ GTile<T, BN, BK, BKF> Bs[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / NWN, wn = wave % NWN;
 
   const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  const int64_t t = xcd_remap(blockIdx.x, (int64_t)tiles_m * tiles_n);
   // 8 tile-rows together, so that concurrently running tiles share A and B panels
   const int64_t group = t / (8 * tiles_n);
   const int first_m = (int)group * 8, gsize = tiles_m - first_m < 8 ? tiles_m - first_m : 8;
   const int within = (int)(t - group * 8 * tiles_n);
   const int m0 = (first_m + within % gsize) * BM, n0 = within / gsize * BN;
-  const int bidx = blockIdx.y / p.splits, sidx = blockIdx.y % p.splits;
 
   const int ntk = (p.K + BK - 1) / BK;   // k-tiles of one x
   int kt = sidx * p.chunk;               // first and end k-tile of this split, over x and k
@@ -364,7 +363,7 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kerne
         }
       }
   } else {
-    T* W = p.work + ((int64_t)sidx * (gridDim.y / p.splits) + bidx) * p.M * p.N;
+    T* W = p.work + ((int64_t)sidx * nbatch + bidx) * p.M * p.N;
 #pragma unroll
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
@@ -378,6 +377,99 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kerne
         }
       }
   }
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int BK, bool AKF, bool BKF, typename Off, int V>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kernel(TileGemm<T> p) {
+  __shared__ GTile<T, BM, BK, AKF> As[2];
+  __shared__ GTile<T, BN, BK, BKF> Bs[2];
+  const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  tile_body<T, BM, BN, WM, WN, BK, AKF, BKF, Off, V>(p, xcd_remap(blockIdx.x, tiles), blockIdx.y / p.splits,
+                                                     blockIdx.y % p.splits, gridDim.y / p.splits, As, Bs);
+}
+
+// Several small independent FP64 contractions in one launch (GemmQueue): 64 x 64 tiles, block b belongs to the
+// contraction with first[i] <= b < first[i + 1]. What bounds them one by one is the launch: at o=5 v=19 and
+// o=9 v=61 a contraction takes 4.5 us to be launched and 4 to 15 to run a handful of work-groups.
+constexpr int GROUP = 12;
+struct GemmGroup {
+  int n;
+  int first[GROUP + 1];
+  int form[GROUP];      // 1: A k-fast, 2: B k-fast, 4: pairs
+  int batch[GROUP];
+  TileGemm<double> g[GROUP];
+};
+template <bool AKF, bool BKF, int V>
+__device__ __forceinline__ void group_body(const TileGemm<double>& p, int nbatch, int local, char* lds) {
+  typedef GTile<double, 64, 16, AKF> TA;
+  typedef GTile<double, 64, 16, BKF> TB;
+  const int tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), y = local / tiles;
+  tile_body<double, 64, 64, 32, 32, 16, AKF, BKF, uint32_t, V>(p, local - y * tiles, y / p.splits, y % p.splits, nbatch,
+                                                               (TA*)lds, (TB*)(lds + 2 * sizeof(TA)));
+}
+__global__ __launch_bounds__(256, 4) void tile_group_kernel(const GemmGroup a) {
+  constexpr size_t ROWS = sizeof(GTile<double, 64, 16, false>), KFAST = sizeof(GTile<double, 64, 16, true>);
+  __shared__ alignas(16) char lds[4 * (ROWS > KFAST ? ROWS : KFAST)];
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+  const int local = blockIdx.x - a.first[i], nb = a.batch[i];
+  const TileGemm<double> g = a.g[i];   // one copy, in scalar registers
+  switch (a.form[i]) {
+    case 0: group_body<false, false, 1>(g, nb, local, lds); break;
+    case 1: group_body<true, false, 1>(g, nb, local, lds); break;
+    case 2: group_body<false, true, 1>(g, nb, local, lds); break;
+    case 3: group_body<true, true, 1>(g, nb, local, lds); break;
+    case 4: group_body<false, false, 2>(g, nb, local, lds); break;
+    case 5: group_body<true, false, 2>(g, nb, local, lds); break;
+    case 6: group_body<false, true, 2>(g, nb, local, lds); break;
+    default: group_body<true, true, 2>(g, nb, local, lds); break;
+  }
+}
+
+// The split-K sums of a group: 64 outputs and 4 groups of splits per block (more than FIXED_K_SPLITS splits), or 256
+// outputs with their partials in order.
+struct SumGroup {
+  int n;
+  int first[GROUP + 1];
+  int64_t batch[GROUP];
+  TileGemm<double> g[GROUP];
+};
+__global__ __launch_bounds__(256) void sum_group_kernel(const SumGroup a) {
+  __shared__ double part[4][64];
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+  const TileGemm<double>& p = a.g[i];
+  const int local = blockIdx.x - a.first[i];
+  const int64_t total = a.batch[i] * p.M * p.N;
+  const bool wide = p.splits > FIXED_K_SPLITS;
+  const int G = wide ? 4 : 1, g = wide ? threadIdx.x >> 6 : 0;
+  const int64_t e = wide ? (int64_t)local * 64 + (threadIdx.x & 63) : (int64_t)local * 256 + threadIdx.x;
+  double s = 0;
+  if (e < total) {
+    const double* w = p.work + e;
+    int k = g;
+    for (; k + 7 * G < p.splits; k += 8 * G) {
+      double x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = w[(int64_t)(k + u * G) * total];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += x[u];
+    }
+    for (; k < p.splits; k += G) s += w[(int64_t)k * total];
+  }
+  if (wide) {
+    part[g][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (g > 0) return;
+    s = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+  }
+  if (e >= total) return;
+  const uint32_t mn = (uint32_t)p.M * (uint32_t)p.N, b = (uint32_t)(e / mn), r = (uint32_t)(e - (int64_t)b * mn);
+  const uint32_t m = r / (uint32_t)p.N;
+  double* dst = p.C + b * p.c_b + off2(p.cm, m) + off2(p.cn, r - m * (uint32_t)p.N);
+  double v = p.alpha * s;
+  if (p.beta != 0.0) v += p.beta * *dst;
+  *dst = v;
 }
 
 template <typename T, int BM, int BN, int WM, int WN, typename Off, int V>
@@ -563,12 +655,13 @@ static bool as_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
 struct Plan {
   int tile = 128, splits = 1, chunk = 0;
 };
-static Plan plan_f64(const GemmParams<double>& p, size_t limit) {
+static Plan plan_f64(const GemmParams<double>& p, size_t limit, int cus = 256, bool only64 = false) {
   static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128, 192, 256};
   const int64_t ntk = std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx);
   Plan best;
   double t_best = 0.0;
   for (int tile : {128, 64}) {
+    if (only64 && tile != 64) continue;
     const int64_t tiles = ceil_div(p.M, tile) * ceil_div(p.N, tile) * p.batch;
     const double t_ktile = 2.0 * tile * tile * 16 / 0.24e6;
     const int per_cu = tile == 128 ? 2 : 4;   // resident work-groups (LDS)
@@ -577,7 +670,7 @@ static Plan plan_f64(const GemmParams<double>& p, size_t limit) {
       if (want > 1 && (chunk < 4 || splits * p.batch > 65535)) break;
       const double bytes = 8.0 * (double)splits * (double)p.batch * (double)p.M * (double)p.N;
       if (want > 1 && bytes > (double)limit) break;
-      const int64_t on_cu = ceil_div(tiles * splits, 256);
+      const int64_t on_cu = ceil_div(tiles * splits, cus);
       double t = 6.0 + (double)chunk * (0.25 * (double)ceil_div(on_cu, per_cu) + (double)on_cu * t_ktile);
       if (splits > 1) t += 5.0 + 2.0 * bytes / 4.0e6;
       if (t_best == 0.0 || t < t_best) {
@@ -620,37 +713,45 @@ static Plan plan_fixed(const GemmParams<T>& p, size_t limit) {
   return r;
 }
 static Plan plan(const GemmParams<float>& p, const Workspace& ws) { return plan_fixed(p, ws.limit); }
-static Plan plan(const GemmParams<double>& p, const Workspace& ws) {
+static Plan plan(const GemmParams<double>& p, const Workspace& ws, int cus = 256, bool only64 = false) {
   if (ws.fixed_k) {
     Plan f = plan_fixed(p, ws.limit);
     if (f.splits <= FIXED_K_SPLITS) {   // the tile is free
-      if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch * f.splits < 512) f.tile = 64;
+      if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch * f.splits < 512 || only64) f.tile = 64;
       return f;
     }
   }
-  return plan_f64(p, ws.limit);
+  return plan_f64(p, ws.limit, cus, only64);
+}
+
+// How a contraction is loaded: which operands are k-fast, lane offsets in 32 bits, pairs.
+struct Form {
+  bool akf, bkf, off32, two;
+};
+template <typename T>
+static Form form_of(const GemmParams<T>& p, int tile) {
+  Form f;
+  // A is "k-fast" when its inner k index is contiguous (coalesced loads along k); otherwise the
+  // loader walks along m. Same for B with n.
+  f.akf = !(p.am.s2 == 1 && p.ak.s2 != 1);
+  f.bkf = !(p.bn.s2 == 1 && p.bk.s2 != 1);
+  // lane offsets in 32 bits: what a lane adds to the uniform base stays under 4 GiB -- the rows, and k where it is
+  // not the same in a whole wave (k-fast, and pairs of rows in a 64-wide tile)
+  auto narrow = [&](const Idx2& r, int64_t nr, const Idx2& k, bool with_k) {
+    const int64_t a = span(r, nr), b = with_k ? span(k, std::max<int64_t>(p.K, 1)) : 0;
+    return a >= 0 && b >= 0 && (a + b + 1) * (int64_t)sizeof(T) <= (1ll << 32);
+  };
+  f.off32 = narrow(p.am, p.M, p.ak, f.akf) && narrow(p.bn, p.N, p.bk, f.bkf);
+  // pairs along the contiguous index of both operands
+  auto pairs = [](const Idx2& d, int64_t n) { return d.s2 == 1 && n >= 2 && (d.n2 % 2 == 0 || n <= d.n2); };
+  f.two = sizeof(T) == 8 && f.off32 &&
+          (tile == 128 || (narrow(p.am, p.M, p.ak, true) && narrow(p.bn, p.N, p.bk, true))) &&
+          pairs(f.akf ? p.ak : p.am, f.akf ? p.K : p.M) && pairs(f.bkf ? p.bk : p.bn, f.bkf ? p.K : p.N);
+  return f;
 }
 
 template <typename T>
-void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
-  if (p.M == 0 || p.N == 0 || p.batch == 0) return;
-  {
-    // enough 128 x 128 tiles to fill the 256 CUs: the plain-matrix kernel
-    PlainGemm<T> q;
-    if (p.kx == 1 && ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q)) {
-      plain_dispatch<T>(q, ws, s);
-      return;
-    }
-  }
-  CCX_CHECK(p.M < (1ll << 31) && p.N < (1ll << 31) && p.K < (1ll << 31) && p.K * p.kx < (1ll << 31), ERR_ARG,
-            "gemm extent too large");
-  CCX_CHECK(p.batch < 65536, ERR_ARG, "gemm batch too large");
-  // A is "k-fast" when its inner k index is contiguous (coalesced loads along k); otherwise the
-  // loader walks along m. Same for B with n.
-  const bool akf = !(p.am.s2 == 1 && p.ak.s2 != 1);
-  const bool bkf = !(p.bn.s2 == 1 && p.bk.s2 != 1);
-  const Plan pl = plan(p, ws);
-  CCX_CHECK(ceil_div(p.M, pl.tile) * ceil_div(p.N, pl.tile) < (1ll << 31), ERR_ARG, "gemm grid too large");
+static TileGemm<T> describe(const GemmParams<T>& p, const Plan& pl) {
   TileGemm<T> g;
   g.M = (int)p.M;
   g.N = (int)p.N;
@@ -674,30 +775,190 @@ void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
   g.A = p.A;
   g.B = p.B;
   g.C = p.C;
-  g.work = pl.splits > 1 ? (T*)ws.get((size_t)pl.splits * p.batch * p.M * p.N * sizeof(T)) : nullptr;
+  g.work = nullptr;
+  return g;
+}
+
+template <typename T>
+static void check_extents(const GemmParams<T>& p) {
+  CCX_CHECK(p.M < (1ll << 31) && p.N < (1ll << 31) && p.K < (1ll << 31) && p.K * p.kx < (1ll << 31), ERR_ARG,
+            "gemm extent too large");
+  CCX_CHECK(p.batch < 65536, ERR_ARG, "gemm batch too large");
+}
+
+template <typename T>
+void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
+  if (p.M == 0 || p.N == 0 || p.batch == 0) return;
+  {
+    // enough 128 x 128 tiles to fill the 256 CUs: the plain-matrix kernel
+    PlainGemm<T> q;
+    if (p.kx == 1 && ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q)) {
+      plain_dispatch<T>(q, ws, s);
+      return;
+    }
+  }
+  check_extents(p);
+  const Plan pl = plan(p, ws);
+  CCX_CHECK(ceil_div(p.M, pl.tile) * ceil_div(p.N, pl.tile) < (1ll << 31), ERR_ARG, "gemm grid too large");
+  TileGemm<T> g = describe(p, pl);
+  if (pl.splits > 1) g.work = (T*)ws.get((size_t)pl.splits * p.batch * p.M * p.N * sizeof(T));
+  const Form f = form_of(p, pl.tile);
   if (std::getenv("CCX_TRACE"))
-    std::fprintf(stderr, "[ccx]   -> tile %d%s%s batch %lld splits %d\n", pl.tile, akf ? " Ak" : " Am",
-                 bkf ? " Bk" : " Bn", (long long)p.batch, pl.splits);
-  // lane offsets in 32 bits: what a lane adds to the uniform base stays under 4 GiB -- the rows, and k where it is
-  // not the same in a whole wave (k-fast, and pairs of rows in a 64-wide tile)
-  auto narrow = [&](const Idx2& r, int64_t nr, const Idx2& k, bool with_k) {
-    const int64_t a = span(r, nr), b = with_k ? span(k, std::max<int64_t>(p.K, 1)) : 0;
-    return a >= 0 && b >= 0 && (a + b + 1) * (int64_t)sizeof(T) <= (1ll << 32);
-  };
-  const bool off32 = narrow(p.am, p.M, p.ak, akf) && narrow(p.bn, p.N, p.bk, bkf);
-  // pairs along the contiguous index of both operands
-  auto pairs = [](const Idx2& d, int64_t n) { return d.s2 == 1 && n >= 2 && (d.n2 % 2 == 0 || n <= d.n2); };
-  const bool two = off32 && (pl.tile == 128 || (narrow(p.am, p.M, p.ak, true) && narrow(p.bn, p.N, p.bk, true))) &&
-                   pairs(akf ? p.ak : p.am, akf ? p.K : p.M) && pairs(bkf ? p.bk : p.bn, bkf ? p.K : p.N);
+    std::fprintf(stderr, "[ccx]   -> tile %d%s%s batch %lld splits %d\n", pl.tile, f.akf ? " Ak" : " Am",
+                 f.bkf ? " Bk" : " Bn", (long long)p.batch, pl.splits);
   if constexpr (sizeof(T) == 8) {
-    if (two) launch_tile<T, uint32_t, 2>(pl.tile, g, p.batch, akf, bkf, s);
-    else if (off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
-    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+    if (f.two) launch_tile<T, uint32_t, 2>(pl.tile, g, p.batch, f.akf, f.bkf, s);
+    else if (f.off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
+    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
   } else {
-    if (off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
-    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, akf, bkf, s);
+    if (f.off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
+    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
   }
   if (pl.splits > 1) splitk_reduce<T>(p, g.work, pl.splits, s);
+}
+
+// ---- GemmQueue ------------------------------------------------------------------------------------
+namespace {
+// addresses [lo, hi) that an operand spans
+struct Range {
+  uintptr_t lo = 0, hi = 0;
+  bool meets(const Range& o) const { return lo < o.hi && o.lo < hi; }
+};
+Range range_of(const double* base, std::initializer_list<std::pair<int64_t, int64_t>> dims) {
+  int64_t lo = 0, hi = 0;   // (extent, stride)
+  for (auto& d : dims) {
+    const int64_t e = (d.first - 1) * d.second;
+    (e < 0 ? lo : hi) += e;
+  }
+  return Range{(uintptr_t)(base + lo), (uintptr_t)(base + hi + 1)};
+}
+Range range_of(const double* base, const Idx2& r, int64_t nr, const Idx2& c, int64_t nc, int64_t nx, int64_t sx, int64_t nb,
+               int64_t sb) {
+  return range_of(base, {{std::min(nr, r.n2), r.s2}, {(nr - 1) / r.n2 + 1, r.s1}, {std::min(nc, c.n2), c.s2},
+                         {(nc - 1) / c.n2 + 1, c.s1}, {nx, sx}, {nb, sb}});
+}
+}  // namespace
+
+struct GemmQueue::Op {
+  GemmParams<double> p;
+  Range a, b, c;
+  int part;
+};
+struct GemmQueue::Elt {
+  EltOp op;
+  Range a, c;
+};
+
+GemmQueue::GemmQueue(Workspace& w, hipStream_t st) : ws(w), s(st) {}
+GemmQueue::~GemmQueue() {}
+
+bool GemmQueue::empty() const { return ops.empty() && elts.empty(); }
+
+void GemmQueue::axpby(const EltOp& e, int64_t n) {
+  if (n == 0) return;
+  Elt x{e, Range{}, Range{}};
+  auto range = [&](const double* p, const int64_t* str) {
+    int64_t hi = 0;
+    for (int k = 0; k < e.rank; ++k) hi += (e.ext[k] - 1) * str[k];
+    return Range{(uintptr_t)p, (uintptr_t)(p + hi + 1)};
+  };
+  if (e.A) x.a = range(e.A, e.sa);
+  x.c = range(e.C, e.sc);
+  bool clash = false;   // it runs before the queued contractions, and beside the queued elementwise ones
+  for (auto& o : ops) clash = clash || x.c.meets(o.a) || x.c.meets(o.b) || x.c.meets(o.c) || x.a.meets(o.c);
+  for (auto& o : elts) clash = clash || x.c.meets(o.a) || x.c.meets(o.c) || x.a.meets(o.c);
+  if (clash) flush();
+  elts.push_back(x);
+}
+
+void GemmQueue::gemm(const GemmParams<double>& p, int part) {
+  if (p.M == 0 || p.N == 0 || p.batch == 0) return;
+  check_extents(p);
+  Op o{p, Range{}, Range{}, range_of(p.C, p.cm, p.M, p.cn, p.N, 1, 0, p.batch, p.c_b), part};
+  if (p.K > 0) {
+    o.a = range_of(p.A, p.am, p.M, p.ak, p.K, p.kx, p.a_x, p.batch, p.a_b);
+    o.b = range_of(p.B, p.bn, p.N, p.bk, p.K, p.kx, p.b_x, p.batch, p.b_b);
+  }
+  for (auto& q : ops) {
+    const bool apart = part && q.part && part != q.part;   // the caller's word that the outputs do not meet
+    if ((!apart && o.c.meets(q.c)) || o.c.meets(q.a) || o.c.meets(q.b) || o.a.meets(q.c) || o.b.meets(q.c)) {
+      flush();
+      break;
+    }
+  }
+  const int64_t tiles = ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batch;
+  if (tiles > GROUP_TILES || 2.0 * p.M * p.N * p.K * p.kx * p.batch > GROUP_FLOPS || !form_of(p, 64).off32) {
+    // it fills the chip by itself: now, before the queued ones, which it does not meet
+    bool clash = false;
+    for (auto& e : elts) clash = clash || o.a.meets(e.c) || o.b.meets(e.c) || o.c.meets(e.c) || o.c.meets(e.a);
+    if (clash) flush();
+    tc_gemm<double>(p, ws, s);
+    return;
+  }
+  ops.push_back(o);
+}
+
+void GemmQueue::flush() {
+  if (!elts.empty()) {
+    std::vector<EltOp> e;
+    for (auto& x : elts) e.push_back(x.op);
+    elts.clear();
+    elementwise(e, s);
+  }
+  std::vector<Op> todo;
+  todo.swap(ops);
+  for (size_t at = 0; at < todo.size();) {
+    if (todo.size() - at == 1) {
+      tc_gemm<double>(todo[at].p, ws, s);
+      return;
+    }
+    // planned for their share of the chip, the longest first
+    const size_t left = std::min<size_t>(todo.size() - at, GROUP);
+    const int cus = std::max<int>(32, 256 / (int)left);
+    struct Item {
+      const Op* o;
+      Plan pl;
+    };
+    std::vector<Item> items;
+    size_t bytes = 0;
+    for (; items.size() < left; ++at) {
+      const GemmParams<double>& p = todo[at].p;
+      const Plan pl = plan(p, ws, cus, true);
+      const size_t w = pl.splits > 1 ? (size_t)pl.splits * p.batch * p.M * p.N * sizeof(double) : 0;
+      if (!items.empty() && bytes + w > ws.limit) break;
+      bytes += w;
+      items.push_back(Item{&todo[at], pl});
+    }
+    std::stable_sort(items.begin(), items.end(), [](const Item& x, const Item& y) { return x.pl.chunk > y.pl.chunk; });
+    double* work = bytes ? (double*)ws.get(bytes) : nullptr;
+    GemmGroup a{};
+    SumGroup r{};
+    for (const Item& it : items) {
+      const GemmParams<double>& p = it.o->p;
+      TileGemm<double> g = describe(p, it.pl);
+      const Form f = form_of(p, 64);
+      const int64_t outputs = p.batch * p.M * p.N;
+      if (it.pl.splits > 1) {
+        g.work = work;
+        work += it.pl.splits * outputs;
+        r.g[r.n] = g;
+        r.batch[r.n] = p.batch;
+        r.first[r.n + 1] = r.first[r.n] + (int)ceil_div(outputs, it.pl.splits > FIXED_K_SPLITS ? 64 : 256);
+        ++r.n;
+      }
+      a.g[a.n] = g;
+      a.batch[a.n] = (int)p.batch;
+      a.form[a.n] = (f.akf ? 1 : 0) + (f.bkf ? 2 : 0) + (f.two ? 4 : 0);
+      a.first[a.n + 1] = a.first[a.n] + (int)(ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batch * it.pl.splits);
+      ++a.n;
+    }
+    tile_group_kernel<<<(unsigned)a.first[a.n], 256, 0, s>>>(a);
+    CCX_HIP(hipGetLastError());
+    if (r.n) {
+      sum_group_kernel<<<(unsigned)r.first[r.n], 256, 0, s>>>(r);
+      CCX_HIP(hipGetLastError());
+    }
+  }
 }
 
 template void tc_gemm<double>(const GemmParams<double>&, Workspace&, hipStream_t);

@@ -47,9 +47,11 @@ __global__ void unpack_vvvv_kernel(int64_t o, int64_t v, const double* __restric
   }
 }
 
-// out[i][j][a][b] = alpha * (h[i][j][a][b] + h[j][i][b][a]), through 32 x 33 LDS tiles.
-__global__ __launch_bounds__(256) void pair_sym_kernel(int64_t o, int64_t v, double alpha,
+// out[i][j][a][b] = alpha * (h[i][j][a][b] + h[j][i][b][a]), through 32 x 33 LDS tiles; h is the sum of `parts` arrays,
+// one after the other (HalfSum below).
+__global__ __launch_bounds__(256) void pair_sym_kernel(int64_t o, int64_t v, double alpha, int parts,
                                                        const double* __restrict__ h, double* __restrict__ out) {
+  const int64_t size = o * o * v * v;
   __shared__ double sh[32][33];
   const int64_t ij = blockIdx.y, i = ij / o, j = ij % o;
   const int64_t tiles_b = (v + 31) / 32;
@@ -57,14 +59,19 @@ __global__ __launch_bounds__(256) void pair_sym_kernel(int64_t o, int64_t v, dou
   const int x = threadIdx.x & 31, y0 = threadIdx.x >> 5;
   for (int y = y0; y < 32; y += 8) {
     const int64_t a = a0 + x, b = b0 + y;
-    sh[y][x] = (a < v && b < v) ? h[((j * o + i) * v + b) * v + a] : 0.0;
+    double t = 0.0;
+    if (a < v && b < v)
+      for (int p = 0; p < parts; ++p) t += h[p * size + ((j * o + i) * v + b) * v + a];
+    sh[y][x] = t;
   }
   __syncthreads();
   for (int y = y0; y < 32; y += 8) {
     const int64_t a = a0 + y, b = b0 + x;
     if (a >= v || b >= v) continue;
     const int64_t e = ((i * o + j) * v + a) * v + b;
-    out[e] = alpha * (h[e] + sh[x][y]);
+    double t = 0.0;
+    for (int p = 0; p < parts; ++p) t += h[p * size + e];
+    out[e] = alpha * (t + sh[x][y]);
   }
 }
 
@@ -123,10 +130,10 @@ __global__ void sum_terms_kernel(int n, const double* __restrict__ x, double* __
 
 }  // namespace
 
-void pair_symmetrize(int64_t o, int64_t v, double alpha, const double* h, double* out, hipStream_t s) {
+void pair_symmetrize(int64_t o, int64_t v, double alpha, int parts, const double* h, double* out, hipStream_t s) {
   CCX_CHECK(o * o < 65536, ERR_ARG, "too many occupied orbitals for the pair grid");
   int64_t tiles = ceil_div(v, 32);
-  pair_sym_kernel<<<dim3((unsigned)(tiles * tiles), (unsigned)(o * o)), 256, 0, s>>>(o, v, alpha, h, out);
+  pair_sym_kernel<<<dim3((unsigned)(tiles * tiles), (unsigned)(o * o)), 256, 0, s>>>(o, v, alpha, parts, h, out);
   CCX_HIP(hipGetLastError());
 }
 
@@ -144,15 +151,19 @@ static void alloc_hbar(Ctx& c, bool stored) {
     c.Hovov = c.alloc<double>(ov * ov);
     c.Hovoo = c.alloc<double>(o * o * ov);
     c.Ltmp = c.alloc<double>(ov * ov);
+    const bool more = doubles_parts(ov * ov) > 1;   // one temporary for each of three independent products
+    c.Ltmp2 = more ? c.alloc<double>(ov * ov) : c.Ltmp;
+    c.Ltmp3 = more ? c.alloc<double>(ov * ov) : c.Ltmp;
     c.Goo = c.alloc<double>(o * o);
     c.Gvv = c.alloc<double>(v * v);
-    c.Lh = c.alloc<double>(ov * ov);
+    c.Lh = c.alloc<double>((size_t)doubles_parts(ov * ov) * ov * ov);
+    c.Lr = c.alloc<double>(SINGLES_PARTS * ov);
     c.Lsym = c.alloc<double>(ov * ov);
     c.LY = c.alloc<double>(ov * ov);
     c.LVf = c.alloc<double>(o * o * ov);
     c.LVg = c.alloc<double>(o * o * ov);
     c.LU = c.alloc<double>(o * o * o * o);
-    c.LQ = c.alloc<double>(o * o * ov);
+    c.LQ = c.alloc<double>(6 * o * o * ov);
     c.Lsm = c.alloc<double>(2 * o * o + 2 * ov);
     c.Jsm = c.alloc<double>(v * v + 4 * o * o + 2 * ov);
     c.have_hbar_bufs = true;
@@ -183,9 +194,11 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
   const std::vector<int64_t> OOOV{o, o, o, v}, OVVV{o, v, v, v}, OOOO{o, o, o, o}, VVVV{v, v, v, v};
   const std::vector<int64_t> VOVV{v, o, v, v}, OVVO{o, v, v, o}, VVVO{v, v, v, o}, OVOO{o, v, o, o};
   const bool x3 = c.mode == MODE_MIXED_F16X3;
+  GemmQueue q(ws, s);
   auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C) {
-    contract<double>(a, A, B, b, C, ws, s, x3);
+    contract<double>(a, A, B, b, C, ws, s, x3, &q);
   };
+  auto axpby = [&](double a, const TV& A, double b, const TV& C, hipStream_t) { ccx::axpby<double>(a, A, b, C, s, &q); };
   CCX_HIP(hipMemcpyAsync(c.Ht1, t1, ov * sizeof(double), hipMemcpyDeviceToDevice, s));
   CCX_HIP(hipMemcpyAsync(c.Ht2, t2, ov * ov * sizeof(double), hipMemcpyDeviceToDevice, s));
   auto T1 = [&](const char* l) { return tv(c.Ht1, l, OV); };
@@ -205,12 +218,12 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
 
   // ---- Hov: cchbar.py:152-153 ----
   const TV Hov = tv(c.Hov, "me", OV);
-  axpby<double>(1.0, Fov, 0.0, Hov, s);
+  axpby(1.0, Fov, 0.0, Hov, s);
   cd(1.0, T1("nf"), LOVV("mnef"), 1.0, Hov);
 
   // ---- Hvv: :206-209 (L_amef = 2(mf|ae) - (me|af)) ----
   const TV Hvv = tv(c.Hvv, "ae", VV);
-  axpby<double>(1.0, Fvv, 0.0, Hvv, s);
+  axpby(1.0, Fvv, 0.0, Hvv, s);
   cd(-1.0, Fov, T1("ma"), 1.0, Hvv);
   cd(2.0, T1("mf"), CVVV("mfae"), 1.0, Hvv);
   cd(-1.0, T1("mf"), CVVV("meaf"), 1.0, Hvv);
@@ -218,26 +231,26 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
 
   // ---- Hoo: :269-272 ----
   const TV Hoo = tv(c.Hoo, "mi", OO);
-  axpby<double>(1.0, Foo, 0.0, Hoo, s);
+  axpby(1.0, Foo, 0.0, Hoo, s);
   cd(1.0, T1("ie"), Fov, 1.0, Hoo);
   cd(1.0, T1("ne"), LOOV("imne"), 1.0, Hoo);
   cd(1.0, TAU("inef"), LOVV("mnef"), 1.0, Hoo);
 
   // ---- Hoooo: :331-337 -- <mn|ij> + t_je <mn|ie> + t_ie <nm|je> + tau_ijef <mn|ef> ----
   const TV Hoooo = tv(c.Hoooo, "mnij", OOOO);
-  axpby<double>(1.0, tv(c.Coooo, "minj", OOOO), 0.0, Hoooo, s);     // (mi|nj)
+  axpby(1.0, tv(c.Coooo, "minj", OOOO), 0.0, Hoooo, s);     // (mi|nj)
   cd(1.0, T1("je"), COOV("mine"), 1.0, Hoooo);                       // (mi|ne)
   cd(1.0, T1("ie"), COOV("njme"), 1.0, Hoooo);                       // (nj|me)
   cd(1.0, TAU("ijef"), IOVV("mnef"), 1.0, Hoooo);
 
   // ---- Hooov: :505-506 -- <mn|ie> + t_if <nm|ef> ----
   const TV Hooov = tv(c.Hooov, "mnie", OOOV);
-  axpby<double>(1.0, COOV("mine"), 0.0, Hooov, s);
+  axpby(1.0, COOV("mine"), 0.0, Hooov, s);
   cd(1.0, T1("if"), IOVV("nmef"), 1.0, Hooov);
 
   // ---- Hovvo: :563-568 -- <mb|ej> + t_jf <mb|ef> - t_nb <mn|ej> - tau_jnfb <mn|ef> + t_njfb L_mnef ----
   const TV Hovvo = tv(c.Hovvo, "mbej", OVVO);
-  axpby<double>(1.0, COVO("mejb"), 0.0, Hovvo, s);                  // (me|jb)
+  axpby(1.0, COVO("mejb"), 0.0, Hovvo, s);                  // (me|jb)
   cd(1.0, T1("jf"), CVVV("mebf"), 1.0, Hovvo);                       // (me|bf)
   cd(-1.0, T1("nb"), COOV("njme"), 1.0, Hovvo);                      // (nj|me)
   cd(-1.0, TAU("jnfb"), IOVV("mnef"), 1.0, Hovvo);
@@ -245,14 +258,14 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
 
   // ---- Hovov: :625-629 -- <mb|je> + t_jf <bm|ef> - t_nb <mn|je> - tau_jnfb <nm|ef> ----
   const TV Hovov = tv(c.Hovov, "mbje", OVOV);
-  axpby<double>(1.0, COVV("mjbe"), 0.0, Hovov, s);                  // (mj|be)
+  axpby(1.0, COVV("mjbe"), 0.0, Hovov, s);                  // (mj|be)
   cd(1.0, T1("jf"), CVVV("mfbe"), 1.0, Hovov);                       // <bm|ef> = (mf|be)
   cd(-1.0, T1("nb"), COOV("mjne"), 1.0, Hovov);                      // <mn|je> = (mj|ne)
   cd(-1.0, TAU("jnfb"), IOVV("nmef"), 1.0, Hovov);
 
   // ---- Hovoo: :806-819 ----
   const TV Hovoo = tv(c.Hovoo, "mbij", OVOO);
-  axpby<double>(1.0, COOV("mijb"), 0.0, Hovoo, s);                  // <mb|ij> = (mi|jb)    :806
+  axpby(1.0, COOV("mijb"), 0.0, Hovoo, s);                  // <mb|ij> = (mi|jb)    :806
   cd(1.0, Hov, T2("ijeb"), 1.0, Hovoo);                              //                      :807
   cd(-1.0, T1("nb"), Hoooo, 1.0, Hovoo);                             //                      :808
   cd(1.0, TAU("ijef"), CVVV("mebf"), 1.0, Hovoo);                    // <mb|ef> = (me|bf)    :809
@@ -261,13 +274,13 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
   cd(1.0, T2("njeb"), LOOV("imne"), 1.0, Hovoo);                     // L_mnie               :812
   {
     const TV tmp = tv(c.Ltmp, "mbie", OVOV);                        //                      :813-815
-    axpby<double>(1.0, COVV("mibe"), 0.0, tmp, s);                   // <mb|ie> = (mi|be)
+    axpby(1.0, COVV("mibe"), 0.0, tmp, s);                   // <mb|ie> = (mi|be)
     cd(-1.0, T2("infb"), IOVV("mnfe"), 1.0, tmp);
     cd(1.0, T1("je"), tmp, 1.0, Hovoo);
   }
   {
     const TV tmp = tv(c.Ltmp, "bmje", {v, o, o, v});                //                      :816-819
-    axpby<double>(1.0, COVO("mejb"), 0.0, tmp, s);                   // <bm|je> = (me|jb)
+    axpby(1.0, COVO("mejb"), 0.0, tmp, s);                   // <bm|je> = (me|jb)
     cd(-1.0, T2("jnfb"), IOVV("mnef"), 1.0, tmp);
     cd(1.0, T2("njfb"), LOVV("mnef"), 1.0, tmp);
     cd(1.0, T1("ie"), tmp, 1.0, Hovoo);
@@ -287,12 +300,12 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
 
     // ---- Hvovv: :455-456 -- <am|ef> - t_na <nm|ef> ----
     const TV Hvovv = tv(c.Hvovv, "amef", VOVV);
-    axpby<double>(1.0, CVVV("mfae"), 0.0, Hvovv, s);
+    axpby(1.0, CVVV("mfae"), 0.0, Hvovv, s);
     cd(-1.0, T1("na"), IOVV("nmef"), 1.0, Hvovv);
 
     // ---- Hvvvo: :682-695 ----
     const TV Hvvvo = tv(c.Hvvvo, "abei", VVVO);
-    axpby<double>(1.0, CVVV("ibae"), 0.0, Hvvvo, s);                // <ab|ei> = (ib|ae)    :682
+    axpby(1.0, CVVV("ibae"), 0.0, Hvvvo, s);                // <ab|ei> = (ib|ae)    :682
     cd(-1.0, Hov, T2("miab"), 1.0, Hvvvo);                           //                      :683
     cd(1.0, T1("if"), Hvvvv, 1.0, Hvvvo);                            //                      :684
     cd(1.0, TAU("mnab"), COOV("nime"), 1.0, Hvvvo);                  // <mn|ei> = (ni|me)    :685
@@ -302,18 +315,19 @@ void hbar_build(Ctx& c, const double* F, const double* t1, const double* t2, boo
     cd(-1.0, T2("mifb"), CVVV("meaf"), 1.0, Hvvvo);                  //        - (me|af)
     {
       const TV tmp = tv(c.Ltmp, "amei", {v, o, v, o});              //                      :689-691
-      axpby<double>(1.0, COVV("miae"), 0.0, tmp, s);                 // <am|ei> = (mi|ae)
+      axpby(1.0, COVV("miae"), 0.0, tmp, s);                 // <am|ei> = (mi|ae)
       cd(-1.0, T2("infa"), IOVV("mnfe"), 1.0, tmp);
       cd(-1.0, T1("mb"), tmp, 1.0, Hvvvo);
     }
     {
       const TV tmp = tv(c.Ltmp, "bmie", {v, o, o, v});              //                      :692-695
-      axpby<double>(1.0, COVO("meib"), 0.0, tmp, s);                 // <bm|ie> = (me|ib)
+      axpby(1.0, COVO("meib"), 0.0, tmp, s);                 // <bm|ie> = (me|ib)
       cd(-1.0, T2("infb"), IOVV("mnef"), 1.0, tmp);
       cd(1.0, T2("nifb"), LOVV("mnef"), 1.0, tmp);
       cd(-1.0, T1("ma"), tmp, 1.0, Hvvvo);
     }
   }
+  q.flush();
   c.have_hbar = true;
 }
 
@@ -355,8 +369,23 @@ void lambda_residual(Ctx& c, const double* l1, const double* l2, double* r1, dou
   const std::vector<int64_t> VOVV{v, o, v, v}, OVVO{o, v, v, o}, VVVO{v, v, v, o}, OVOO{o, v, o, o};
   const std::vector<int64_t> OOVO{o, o, v, o};
   const bool x3 = c.mode == MODE_MIXED_F16X3;
+  // The terms are ordered by what they depend on -- inputs and HBAR, then the intermediates, then Y -- and summed into
+  // partial sums, so that at small sizes the queue runs each level in one or two launches (at o=13 v=101
+  // 97 launches become about 40). At large sizes every term is launched by itself, as it comes.
+  GemmQueue q(ws, s);
   auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C) {
-    contract<double>(a, A, B, b, C, ws, s, x3);
+    contract<double>(a, A, B, b, C, ws, s, x3, &q);
+  };
+  PartSum r1s(c.Lr, ov, SINGLES_PARTS), r2s(c.Lh, ov * ov, doubles_parts(ov * ov));
+  auto R1 = [&](double a, const TV& A, const TV& B) {   // r_L1 += a A B
+    double beta;
+    double* p = r1s.take(beta);
+    cd(a, A, B, beta, tv(p, "ia", OV));
+  };
+  auto H = [&](double a, const TV& A, const TV& B) {    // r_L2 before P(ij,ab) += a A B
+    double beta;
+    double* p = r2s.take(beta);
+    cd(a, A, B, beta, tv(p, "ijab", OOVV));
   };
   auto L1 = [&](const char* l) { return tv(l1, l, OV); };
   auto L2 = [&](const char* l) { return tv(l2, l, OOVV); };
@@ -369,130 +398,135 @@ void lambda_residual(Ctx& c, const double* l1, const double* l2, double* r1, dou
   auto IOVV = [&](const char* l) { return tv(c.Ioovv, l, OOVV); };
   auto LOVV = [&](const char* l) { return tv(c.Loovv, l, OOVV); };
 
-  // ---- Goo, Gvv: cclambda.py:281, :306 ----
-  const TV Goo = tv(c.Goo, "mi", OO), Gvv = tv(c.Gvv, "ae", VV);
-  cd(1.0, T2("mjab"), L2("ijab"), 0.0, Goo);
-  cd(-1.0, T2("ijeb"), L2("ijab"), 0.0, Gvv);
-
-  // ---- r_L1: :348-369 ----
-  const TV R1 = tv(r1, "ia", OV);
-  if (with_source) axpby<double>(2.0, tv(c.Hov, "ia", OV), 0.0, R1, s);          // :348
-  else scale<double>(0.0, R1, s);
-  cd(1.0, L1("ie"), tv(c.Hvv, "ea", VV), 1.0, R1);                               // :354
-  cd(-1.0, L1("ma"), tv(c.Hoo, "im", OO), 1.0, R1);                              // :355
-  cd(-1.0, L2("mnae"), tv(c.Hovoo, "iemn", OVOO), 1.0, R1);                      // :357
-  cd(2.0, L1("me"), tv(c.Hovvo, "ieam", OVVO), 1.0, R1);                         // :358
-  cd(-1.0, L1("me"), tv(c.Hovov, "iema", OVOV), 1.0, R1);
-  cd(-2.0, relabel(Goo, "mn"), tv(c.Hooov, "mina", OOOV), 1.0, R1);              // :368
-  cd(1.0, relabel(Goo, "mn"), tv(c.Hooov, "imna", OOOV), 1.0, R1);               // :369
-
-  // ---- r_L2 before P(ij,ab): :468-494 ----
-  const TV H = tv(c.Lh, "ijab", OOVV);
-  if (with_source) axpby<double>(1.0, LOVV("ijab"), 0.0, H, s);                  // :468
-  else scale<double>(0.0, H, s);
-  cd(2.0, L1("ia"), tv(c.Hov, "jb", OV), 1.0, H);                                // :476
-  cd(-1.0, L1("ja"), tv(c.Hov, "ib", OV), 1.0, H);                               // :477
-  cd(-2.0, L1("mb"), tv(c.Hooov, "jima", OOOV), 1.0, H);                         // :480
-  cd(1.0, L1("mb"), tv(c.Hooov, "ijma", OOOV), 1.0, H);                          // :481
-  cd(1.0, L2("ijeb"), tv(c.Hvv, "ea", VV), 1.0, H);                              // :486
-  cd(-1.0, L2("mjab"), tv(c.Hoo, "im", OO), 1.0, H);                             // :487
-  cd(0.5, L2("mnab"), tv(c.Hoooo, "ijmn", OOOO), 1.0, H);                        // :488
-  cd(2.0, L2("mjeb"), tv(c.Hovvo, "ieam", OVVO), 1.0, H);                        // :490
-  cd(-1.0, L2("mjeb"), tv(c.Hovov, "iema", OVOV), 1.0, H);
-  cd(-1.0, L2("mibe"), tv(c.Hovov, "jema", OVOV), 1.0, H);                       // :491
-  cd(-1.0, L2("mieb"), tv(c.Hovvo, "jeam", OVVO), 1.0, H);                       // :492
-  cd(1.0, Gvv, LOVV("ijeb"), 1.0, H);                                            // :493
-  cd(-1.0, Goo, LOVV("mjab"), 1.0, H);                                           // :494
+  // ---- from the inputs and HBAR ----
+  const TV Goo = tv(c.Goo, "mi", OO), Gvv = tv(c.Gvv, "ae", VV), Gef = relabel(Gvv, "ef");
+  cd(1.0, T2("mjab"), L2("ijab"), 0.0, Goo);                                     // cclambda.py:281
+  cd(-1.0, T2("ijeb"), L2("ijab"), 0.0, Gvv);                                    // :306
+  if (with_source) {
+    double beta;
+    axpby<double>(1.0, LOVV("ijab"), 0.0, tv(r2s.take(beta), "ijab", OOVV), s, &q);   // :468
+  }
+  R1(1.0, L1("ie"), tv(c.Hvv, "ea", VV));                                        // :354
+  R1(-1.0, L1("ma"), tv(c.Hoo, "im", OO));                                       // :355
+  R1(-1.0, L2("mnae"), tv(c.Hovoo, "iemn", OVOO));                               // :357
+  R1(2.0, L1("me"), tv(c.Hovvo, "ieam", OVVO));                                  // :358
+  R1(-1.0, L1("me"), tv(c.Hovov, "iema", OVOV));
+  H(2.0, L2("mjeb"), tv(c.Hovvo, "ieam", OVVO));                                 // :490
+  H(-1.0, L2("mjeb"), tv(c.Hovov, "iema", OVOV));
+  H(-1.0, L2("mibe"), tv(c.Hovov, "jema", OVOV));                                // :491
+  H(-1.0, L2("mieb"), tv(c.Hovvo, "jeam", OVVO));                                // :492
+  H(1.0, L2("ijeb"), tv(c.Hvv, "ea", VV));                                       // :486
+  H(-1.0, L2("mjab"), tv(c.Hoo, "im", OO));                                      // :487
+  H(0.5, L2("mnab"), tv(c.Hoooo, "ijmn", OOOO));                                 // :488
+  H(2.0, L1("ia"), tv(c.Hov, "jb", OV));                                         // :476
+  H(-1.0, L1("ja"), tv(c.Hov, "ib", OV));                                        // :477
+  H(-2.0, L1("mb"), tv(c.Hooov, "jima", OOOV));                                  // :480
+  H(1.0, L1("mb"), tv(c.Hooov, "ijma", OOOV));                                   // :481
 
   if (c.hbar_stored) {
-    cd(1.0, L2("imef"), tv(c.Hvvvo, "efam", VVVO), 1.0, R1);                     // :356
-    cd(-2.0, relabel(Gvv, "ef"), tv(c.Hvovv, "eifa", VOVV), 1.0, R1);            // :366
-    cd(1.0, relabel(Gvv, "ef"), tv(c.Hvovv, "eiaf", VOVV), 1.0, R1);             // :367
-    cd(2.0, L1("ie"), tv(c.Hvovv, "ejab", VOVV), 1.0, H);                        // :478
-    cd(-1.0, L1("ie"), tv(c.Hvovv, "ejba", VOVV), 1.0, H);                       // :479
-    cd(0.5, L2("ijef"), tv(c.Hvvvv, "efab", {v, v, v, v}), 1.0, H);              // :489
+    R1(1.0, L2("imef"), tv(c.Hvvvo, "efam", VVVO));                              // :356
+    H(2.0, L1("ie"), tv(c.Hvovv, "ejab", VOVV));                                 // :478
+    H(-1.0, L1("ie"), tv(c.Hvovv, "ejba", VOVV));                                // :479
+    H(0.5, L2("ijef"), tv(c.Hvvvv, "efab", {v, v, v, v}));                       // :489
+    R1(-2.0, Gef, tv(c.Hvovv, "eifa", VOVV));                                    // :366
+    R1(1.0, Gef, tv(c.Hvovv, "eiaf", VOVV));                                     // :367
   } else {
     // Factored form of the terms that read Hvvvv, Hvovv and Hvvvo, with the intermediates
     //   Vf_ijem = l2_ijef t_mf,  Vg_ijfm = l2_ijef t_me,  U_ijmn = l2_ijef tau_mnef,
     //   Y_ijab  = l2_ijef Hvvvv_efab
     //           = ladder(l2)_ijab - Vf_ijem <em|ab> - Vg_ijfm <fm|ba> + U_ijmn <mn|ab>   (:395-401)
-    build_tau(o, v, 1.0, 1.0, c.Ht1, c.Ht2, c.tau, s);
+    build_tau(o, v, 1.0, 1.0, c.Ht1, c.Ht2, c.tau, s);   // meets nothing queued
     auto TAU = [&](const char* l) { return tv(c.tau, l, OOVV); };
     const TV Vf = tv(c.LVf, "ijem", OOVO), Vg = tv(c.LVg, "ijfm", OOVO), U = tv(c.LU, "ijmn", OOOO);
     const TV Y = tv(c.LY, "ijab", OOVV);
+    const int64_t npP = c.npP(), npM = c.npM(), noP = c.noP(), noM = c.noM();
+    if (x3) {   // the packed ladder GEMM of the forward residual applied to l2, (ab) columns only: FP16x3 against the
+                // context's split ladder rows, FP32 output
+      ladder_x3_l2(c, l2, s);
+    } else {
+      tau_pack<double>(o, v, nullptr, l2, (double*)c.Tp, (double*)c.Tm, s);
+      cd(1.0, tv(c.Tp, "xk", {noP, npP}), tvs(c.LP, "ky", {npP, npP}, {npP + ov, 1}), 0.0,
+         tvs(c.CP, "xy", {noP, npP}, {npP + ov, 1}));
+      if (noM > 0)
+        cd(1.0, tv(c.Tm, "xk", {noM, npM}), tvs(c.LM, "ky", {npM, npM}, {npM + ov, 1}), 0.0,
+           tvs(c.CM, "xy", {noM, npM}, {npM + ov, 1}));
+    }
     cd(1.0, L2("ijef"), T1("mf"), 0.0, Vf);
     cd(1.0, L2("ijef"), T1("me"), 0.0, Vg);
     cd(1.0, L2("ijef"), TAU("mnef"), 0.0, U);
+    const TV Xoo = tv(c.Lsm, "ip", OO), lt = tv(c.Lsm + o * o + ov, "in", OO);
+    cd(1.0, L2("imef"), T2("pmef"), 0.0, Xoo);
+    cd(1.0, L1("ie"), T1("ne"), 0.0, lt);                      // lt_in = l1_ie t_ne
+    R1(1.0, L2("imef"), CVVV("mfea"));                         // :682 <ef|am> = (mf|ea)
+    // :478-479  l1_ie Hvovv_ejab, Hvovv_ejab = <ej|ab> - t_ne <nj|ab>
+    H(2.0, L1("ie"), CVVV("jbea"));                            // <ej|ab> = (jb|ea)
+    H(-1.0, L1("ie"), CVVV("jaeb"));                           // <ej|ba> = (ja|eb)
+
+    // ---- from those intermediates ----
+    // :356  l2_imef Hvvvo_efam, term by term over :682-695 (p, q occupied and g virtual dummies)
+    const TV W = tv(c.Ltmp, "ifpg", OVOV);                     // :686 -t_mpge <fp|ga>, (pa|fg)
+    cd(1.0, L2("imef"), T2("mpge"), 0.0, W);
+    const bool apart = c.Ltmp2 != c.Ltmp;                      // else each product is used before the next is formed
+    const TV W6 = tv(c.Ltmp2, "iepg", OVOV);                   // :687 -t_mpgf <ep|ag>, (pg|ea)
+    const TV W7 = tv(c.Ltmp3, "iepg", OVOV);                   // :688 t_pmgf L_epag
+    if (apart) {
+      cd(1.0, L2("imef"), T2("mpgf"), 0.0, W6);
+      cd(1.0, L2("imef"), T2("pmgf"), 0.0, W7);
+    }
+    R1(-1.0, W, CVVV("pafg"));
+    if (!apart) cd(1.0, L2("imef"), T2("mpgf"), 0.0, W6);
+    R1(-1.0, W6, CVVV("pgea"));
+    if (!apart) cd(1.0, L2("imef"), T2("pmgf"), 0.0, W7);
+    R1(2.0, W7, CVVV("pgea"));                                 //   L_epag = 2(pg|ea) - (pa|eg)
+    R1(-1.0, W7, CVVV("paeg"));
+    R1(-1.0, Xoo, tv(c.Hov, "pa", OV));                        // :683 -Hov_pa l2_imef t_pmef
+    R1(1.0, relabel(U, "impq"), COOV("qmpa"));                 // :685 <pq|am> = (qm|pa)
+    // :689-691  -t_pf A_epam,  A_epam = <ep|am> - t_mqge <pq|ga>;  Vf_imep = l2_imef t_pf
+    R1(-1.0, relabel(Vf, "imep"), COVV("pmea"));               //   <ep|am> = (pm|ea)
+    const TV Q1 = tv(c.LQ, "ipqg", OOOV), Q2 = tv(c.LQ + o * o * ov, "ipqg", OOOV);
+    const TV Q3 = tv(c.LQ + 2 * o * o * ov, "ipqg", OOOV);
+    cd(1.0, relabel(Vf, "imep"), T2("mqge"), 0.0, Q1);
+    // :692-695  -t_pe B_fpma,  B_fpma = <fp|ma> - t_mqgf <pq|ag> + t_qmgf L_pqag;  Vg_imfp = l2_imef t_pe
+    R1(-1.0, relabel(Vg, "imfp"), COVO("mfpa"));               //   <fp|ma> = (mf|pa)
+    cd(1.0, relabel(Vg, "imfp"), T2("mqgf"), 0.0, Q2);
+    cd(1.0, relabel(Vg, "imfp"), T2("qmgf"), 0.0, Q3);
+    // :366-367  Gvv_ef Hvovv, Hvovv_eifa = <ei|fa> - t_ne <ni|fa>
+    R1(-2.0, Gef, CVVV("iaef"));                               // <ei|fa> = (ia|ef)
+    R1(1.0, Gef, CVVV("ifea"));                                // <ei|af> = (if|ea)
+    const TV gt = tv(c.Lsm + o * o, "nf", OV);                 // gt_nf = Gvv_ef t_ne
+    cd(1.0, Gef, T1("ne"), 0.0, gt);
+    H(-2.0, lt, IOVV("njab"));
+    H(1.0, lt, IOVV("njba"));
+    q.flush();
     {
-      // the packed ladder GEMM of the forward residual applied to l2, (ab) columns only
-      const int64_t npP = c.npP(), npM = c.npM(), noP = c.noP(), noM = c.noM();
       dim3 grid((unsigned)std::min<int64_t>(ceil_div(v * v, 256), 64), (unsigned)(o * o));
-      if (x3) {   // FP16x3 against the context's split ladder rows, FP32 output
-        ladder_x3_l2(c, l2, s);
-        ladder_unpack_kernel<float><<<grid, 256, 0, s>>>(o, v, (const float*)c.CP, (const float*)c.CM, c.LY);
-      } else {
-        tau_pack<double>(o, v, nullptr, l2, (double*)c.Tp, (double*)c.Tm, s);
-        cd(1.0, tv(c.Tp, "xk", {noP, npP}), tvs(c.LP, "ky", {npP, npP}, {npP + ov, 1}), 0.0,
-           tvs(c.CP, "xy", {noP, npP}, {npP + ov, 1}));
-        if (noM > 0)
-          cd(1.0, tv(c.Tm, "xk", {noM, npM}), tvs(c.LM, "ky", {npM, npM}, {npM + ov, 1}), 0.0,
-             tvs(c.CM, "xy", {noM, npM}, {npM + ov, 1}));
-        ladder_unpack_kernel<double><<<grid, 256, 0, s>>>(o, v, (const double*)c.CP, (const double*)c.CM, c.LY);
-      }
+      if (x3) ladder_unpack_kernel<float><<<grid, 256, 0, s>>>(o, v, (const float*)c.CP, (const float*)c.CM, c.LY);
+      else ladder_unpack_kernel<double><<<grid, 256, 0, s>>>(o, v, (const double*)c.CP, (const double*)c.CM, c.LY);
       CCX_HIP(hipGetLastError());
     }
     cd(-1.0, Vf, CVVV("mbea"), 1.0, Y);                        // <em|ab> = (mb|ea)
+    R1(1.0, Q1, IOVV("pqga"));
+    R1(1.0, Q2, IOVV("pqag"));
+    R1(-1.0, Q3, LOVV("pqag"));
+    R1(2.0, gt, IOVV("nifa"));
+    R1(-1.0, gt, IOVV("niaf"));
     cd(-1.0, Vg, CVVV("mafb"), 1.0, Y);                        // <fm|ba> = (ma|fb)
     cd(1.0, U, IOVV("mnab"), 1.0, Y);                          // <mn|ab>
-    axpby<double>(0.5, Y, 1.0, H, s);                                            // :489
-
-    // :356  l2_imef Hvvvo_efam, term by term over :682-695 (p, q occupied and g virtual dummies)
-    cd(1.0, L2("imef"), CVVV("mfea"), 1.0, R1);                // :682 <ef|am> = (mf|ea)
-    const TV Xoo = tv(c.Lsm, "ip", OO);                        // :683 -Hov_pa l2_imef t_pmef
-    cd(1.0, L2("imef"), T2("pmef"), 0.0, Xoo);
-    cd(-1.0, Xoo, tv(c.Hov, "pa", OV), 1.0, R1);
-    cd(1.0, T1("mg"), relabel(Y, "imag"), 1.0, R1);            // :684 t_mg Hvvvv_efag -> t_mg Y_imag
-    cd(1.0, relabel(U, "impq"), COOV("qmpa"), 1.0, R1);        // :685 <pq|am> = (qm|pa)
-    const TV W = tv(c.Ltmp, "ifpg", OVOV);                     // :686 -t_mpge <fp|ga>, (pa|fg)
-    cd(1.0, L2("imef"), T2("mpge"), 0.0, W);
-    cd(-1.0, W, CVVV("pafg"), 1.0, R1);
-    const TV W6 = tv(c.Ltmp, "iepg", OVOV);                    // :687 -t_mpgf <ep|ag>, (pg|ea)
-    cd(1.0, L2("imef"), T2("mpgf"), 0.0, W6);
-    cd(-1.0, W6, CVVV("pgea"), 1.0, R1);
-    cd(1.0, L2("imef"), T2("pmgf"), 0.0, W6);                  // :688 t_pmgf L_epag
-    cd(2.0, W6, CVVV("pgea"), 1.0, R1);                        //   L_epag = 2(pg|ea) - (pa|eg)
-    cd(-1.0, W6, CVVV("paeg"), 1.0, R1);
-    // :689-691  -t_pf A_epam,  A_epam = <ep|am> - t_mqge <pq|ga>;  Vf_imep = l2_imef t_pf
-    cd(-1.0, relabel(Vf, "imep"), COVV("pmea"), 1.0, R1);      //   <ep|am> = (pm|ea)
-    const TV Q = tv(c.LQ, "ipqg", OOOV);
-    cd(1.0, relabel(Vf, "imep"), T2("mqge"), 0.0, Q);
-    cd(1.0, Q, IOVV("pqga"), 1.0, R1);
-    // :692-695  -t_pe B_fpma,  B_fpma = <fp|ma> - t_mqgf <pq|ag> + t_qmgf L_pqag;  Vg_imfp = l2_imef t_pe
-    cd(-1.0, relabel(Vg, "imfp"), COVO("mfpa"), 1.0, R1);      //   <fp|ma> = (mf|pa)
-    cd(1.0, relabel(Vg, "imfp"), T2("mqgf"), 0.0, Q);
-    cd(1.0, Q, IOVV("pqag"), 1.0, R1);
-    cd(1.0, relabel(Vg, "imfp"), T2("qmgf"), 0.0, Q);
-    cd(-1.0, Q, LOVV("pqag"), 1.0, R1);
-
-    // :366-367  Gvv_ef Hvovv, Hvovv_eifa = <ei|fa> - t_ne <ni|fa>
-    const TV Gef = relabel(Gvv, "ef");
-    cd(-2.0, Gef, CVVV("iaef"), 1.0, R1);                      // <ei|fa> = (ia|ef)
-    cd(1.0, Gef, CVVV("ifea"), 1.0, R1);                       // <ei|af> = (if|ea)
-    const TV gt = tv(c.Lsm + o * o, "nf", OV);                 // gt_nf = Gvv_ef t_ne
-    cd(1.0, Gef, T1("ne"), 0.0, gt);
-    cd(2.0, gt, IOVV("nifa"), 1.0, R1);
-    cd(-1.0, gt, IOVV("niaf"), 1.0, R1);
-
-    // :478-479  l1_ie Hvovv_ejab, Hvovv_ejab = <ej|ab> - t_ne <nj|ab>
-    cd(2.0, L1("ie"), CVVV("jbea"), 1.0, H);                   // <ej|ab> = (jb|ea)
-    cd(-1.0, L1("ie"), CVVV("jaeb"), 1.0, H);                  // <ej|ba> = (ja|eb)
-    const TV lt = tv(c.Lsm + o * o + ov, "in", OO);            // lt_in = l1_ie t_ne
-    cd(1.0, L1("ie"), T1("ne"), 0.0, lt);
-    cd(-2.0, lt, IOVV("njab"), 1.0, H);
-    cd(1.0, lt, IOVV("njba"), 1.0, H);
+    R1(1.0, T1("mg"), relabel(Y, "imag"));                     // :684 t_mg Hvvvv_efag -> t_mg Y_imag
+    double beta;
+    double* h = r2s.take(beta);
+    axpby<double>(0.5, Y, beta, tv(h, "ijab", OOVV), s, &q);   // :489
   }
+  R1(-2.0, relabel(Goo, "mn"), tv(c.Hooov, "mina", OOOV));                       // :368
+  R1(1.0, relabel(Goo, "mn"), tv(c.Hooov, "imna", OOOV));                        // :369
+  H(1.0, Gvv, LOVV("ijeb"));                                                     // :493
+  H(-1.0, Goo, LOVV("mjab"));                                                    // :494
+  q.flush();
 
-  pair_symmetrize(o, v, alpha, c.Lh, r2, s);                                     // :496
+  SumJobs j;
+  j.add(ov, v, v, 1, with_source ? c.Hov : nullptr, r1s, r1, nullptr, 2.0);      // :348
+  sum_jobs(j, s);
+  pair_symmetrize(o, v, alpha, r2s.used, c.Lh, r2, s);                           // :496
 }
 
 // The CCSD Jacobian applied to (x1, x2) on the current HBAR (CCderiv._ccsd_jacobian,
@@ -507,8 +541,20 @@ void jacobian(Ctx& c, const double* x1, const double* x2, double* j1, double* j2
   const std::vector<int64_t> OV{o, v}, OO{o, o}, VV{v, v}, OOVV{o, o, v, v}, OVOV{o, v, o, v};
   const std::vector<int64_t> OOOV{o, o, o, v}, OOOO{o, o, o, o}, OVVV{o, v, v, v};
   const std::vector<int64_t> VOVV{v, o, v, v}, OVVO{o, v, v, o}, VVVO{v, v, v, o}, OVOO{o, v, o, o};
+  GemmQueue q(ws, s);   // as in lambda_residual: partial sums, small terms gathered into few launches
   auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C) {
-    contract<double>(a, A, B, b, C, ws, s);
+    contract<double>(a, A, B, b, C, ws, s, false, &q);
+  };
+  PartSum r1s(c.Lr, ov, SINGLES_PARTS), r2s(c.Lh, ov * ov, doubles_parts(ov * ov));
+  auto R1 = [&](double a, const TV& A, const TV& B) {   // sigma1 += a A B
+    double beta;
+    double* p = r1s.take(beta);
+    cd(a, A, B, beta, tv(p, "ia", OV));
+  };
+  auto H = [&](double a, const TV& A, const TV& B) {    // sigma2 before P(ij,ab) += a A B
+    double beta;
+    double* p = r2s.take(beta);
+    cd(a, A, B, beta, tv(p, "ijab", OOVV));
   };
   auto X1 = [&](const char* l) { return tv(x1, l, OV); };
   auto X2 = [&](const char* l) { return tv(x2, l, OOVV); };
@@ -526,15 +572,14 @@ void jacobian(Ctx& c, const double* x1, const double* x2, double* j1, double* j2
   const TV Zvv = tv(sm, "ae", VV), Zoo = tv(sm + v * v, "mi", OO);
 
   // ---- sigma1: ccderiv.py:165-169 ----
-  const TV R1 = tv(j1, "ia", OV);
-  cd(1.0, X1("ie"), tv(c.Hvv, "ae", VV), 0.0, R1);                                    // :165
-  cd(-1.0, X1("ma"), tv(c.Hoo, "mi", OO), 1.0, R1);
-  cd(2.0, X1("me"), tv(c.Hovvo, "maei", OVVO), 1.0, R1);                              // :166
-  cd(-1.0, X1("me"), tv(c.Hovov, "maie", OVOV), 1.0, R1);
-  cd(2.0, Hov, X2("miea"), 1.0, R1);                                                  // :167
-  cd(-1.0, Hov, X2("imea"), 1.0, R1);
-  cd(-2.0, X2("mnae"), HOOV("mnie"), 1.0, R1);                                        // :169
-  cd(1.0, X2("mnae"), HOOV("nmie"), 1.0, R1);
+  R1(1.0, X1("ie"), tv(c.Hvv, "ae", VV));                                    // :165
+  R1(-1.0, X1("ma"), tv(c.Hoo, "mi", OO));
+  R1(2.0, X1("me"), tv(c.Hovvo, "maei", OVVO));                              // :166
+  R1(-1.0, X1("me"), tv(c.Hovov, "maie", OVOV));
+  R1(2.0, Hov, X2("miea"));                                                  // :167
+  R1(-1.0, Hov, X2("imea"));
+  R1(-2.0, X2("mnae"), HOOV("mnie"));                                        // :169
+  R1(1.0, X2("mnae"), HOOV("nmie"));
   // Zvv, Zoo: :170-171 (the Hvvmvo parts below, by HBAR form)
   cd(-1.0, LOVV("mnef"), X2("mnaf"), 0.0, Zvv);
   cd(-2.0, HOOV("mnie"), X1("ne"), 0.0, Zoo);
@@ -542,73 +587,77 @@ void jacobian(Ctx& c, const double* x1, const double* x2, double* j1, double* j2
   cd(-1.0, LOVV("mnef"), X2("inef"), 1.0, Zoo);
 
   // ---- sigma2 before the final P(ij,ab): ccderiv.py:172-177 ----
-  const TV H = tv(c.Lh, "ijab", OOVV);
-  cd(-1.0, X1("ma"), tv(c.Hovoo, "mbij", OVOO), 0.0, H);                              // :172
-  cd(1.0, X2("ijeb"), tv(c.Hvv, "ae", VV), 1.0, H);                                   // :174
-  cd(-1.0, X2("mjab"), tv(c.Hoo, "mi", OO), 1.0, H);
-  cd(0.5, X2("mnab"), tv(c.Hoooo, "mnij", OOOO), 1.0, H);                             // :175
-  cd(-1.0, X2("imeb"), tv(c.Hovov, "maje", OVOV), 1.0, H);                            // :176
-  cd(-1.0, X2("imea"), tv(c.Hovvo, "mbej", OVVO), 1.0, H);
-  cd(2.0, X2("miea"), tv(c.Hovvo, "mbej", OVVO), 1.0, H);                             // :177
-  cd(-1.0, X2("miea"), tv(c.Hovov, "mbje", OVOV), 1.0, H);
+  H(-1.0, X1("ma"), tv(c.Hovoo, "mbij", OVOO));                              // :172
+  H(1.0, X2("ijeb"), tv(c.Hvv, "ae", VV));                                   // :174
+  H(-1.0, X2("mjab"), tv(c.Hoo, "mi", OO));
+  H(0.5, X2("mnab"), tv(c.Hoooo, "mnij", OOOO));                             // :175
+  H(-1.0, X2("imeb"), tv(c.Hovov, "maje", OVOV));                            // :176
+  H(-1.0, X2("imea"), tv(c.Hovvo, "mbej", OVVO));
+  H(2.0, X2("miea"), tv(c.Hovvo, "mbej", OVVO));                             // :177
+  H(-1.0, X2("miea"), tv(c.Hovov, "mbje", OVOV));
 
   if (c.hbar_stored) {
     // Hvvmvo = 2 Hvovv - Hvovv^(ef) (:163)
-    cd(2.0, X2("imef"), tv(c.Hvovv, "amef", VOVV), 1.0, R1);                          // :168
-    cd(-1.0, X2("imef"), tv(c.Hvovv, "amfe", VOVV), 1.0, R1);
+    R1(2.0, X2("imef"), tv(c.Hvovv, "amef", VOVV));                          // :168
+    R1(-1.0, X2("imef"), tv(c.Hvovv, "amfe", VOVV));
     cd(2.0, tv(c.Hvovv, "amef", VOVV), X1("mf"), 1.0, Zvv);                           // :170
     cd(-1.0, tv(c.Hvovv, "amfe", VOVV), X1("mf"), 1.0, Zvv);
-    cd(1.0, X1("ie"), tv(c.Hvvvo, "abej", VVVO), 1.0, H);                             // :172
-    cd(0.5, X2("ijef"), tv(c.Hvvvv, "abef", {v, v, v, v}), 1.0, H);                   // :175
+    H(1.0, X1("ie"), tv(c.Hvvvo, "abej", VVVO));                             // :172
+    H(0.5, X2("ijef"), tv(c.Hvvvv, "abef", {v, v, v, v}));                   // :175
   } else {
     // Hvvmvo_amef = L_amef - t_na L_nmef with L_amef = 2 (mf|ae) - (me|af)
-    const TV Win = tv(sm + v * v + o * o, "in", OO), q = tv(sm + v * v + 2 * o * o, "ne", OV);
-    cd(2.0, X2("imef"), CVVV("mfae"), 1.0, R1);                                       // :168
-    cd(-1.0, X2("imef"), CVVV("meaf"), 1.0, R1);
+    const TV Win = tv(sm + v * v + o * o, "in", OO), xL = tv(sm + v * v + 4 * o * o, "ne", OV);
+    R1(2.0, X2("imef"), CVVV("mfae"));                                                // :168
+    R1(-1.0, X2("imef"), CVVV("meaf"));
     cd(1.0, X2("imef"), LOVV("nmef"), 0.0, Win);
-    cd(-1.0, T1("na"), Win, 1.0, R1);
-    cd(2.0, CVVV("mfae"), X1("mf"), 1.0, Zvv);                                        // :170
-    cd(-1.0, CVVV("meaf"), X1("mf"), 1.0, Zvv);
-    cd(1.0, X1("mf"), LOVV("nmef"), 0.0, q);
-    cd(-1.0, T1("na"), q, 1.0, Zvv);
-    // x_ie Hvvvo_abej over cchbar.py:682-695 (its Hvvvv part joins the x2 ladder below)
-    build_tau(o, v, 1.0, 1.0, c.Ht1, c.Ht2, c.tau, s);
+    cd(1.0, X1("mf"), LOVV("nmef"), 0.0, xL);
+    // x_ie Hvvvo_abej over cchbar.py:682-695 (its Hvvvv part joins the x2 ladder below): the products of x1 with the
+    // integrals first
+    build_tau(o, v, 1.0, 1.0, c.Ht1, c.Ht2, c.tau, s);   // meets nothing queued
     auto TAU = [&](const char* l) { return tv(c.tau, l, OOVV); };
-    cd(1.0, X1("ie"), CVVV("jbae"), 1.0, H);                                          // <ab|ej> = (jb|ae)
+    const bool apart = c.Ltmp2 != c.Ltmp;                // else G is used before G2 is formed
+    auto q3 = [&](int k, const char* l) { return tv(c.LQ + k * o * o * ov, l, OOOV); };
     const TV u = tv(sm + v * v + 3 * o * o, "im", OO);                                // -Hov_me t_mjab
-    cd(1.0, X1("ie"), Hov, 0.0, u);
-    cd(-1.0, u, T2("mjab"), 1.0, H);
     const TV V = tv(c.LU, "mnij", OOOO);                                              // tau_mnab <mn|ej>
+    const TV G = tv(c.Ltmp, "imbf", OOVV), G2 = tv(c.Ltmp2, "imfa", OOVV), G4 = tv(c.LY, "imfa", OOVV);
+    const TV K1 = tv(c.LVf, "imja", OOOV), K4 = tv(c.LVg, "imjb", OOOV);
+    const TV K2 = q3(0, "imnf"), K5 = q3(1, "imnf"), K7 = q3(2, "imnf");
+    const TV K3 = q3(3, "ijma"), K6 = q3(4, "ijmb"), K8 = q3(5, "ijmb");
+    cd(1.0, X1("ie"), Hov, 0.0, u);
     cd(1.0, X1("ie"), COOV("njme"), 0.0, V);
-    cd(1.0, TAU("mnab"), V, 1.0, H);
-    const TV G = tv(c.Ltmp, "imbf", OOVV);                                            // -t_jmfa <bm|fe>
-    cd(1.0, X1("ie"), CVVV("mebf"), 0.0, G);
-    cd(-1.0, T2("jmfa"), G, 1.0, H);
-    const TV G2 = tv(c.Ltmp, "imfa", OOVV), G4 = tv(c.LY, "imfa", OOVV);
-    cd(1.0, X1("ie"), CVVV("mfae"), 0.0, G2);                                         // x_ie <am|ef>
-    cd(-1.0, T2("jmfb"), G2, 1.0, H);                                                 // -t_jmfb <am|ef>
-    cd(2.0, T2("mjfb"), G2, 1.0, H);                                                  // +t_mjfb L_amef
+    cd(1.0, X1("ie"), CVVV("mebf"), 0.0, G);                                          // x_ie <bm|fe>
+    if (apart) cd(1.0, X1("ie"), CVVV("mfae"), 0.0, G2);                              // x_ie <am|ef>
     cd(1.0, X1("ie"), CVVV("meaf"), 0.0, G4);
-    cd(-1.0, T2("mjfb"), G4, 1.0, H);
-    const TV K1 = tv(c.LVf, "imja", OOOV), K2 = tv(c.LVg, "imnf", OOOV), K3 = tv(c.LQ, "ijma", OOOV);
-    cd(1.0, X1("ie"), COVV("mjae"), 0.0, K1);                                         // -t_mb A_amej
-    cd(-1.0, T1("mb"), K1, 1.0, H);
+    cd(1.0, X1("ie"), COVV("mjae"), 0.0, K1);
     cd(1.0, X1("ie"), IOVV("mnfe"), 0.0, K2);
-    cd(1.0, T2("jnfa"), K2, 0.0, K3);
-    cd(1.0, T1("mb"), K3, 1.0, H);
-    const TV K4 = tv(c.LVf, "imjb", OOOV), K5 = tv(c.LVg, "imnf", OOOV), K6 = tv(c.LQ, "ijmb", OOOV);
-    cd(1.0, X1("ie"), COVO("mejb"), 0.0, K4);                                         // -t_ma B_bmje
-    cd(-1.0, T1("ma"), K4, 1.0, H);
+    cd(1.0, X1("ie"), COVO("mejb"), 0.0, K4);
     cd(1.0, X1("ie"), IOVV("mnef"), 0.0, K5);
-    cd(1.0, T2("jnfb"), K5, 0.0, K6);
-    cd(1.0, T1("ma"), K6, 1.0, H);
-    const TV K7 = tv(c.LVg, "imnf", OOOV), K8 = tv(c.LQ, "ijmb", OOOV);
     cd(1.0, X1("ie"), LOVV("mnef"), 0.0, K7);
+    H(1.0, X1("ie"), CVVV("jbae"));                                                   // <ab|ej> = (jb|ae)
+    cd(2.0, CVVV("mfae"), X1("mf"), 1.0, Zvv);                                        // :170
+    // then what uses them
+    cd(1.0, T2("jnfa"), K2, 0.0, K3);
+    cd(1.0, T2("jnfb"), K5, 0.0, K6);
     cd(1.0, T2("njfb"), K7, 0.0, K8);
-    cd(-1.0, T1("ma"), K8, 1.0, H);
+    R1(-1.0, T1("na"), Win);
+    H(-1.0, u, T2("mjab"));
+    H(1.0, TAU("mnab"), V);
+    H(-1.0, T2("jmfa"), G);                                                           // -t_jmfa <bm|fe>
+    if (!apart) cd(1.0, X1("ie"), CVVV("mfae"), 0.0, G2);
+    H(-1.0, T2("jmfb"), G2);                                                          // -t_jmfb <am|ef>
+    cd(-1.0, CVVV("meaf"), X1("mf"), 1.0, Zvv);
+    H(2.0, T2("mjfb"), G2);                                                           // +t_mjfb L_amef
+    H(-1.0, T2("mjfb"), G4);
+    H(-1.0, T1("mb"), K1);                                                            // -t_mb A_amej
+    H(-1.0, T1("ma"), K4);                                                            // -t_ma B_bmje
+    cd(-1.0, T1("na"), xL, 1.0, Zvv);
+    H(1.0, T1("mb"), K3);
+    H(1.0, T1("ma"), K6);
+    H(-1.0, T1("ma"), K8);
     // 1/2 x2 Hvvvv (:175) and x_ie t_jf Hvvvv_abef (:684 in :172) are, after P(ij,ab), the one
     // pair-symmetric contraction 1/2 Y(Z) with Z = x2 + x1 t1 + t1 x1 and Y(Z)_ijab = Z_ijef Hvvvv_abef
     //   = ladder(Z) - t_mb Z_ijef <am|ef> - t_ma Z_ijef <bm|fe> + tau_mnab Z_ijef <mn|ef>
+    q.flush();
     CCX_HIP(hipMemcpyAsync(c.LY, x2, ov * ov * sizeof(double), hipMemcpyDeviceToDevice, s));
     pair_outer_kernel<<<(unsigned)std::min<int64_t>(ceil_div(ov * ov, 256), 65536), 256, 0, s>>>(o, v, x1, c.Ht1,
                                                                                                  c.LY);
@@ -620,22 +669,29 @@ void jacobian(Ctx& c, const double* x1, const double* x2, double* j1, double* j2
     cd(1.0, tv(c.Tp, "xk", {noP, npP}), tv(c.LP, "ky", {npP, npP + ov}), 0.0, tv(c.CP, "xy", {noP, npP + ov}));
     if (noM > 0)
       cd(1.0, tv(c.Tm, "xk", {noM, npM}), tv(c.LM, "ky", {npM, npM + ov}), 0.0, tv(c.CM, "xy", {noM, npM + ov}));
+    q.flush();
     dim3 grid((unsigned)std::min<int64_t>(ceil_div(v * v, 256), 64), (unsigned)(o * o));
     ladder_unpack_kernel<double><<<grid, 256, 0, s>>>(o, v, (const double*)c.CP, (const double*)c.CM, c.LY);
     CCX_HIP(hipGetLastError());
     // Zf[m][i][j][b] = Z_ijef <mb|ef> from the (m, b) columns of the same GEMM
     const TV Zf = tv(c.LQ, "mijb", OOOV);
     scale<double>(0.0, Zf, s);
-    zt_add<double>(o, v, (const double*)c.CP, (const double*)c.CM, c.LQ, s);
+    zt_add<double>(o, v, (const double*)c.CP, (const double*)c.CM, nullptr, c.LQ, s);
     const TV Y = tv(c.LY, "ijab", OOVV);
     cd(-1.0, T1("mb"), tv(c.LQ, "mjia", OOOV), 1.0, Y);                               // Z_ijef <am|ef> = Zf[m][j][i][a]
     cd(-1.0, T1("ma"), Zf, 1.0, Y);                                                   // Z_ijef <bm|fe> = Zf[m][i][j][b]
     cd(1.0, TAU("mnab"), Ze, 1.0, Y);
-    axpby<double>(0.5, Y, 1.0, H, s);
+    double beta;
+    double* h = r2s.take(beta);
+    axpby<double>(0.5, Y, beta, tv(h, "ijab", OOVV), s, &q);
   }
-  cd(1.0, Zoo, T2("mjab"), 1.0, H);                                                   // :173
-  cd(1.0, Zvv, T2("ijeb"), 1.0, H);
-  pair_symmetrize(o, v, 1.0, c.Lh, j2, s);
+  H(1.0, Zoo, T2("mjab"));                                                   // :173
+  H(1.0, Zvv, T2("ijeb"));
+  q.flush();
+  SumJobs j;
+  j.add(ov, v, v, 1, nullptr, r1s, j1, nullptr);
+  sum_jobs(j, s);
+  pair_symmetrize(o, v, 1.0, r2s.used, c.Lh, j2, s);
 }
 
 // One- and two-particle densities of the CC Lagrangian E + l1.r1 + 1/2 l2.r2 at (t, l)
@@ -654,9 +710,11 @@ void densities(Ctx& c, const double* t1, const double* t2, const double* l1, con
   Workspace& ws = c.ws;
   const std::vector<int64_t> OV{o, v}, OO{o, o}, VV{v, v}, OOVV{o, o, v, v}, OVOV{o, v, o, v};
   const std::vector<int64_t> OOOV{o, o, o, v}, OOOO{o, o, o, o}, VVVO{v, v, v, o}, VOVO{v, o, v, o};
+  GemmQueue gq(ws, s);
   auto cd = [&](double a, const TV& A, const TV& B, double b, const TV& C) {
-    contract<double>(a, A, B, b, C, ws, s);
+    contract<double>(a, A, B, b, C, ws, s, false, &gq);
   };
+  auto axpby = [&](double a, const TV& A, double b, const TV& C, hipStream_t) { ccx::axpby<double>(a, A, b, C, s, &gq); };
   auto T1 = [&](const char* l) { return tv(t1, l, OV); };
   auto T2 = [&](const char* l) { return tv(t2, l, OOVV); };
   auto L1 = [&](const char* l) { return tv(l1, l, OV); };
@@ -674,8 +732,8 @@ void densities(Ctx& c, const double* t1, const double* t2, const double* l1, con
   cd(-1.0, T2("imef"), L2("jmef"), 1.0, Doo);
   cd(1.0, T1("mb"), L1("ma"), 0.0, Dvv);
   cd(1.0, T2("mnbe"), L2("mnae"), 1.0, Dvv);
-  axpby<double>(1.0, L1("ia"), 0.0, Dvo, s);
-  axpby<double>(2.0, T1("ia"), 0.0, Dov, s);
+  axpby(1.0, L1("ia"), 0.0, Dvo, s);
+  axpby(2.0, T1("ia"), 0.0, Dov, s);
   cd(2.0, L1("me"), T2("imae"), 1.0, Dov);
   cd(-1.0, L1("me"), TAU("miae"), 1.0, Dov);
   const TV soo = tv(c.Lsm, "mi", OO), svv = tv(c.LY, "ea", VV);
@@ -750,9 +808,9 @@ void densities(Ctx& c, const double* t1, const double* t2, const double* l1, con
   {
     const TV Dq = tv(Doovv, "ijab", OOVV);
     cd(4.0, T1("ia"), L1("jb"), 0.0, Dq);                                            // :860
-    axpby<double>(4.0, TAU("ijab"), 1.0, Dq, s);                                     // :861  2 (2 tau - tau^T)
-    axpby<double>(-2.0, TAU("ijba"), 1.0, Dq, s);
-    axpby<double>(1.0, L2("ijab"), 1.0, Dq, s);                                      // :862
+    axpby(4.0, TAU("ijab"), 1.0, Dq, s);                                     // :861  2 (2 tau - tau^T)
+    axpby(-2.0, TAU("ijba"), 1.0, Dq, s);
+    axpby(1.0, L2("ijab"), 1.0, Dq, s);                                      // :862
     const TV x2 = tv(c.Lsm, "jb", OV), x3 = tv(c.LVf, "ijmb", OOOV);
     cd(4.0, L1("me"), T2("jmbe"), 0.0, x2);                                          // :864-865  2 l_me (2 t - t^T)
     cd(-2.0, L1("me"), T2("jmeb"), 1.0, x2);
@@ -816,6 +874,7 @@ void densities(Ctx& c, const double* t1, const double* t2, const double* l1, con
     cd(1.0, T1("nb"), z2, 0.0, z3);                                                  // :921
     cd(1.0, T1("ma"), z3, 1.0, Dq);                                                  // :922
   }
+  gq.flush();
 }
 
 // compute_energy (ccdensity.py:113-211): F_ij D_ij + F_ab D_ab + 1/2 <ij|kl> Doooo + <ij|ka> Dooov

@@ -17,9 +17,9 @@ __host__ __device__ inline int64_t pairM(int64_t a, int64_t b) { return b * (b -
 void gather_chem(const double* eri, int64_t nmo, int64_t p0, int64_t np, int64_t q0, int64_t nq,
                  int64_t r0, int64_t nr, int64_t s0, int64_t ns, double* out, hipStream_t s);
 
-// tau = f1 * t2 + f2 * t1 (x) t1, layout [i][j][a][b]
+// tau = f1 * t2 + f2 * t1 (x) t1, layout [i][j][a][b]; tau_b (may be null) the same with f2_b
 void build_tau(int64_t o, int64_t v, double f1, double f2, const double* t1, const double* t2,
-               double* tau, hipStream_t s);
+               double* tau, hipStream_t s, double* tau_b = nullptr, double f2_b = 0.0);
 
 // Ring-layout operands ([i][a][j][b], i.e. ov x ov matrices), see ring_prep_kernel.
 template <typename T>
@@ -58,17 +58,48 @@ void ladder_pack_bf16x3(int64_t o, int64_t v, int64_t e0, int64_t e1, VVVVSrc sr
 void ladder_pack_o_bf16x3(int64_t o, int64_t v, const double* Covvv, bf16* LP_hi, bf16* LP_lo,
                           bf16* LM_hi, bf16* LM_lo, hipStream_t s);
 
-// Zt[m][i][j][b] += Z_mbij from the packed ladder outputs.
+// Zt[m][i][j][b] += Z_mbij from the packed ladder outputs, and two more arrays of Zt's size one after the other (more; may
+// be null).
 template <typename T>
-void zt_add(int64_t o, int64_t v, const T* CP, const T* CM, double* Zt, hipStream_t s);
+void zt_add(int64_t o, int64_t v, const T* CP, const T* CM, const double* more, double* Zt, hipStream_t s);
+
+// Several sums of partial sums in one launch: out[e] = w src[(e / cols) sr + (e % cols) sc] + sum_p parts[p n + e] (src may
+// be null), out2 (may be null) a copy.
+struct SumJobs {
+  static constexpr int MAX = 4;
+  struct Job {
+    int64_t n, cols, sr, sc;
+    const double* src;
+    const double* parts;
+    int np;
+    double w;
+    double *out, *out2;
+  };
+  int n = 0;
+  int first[MAX + 1] = {0};
+  Job j[MAX];
+  template <typename PS>
+  void add(int64_t size, int64_t cols, int64_t sr, int64_t sc, const double* src, const PS& ps, double* out, double* out2,
+           double w = 1.0) {
+    CCX_CHECK(n < MAX && ceil_div(size, 256) < (1 << 24), ERR_INTERNAL, "too many sums");
+    j[n] = Job{size, cols, sr, sc, src, ps.base, ps.used, w, out, out2};
+    first[n + 1] = first[n] + (int)ceil_div(size, 256);
+    ++n;
+  }
+};
+void sum_jobs(const SumJobs& j, hipStream_t s);
+
+// W[(me)][x][(jb)] += three arrays of W's size one after the other, and the (ov)^2 one behind them to x = 0
+void w_sum(int64_t ov, const double* parts, double* W, hipStream_t s);
 
 // r2[i][j][a][b] = H[ijab] + H[jiba] + ladder[ijab] + P[ia,jb] + P[jb,ia] + Q[ja,ib] + Q[ib,ja]
 //                  - sum_m (t1[m][a] Zt[m][i][j][b] + t1[m][b] Zt[m][j][i][a])
 //                  [+ PTt[i][j][b][a] + PTt[j][i][a][b]] [+ X[ijab] + X[jiba]]   (FP32, each optional)
 //                  [+ I[ijab]] [+ T2d[ijab] Gd[b] + T2d[jiba] Gd[a]]               (FP64, each optional)
-// computed once per pair-symmetric couple and written to both (ij)(ab) partners
+// computed once per pair-symmetric couple and written to both (ij)(ab) partners; H is the sum of h_parts arrays, one after
+// the other
 template <typename T>
-void assemble_r2(int64_t o, int64_t v, const double* H, const T* CP, const T* CM, const T* P,
+void assemble_r2(int64_t o, int64_t v, int h_parts, const double* H, const T* CP, const T* CM, const T* P,
                  const T* Q, const double* t1, const double* Zt, const float* PTt, const float* X,
                  const double* I, const double* T2d, const double* Gd, double* r2, hipStream_t s);
 

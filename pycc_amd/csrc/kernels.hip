@@ -86,7 +86,7 @@ constexpr int TAU_STEPS = 4;
 template <int VEC>
 __global__ __launch_bounds__(256) void tau_kernel(int o, int v, int nchunk, double f1, double f2,
                                                   const double* __restrict__ t1, const double* __restrict__ t2,
-                                                  double* __restrict__ tau) {
+                                                  double* __restrict__ tau, double f2b, double* __restrict__ taub) {
   const int ij = (int)(blockIdx.x / (unsigned)nchunk), chunk = (int)blockIdx.x - ij * nchunk;
   const int i = ij / o, j = ij - i * o;
   const uint32_t plane = (uint32_t)v * (uint32_t)v;
@@ -107,10 +107,16 @@ __global__ __launch_bounds__(256) void tau_kernel(int o, int v, int nchunk, doub
       if (e < plane) {
         const uint32_t a0 = e / (uint32_t)v, b0 = e - a0 * v;
         const uint32_t a1 = (e + 1) / (uint32_t)v, b1 = e + 1 - a1 * v;
+        const double px = ti[a0] * tj[b0], py = ti[a1] * tj[b1];
         double2 y;
-        y.x = f1 * x[k].x + f2 * (ti[a0] * tj[b0]);
-        y.y = f1 * x[k].y + f2 * (ti[a1] * tj[b1]);
+        y.x = f1 * x[k].x + f2 * px;
+        y.y = f1 * x[k].y + f2 * py;
         *(double2*)(tau + base + e) = y;
+        if (taub) {
+          y.x = f1 * x[k].x + f2b * px;
+          y.y = f1 * x[k].y + f2b * py;
+          *(double2*)(taub + base + e) = y;
+        }
       }
     }
   } else {
@@ -119,22 +125,24 @@ __global__ __launch_bounds__(256) void tau_kernel(int o, int v, int nchunk, doub
       const uint32_t e = e0 + k * 256u;
       if (e < plane) {
         const uint32_t a = e / (uint32_t)v, b = e - a * v;
-        tau[base + e] = f1 * t2[base + e] + f2 * (ti[a] * tj[b]);
+        const double x = t2[base + e], p = ti[a] * tj[b];
+        tau[base + e] = f1 * x + f2 * p;
+        if (taub) taub[base + e] = f1 * x + f2b * p;
       }
     }
   }
 }
 
 void build_tau(int64_t o, int64_t v, double f1, double f2, const double* t1, const double* t2,
-               double* tau, hipStream_t s) {
+               double* tau, hipStream_t s, double* tau_b, double f2_b) {
   if (o == 0 || v == 0) return;
   CCX_CHECK(v * v < (1ll << 31), ERR_ARG, "build_tau: v x v plane too large");
   const int vec = (v % 2 == 0) ? 2 : 1;
   const int64_t nchunk = ceil_div(v * v, 256 * vec * TAU_STEPS);
   CCX_CHECK(o * o * nchunk < (1ll << 31), ERR_ARG, "build_tau: grid too large");
   const unsigned grid = (unsigned)(o * o * nchunk);
-  if (vec == 2) tau_kernel<2><<<grid, 256, 0, s>>>((int)o, (int)v, (int)nchunk, f1, f2, t1, t2, tau);
-  else tau_kernel<1><<<grid, 256, 0, s>>>((int)o, (int)v, (int)nchunk, f1, f2, t1, t2, tau);
+  if (vec == 2) tau_kernel<2><<<grid, 256, 0, s>>>((int)o, (int)v, (int)nchunk, f1, f2, t1, t2, tau, f2_b, tau_b);
+  else tau_kernel<1><<<grid, 256, 0, s>>>((int)o, (int)v, (int)nchunk, f1, f2, t1, t2, tau, f2_b, tau_b);
   CCX_HIP(hipGetLastError());
 }
 
@@ -382,7 +390,7 @@ void ladder_pack(int64_t o, int64_t v, int64_t e0, int64_t e1, VVVVSrc src, cons
 // ---------------------------------------------------------------------------------------------
 template <typename T>
 __global__ void zt_add_kernel(int64_t o, int64_t v, const T* __restrict__ CP, const T* __restrict__ CM,
-                              double* __restrict__ Zt) {
+                              const double* __restrict__ more, double* __restrict__ Zt) {
   const int64_t npP = v * (v + 1) / 2, npM = v * (v - 1) / 2;
   const int64_t ldP = npP + o * v, ldM = npM + o * v;
   const int64_t total = o * o * o * v;
@@ -399,13 +407,52 @@ __global__ void zt_add_kernel(int64_t o, int64_t v, const T* __restrict__ CP, co
       double zm = (double)CM[pairM(lo, hi) * ldM + npM + mb];
       z += (i < j) ? zm : -zm;
     }
+    if (more) z += more[e] + more[total + e];
     Zt[e] += z;
   }
 }
 
 template <typename T>
-void zt_add(int64_t o, int64_t v, const T* CP, const T* CM, double* Zt, hipStream_t s) {
-  zt_add_kernel<T><<<grid_for(o * v * o * o), 256, 0, s>>>(o, v, CP, CM, Zt);
+void zt_add(int64_t o, int64_t v, const T* CP, const T* CM, const double* more, double* Zt, hipStream_t s) {
+  zt_add_kernel<T><<<grid_for(o * v * o * o), 256, 0, s>>>(o, v, CP, CM, more, Zt);
+  CCX_HIP(hipGetLastError());
+}
+
+// ---------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void sum_jobs_kernel(const SumJobs a) {
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+  const SumJobs::Job& d = a.j[i];
+  const int64_t e = (int64_t)(blockIdx.x - a.first[i]) * 256 + threadIdx.x;
+  if (e >= d.n) return;
+  double t = 0.0;
+  if (d.src) {
+    const int64_t r = e / d.cols;
+    t = d.w * d.src[r * d.sr + (e - r * d.cols) * d.sc];
+  }
+  for (int p = 0; p < d.np; ++p) t += d.parts[p * d.n + e];
+  d.out[e] = t;
+  if (d.out2) d.out2[e] = t;
+}
+
+void sum_jobs(const SumJobs& j, hipStream_t s) {
+  if (!j.n) return;
+  sum_jobs_kernel<<<(unsigned)j.first[j.n], 256, 0, s>>>(j);
+  CCX_HIP(hipGetLastError());
+}
+
+__global__ __launch_bounds__(256) void w_sum_kernel(int ov, const double* __restrict__ p, double* __restrict__ W) {
+  const int r = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;   // c: (x, jb)
+  if (c >= 2 * ov) return;
+  const int64_t n = 2 * (int64_t)ov * ov, e = (int64_t)r * 2 * ov + c;
+  double t = W[e] + p[e] + p[n + e] + p[2 * n + e];
+  if (c < ov) t += p[3 * n + (int64_t)r * ov + c];
+  W[e] = t;
+}
+
+void w_sum(int64_t ov, const double* parts, double* W, hipStream_t s) {
+  CCX_CHECK(ov < 65536, ERR_ARG, "w_sum: grid too large");
+  w_sum_kernel<<<dim3((unsigned)ceil_div(2 * ov, 256), (unsigned)ov), 256, 0, s>>>((int)ov, parts, W);
   CCX_HIP(hipGetLastError());
 }
 
@@ -430,7 +477,7 @@ void zt_add(int64_t o, int64_t v, const T* CP, const T* CM, double* Zt, hipStrea
 // holds C[4 r + l / 16][l % 16]); each lane then finishes the four elements of its C registers.
 typedef double asm_d4 __attribute__((ext_vector_type(4)));
 template <typename T>
-__global__ __launch_bounds__(256) void assemble_r2_kernel(int64_t o, int64_t v, const double* __restrict__ H,
+__global__ __launch_bounds__(256) void assemble_r2_kernel(int64_t o, int64_t v, int hp, const double* __restrict__ H,
                                                           const T* __restrict__ CP, const T* __restrict__ CM,
                                                           const T* __restrict__ P, const T* __restrict__ Q,
                                                           const double* __restrict__ t1,
@@ -457,6 +504,7 @@ __global__ __launch_bounds__(256) void assemble_r2_kernel(int64_t o, int64_t v, 
       if (a < v && b < v) {
         p = H[((j * o + i) * v + b) * v + a] + (double)P[(j * v + b) * ov + i * v + a] +
             (double)Q[(i * v + b) * ov + j * v + a];
+        for (int h = 1; h < hp; ++h) p += H[h * ov * ov + ((j * o + i) * v + b) * v + a];
         if (PTt) p += (double)PTt[((i * o + j) * v + b) * v + a];
         if (X) p += (double)X[((j * o + i) * v + b) * v + a];
         if (T2d) p += T2d[((j * o + i) * v + b) * v + a] * Gd[a];
@@ -503,6 +551,7 @@ __global__ __launch_bounds__(256) void assemble_r2_kernel(int64_t o, int64_t v, 
     if (a < v && bok) {
       const int64_t ijab = ((i * o + j) * v + a) * v + b;
       e = H[ijab] + part[bl][al];
+      for (int h = 1; h < hp; ++h) e += H[h * ov * ov + ijab];
       const int64_t alo = a < b ? a : b, ahi = a < b ? b : a;
       e += (double)cpr[pairP(alo, ahi)];
       if (cmr && a != b) {
@@ -540,14 +589,14 @@ __global__ __launch_bounds__(256) void assemble_r2_kernel(int64_t o, int64_t v, 
 }
 
 template <typename T>
-void assemble_r2(int64_t o, int64_t v, const double* H, const T* CP, const T* CM, const T* P,
+void assemble_r2(int64_t o, int64_t v, int h_parts, const double* H, const T* CP, const T* CM, const T* P,
                  const T* Q, const double* t1, const double* Zt, const float* PTt, const float* X,
                  const double* I, const double* T2d, const double* Gd, double* r2, hipStream_t s) {
   CCX_CHECK((T2d == nullptr) == (Gd == nullptr), ERR_INTERNAL, "assemble_r2: t2 and G's diagonal go together");
   const int64_t tiles = ceil_div(v, 32);
   CCX_CHECK(o * (o + 1) / 2 < 65536 && tiles * tiles < (1ll << 31), ERR_ARG, "assemble_r2: grid too large");
   dim3 grid((unsigned)(tiles * tiles), (unsigned)(o * (o + 1) / 2));
-  assemble_r2_kernel<T><<<grid, 256, 0, s>>>(o, v, H, CP, CM, P, Q, t1, Zt, PTt, X, I, T2d, Gd, r2);
+  assemble_r2_kernel<T><<<grid, 256, 0, s>>>(o, v, h_parts, H, CP, CM, P, Q, t1, Zt, PTt, X, I, T2d, Gd, r2);
   CCX_HIP(hipGetLastError());
 }
 
@@ -888,12 +937,12 @@ template void ladder_pack<double>(int64_t, int64_t, int64_t, int64_t, VVVVSrc, c
                                   double*, hipStream_t);
 template void ladder_pack<float>(int64_t, int64_t, int64_t, int64_t, VVVVSrc, const double*, float*,
                                  float*, hipStream_t);
-template void zt_add<double>(int64_t, int64_t, const double*, const double*, double*, hipStream_t);
-template void zt_add<float>(int64_t, int64_t, const float*, const float*, double*, hipStream_t);
-template void assemble_r2<double>(int64_t, int64_t, const double*, const double*, const double*, const double*,
+template void zt_add<double>(int64_t, int64_t, const double*, const double*, const double*, double*, hipStream_t);
+template void zt_add<float>(int64_t, int64_t, const float*, const float*, const double*, double*, hipStream_t);
+template void assemble_r2<double>(int64_t, int64_t, int, const double*, const double*, const double*, const double*,
                                   const double*, const double*, const double*, const float*, const float*,
                                   const double*, const double*, const double*, double*, hipStream_t);
-template void assemble_r2<float>(int64_t, int64_t, const double*, const float*, const float*, const float*,
+template void assemble_r2<float>(int64_t, int64_t, int, const double*, const float*, const float*, const float*,
                                  const float*, const double*, const double*, const float*, const float*,
                                  const double*, const double*, const double*, double*, hipStream_t);
 template void cast<double, float>(int64_t, const double*, float*, hipStream_t);

@@ -1502,7 +1502,7 @@ void hh_g_x3(Ctx& c, const double* t2, float* X, hipStream_t s) {
 
 void fae_tauL_x3(Ctx& c, double* Fae, hipStream_t s) {
   const int64_t o = c.o, v = c.v, ov = c.ov(), v32 = c.v32();
-  x3_split_rows<double>(c.tau, o * ov, v, v, c.xs + 11, c.TFh, c.TFl, v32, s);   // tau~ [(m,n,a)][f]
+  x3_split_rows<double>(c.taut, o * ov, v, v, c.xs + 11, c.TFh, c.TFl, v32, s);   // tau~ [(m,n,a)][f]
   // the diagonal sums are of one sign (pair-energy-like): split K finely, sum the FP32 partials in
   // FP64 straight into Fae
   X3Gemm g;   // Fae[a][e] -= sum_(mn, f) tau~[(mn)][a][f] L[(mn)][e][f]
