@@ -103,18 +103,44 @@ struct PlainGemm {
   // split-K: when ktot > 0, grid.y runs over K chunks of length K (the last one shorter), each
   // chunk is a "batch" entry (a_b / b_b advance by one chunk) and ktot is the total K.
   int64_t ktot = 0;
-  // K concatenation (plain_gemm_kcat; A k-contiguous, FP64): k in [K1, K) reads A2 at k - K1 and
-  // row (m mod sw) sw + m / sw, the (x, y) -> (y, x) swap of a row m = x sw + y (M = sw^2); batch b
-  // adds b a2_b to A2.
-  const T* A2 = nullptr;
-  int64_t K1 = 0, sw = 0, a2_b = 0;
 };
 template <typename T>
 bool plain_gemm_ok(const PlainGemm<T>& p);
 template <typename T>
 void plain_gemm(const PlainGemm<T>& p, hipStream_t s);
-// C_b = alpha [A | A2_b swapped] B_b^T + beta C_b over K = K concatenated at K1 (FP64, A and B
-// k-contiguous, fields A2 .. a2_b above; K1 a multiple of 16).
-void plain_gemm_kcat(const PlainGemm<double>& p, hipStream_t s);
+// Blocks of the K-concatenated product s = 0, 1, 2 (Y1, Y2, Y3) of the triple (i, j, k) = (t.x, t.y,
+// t.z): (p, p2, q n + r, q2 n + r2) of [A_p | A_p2^s] . [B_(q,r) | B_(q2,r2)].
+__host__ __device__ inline int4 kcat_blocks(int4 t, int s, int n) {
+  const int i = t.x, j = t.y, k = t.z;
+  if (s == 0) return int4{i, j, j * n + k, i * n + k};
+  if (s == 1) return int4{i, k, k * n + j, i * n + j};
+  return int4{j, k, k * n + i, j * n + i};
+}
+
+// Tile t of nprod such products, three to a triple: the tiles of one triple's products at the same
+// rows (tm) are neighbours, so that the A rows that they share meet in an XCD's L2. Each triple
+// starts at another tm (a golden-section sequence): the XCDs, which are at different triples, would
+// otherwise read the same A rows at the same time.
+__device__ inline void kcat_tile(int64_t t, int64_t tiles_m, int64_t tiles_n, int64_t& b, int64_t& tm, int64_t& tn) {
+  const int64_t per = 3 * tiles_m * tiles_n, e = t / per, r = t - e * per;
+  const int64_t m = r / (3 * tiles_n), r2 = r - m * 3 * tiles_n, q = r2 / tiles_n;
+  tm = m + (((int64_t)((uint32_t)e * 2654435769u) * tiles_m) >> 32);
+  if (tm >= tiles_m) tm -= tiles_m;
+  b = 3 * e + q;
+  tn = r2 - q * tiles_n;
+}
+
+// The FP64 (T) products of ntri triples: C[3 e + s][m][z] = sum_kk [A_p | A_p2^s][m][kk] [B | B2][z][kk]
+// with the blocks of kcat_blocks(tri[e], s, n); A_p is v^2 rows and B_(q,r) v rows of Kp (a multiple
+// of 8), A^s is A with its row index m = x v + y read as y v + x, C blocks are v^2 rows of ldc.
+struct Kcat64 {
+  int64_t v, Kp, ldc;
+  int n;
+  int64_t ntri;
+  const double *A, *B;
+  double* C;
+  const int4* tri;
+};
+void kcat64(const Kcat64& p, hipStream_t s);
 
 }  // namespace ccx

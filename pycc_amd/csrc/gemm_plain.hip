@@ -102,27 +102,6 @@ struct PLoader {
       v[i] = x.u;
     }
   }
-  // row r of the tile at element offset roff[r] (an LDS table, relative to base) instead of r * ld;
-  // guarded like load_safe unless FASTL (rows beyond nrows / k beyond nk are zero)
-  template <bool FASTL>
-  __device__ __forceinline__ void load_off(const T* __restrict__ base, const int* roff, int64_t nrows, int64_t nk) {
-    if constexpr (!KC) return;   // row offsets are for k-contiguous tiles only
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int64_t o = roff[row[i]];
-      if constexpr (FASTL) {
-        v[i] = *(const uint4*)(base + o + seg[i] * VEC);
-      } else {
-        union { uint4 u; T e[VEC]; } x;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-          const int64_t k = (int64_t)seg[i] * VEC + e;
-          x.e[e] = (row[i] < nrows && k < nk) ? base[o + k] : T(0);
-        }
-        v[i] = x.u;
-      }
-    }
-  }
   __device__ __forceinline__ void store(PTile<T, R, BK, KC>& t) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) *(uint4*)&t.d[row[i]][seg[i] * VEC] = v[i];
@@ -131,8 +110,7 @@ struct PLoader {
 
 // BT = 128: 4 waves of 64 x 64, two workgroups per CU. BT = 256 (FP32 only): 4 waves of 128 x 128
 // (256 accumulator registers each), one workgroup per CU, 4x the MFMAs per LDS read and per barrier.
-// KCAT: the K-concatenated form of plain_gemm_kcat (A k-contiguous).
-template <typename T, int BK, bool A_KC, bool B_NC, int BT, bool KCAT = false>
+template <typename T, int BK, bool A_KC, bool B_NC, int BT>
 __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(PlainGemm<T> p) {
   constexpr int BM = BT, BN = BT, WM = BT / 2, WN = BT / 2, NBI = WM / 16, NBJ = WN / 16;
   typedef typename PAcc<T>::type acc_t;
@@ -170,22 +148,6 @@ __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(Plai
   PLoader<T, BN, BK, !B_NC> lb;
   la.init(tid);
   lb.init(tid);
-  // KCAT: the second operand's row offsets, one per tile row, in LDS (sw^2 lda < 2^31, checked on
-  // the host; rows past M clamp to row M - 1 and are not stored). The barrier before the k loop
-  // publishes them.
-  // The first operand's rows get the same treatment (offsets r lda from the tile origin), so that
-  // one load path serves both.
-  const T* A2 = KCAT ? p.A2 + blockIdx.y * p.a2_b : nullptr;
-  __shared__ int roff[2][KCAT ? BM : 1];
-  if constexpr (KCAT) {
-    if (tid < BM) {
-      const int64_t m = m0 + tid < p.M ? m0 + tid : p.M - 1;
-      roff[0][tid] = (int)(tid * p.lda);
-      roff[1][tid] = (int)(((m % p.sw) * p.sw + m / p.sw) * p.lda);
-    }
-    __syncthreads();
-  }
-
   acc_t acc[NBI][NBJ];
 #pragma unroll
   for (int i = 0; i < NBI; ++i)
@@ -200,10 +162,7 @@ __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(Plai
     constexpr bool FAST = decltype(fast_tag)::value;
     auto load = [&](int64_t k0) {
       const int64_t nk = Kb - k0;
-      if constexpr (KCAT) {   // the k-tiles past K1 read the second operand (block-uniform)
-        const bool second = k0 >= p.K1;
-        la.template load_off<FAST>(second ? A2 + (k0 - p.K1) : a_at(k0), roff[second ? 1 : 0], a_rows, nk);
-      } else if constexpr (FAST) {
+      if constexpr (FAST) {
         la.load_fast(a_at(k0), p.lda);
       } else {
         la.load_safe(a_at(k0), p.lda, a_rows, nk);
@@ -290,6 +249,129 @@ void launch_plain(const PlainGemm<T>& p, hipStream_t s) {
   CCX_HIP(hipGetLastError());
 }
 
+typedef double d2p __attribute__((ext_vector_type(2)));
+
+// 16 bytes per lane from global memory into LDS at lds + 16 lane, no register in between
+__device__ __forceinline__ void dma16(const double* g, const double* lds) {
+  const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const double*)lds;
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory");
+}
+
+// The (T) products (kcat64): 128 x 16 NBJ tiles, 4 waves of 32 rows by all 16 NBJ columns. A stage is
+// 8 k values of every row; its operands go from global memory straight into LDS
+// (global_load_lds_dwordx4) through 4 buffers, so that three stages are in flight while one feeds
+// 4 NBJ MFMAs (64 cycles each) per wave, with one barrier per stage. LDS rows are 64 bytes with the
+// 16-byte chunk c of row r at c ^ (r / 2 % 4): neither the DMA nor the fragment reads (8 lanes to a
+// cycle, eight rows of one chunk) conflict. Every wave issues the same number of DMA instructions
+// per stage (blocks past NBJ land in rows of sB that are never read), so that one immediate count
+// waits for a stage. Rows past v^2 or v load a valid row; their results are not stored.
+// Bound by the FP64 MFMA rate (a library product reaches 72.8 TFLOP/s): 67 TFLOP/s of padded work at K =
+// 960, 63 at v = 112 K = 256, 58 at v = 107 K = 240 (40 triples, ends of the short k loop exposed).
+// Fragments loaded straight from global memory: 56, 53, 51; two buffers: 65, 62, 56; registers and
+// LDS with checked loads (v = 107, K padded to 256): 35.
+template <int NBJ>
+__global__ __launch_bounds__(256, 2) void kcat64_kernel(Kcat64 p, int64_t tiles_m, int64_t tiles_n) {
+  constexpr int NB = (NBJ + 3) / 4, D = 2 + NB, ST = 4, BLK = 16 * 8;   // doubles per 16-row block
+  __shared__ __attribute__((aligned(1024))) double sA[ST][8][BLK];
+  __shared__ __attribute__((aligned(1024))) double sB[ST][4 * NB][BLK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fr = lane >> 4, fc = lane & 15;
+  int64_t b, tm, tn;
+  kcat_tile(pxcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, b, tm, tn);
+  const int64_t e = b / 3;
+  const int4 blk = kcat_blocks(p.tri[e], (int)(b - 3 * e), p.n);
+  const int64_t v = p.v, vv = v * v, Kp = p.Kp, ldc = p.ldc, m0 = tm * 128, n0 = tn * (16 * NBJ);
+  // DMA lane: row lane / 4 of its block, chunk (lane % 4) ^ (row / 2 % 4)
+  const int dr = lane >> 2, dc = (lane & 3) ^ ((dr >> 1) & 3);
+  const double *pA[2], *pA2[2], *pB[NB], *pB2[NB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int64_t r = m0 + 16 * (2 * wave + i) + dr, m = r < vv ? r : vv - 1, x = m / v, y = m - x * v;
+    pA[i] = p.A + (blk.x * vv + m) * Kp + 2 * dc;
+    pA2[i] = p.A + (blk.y * vv + y * v + x) * Kp + 2 * dc;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int64_t r = n0 + 16 * (wave + 4 * i) + dr, n = r < v ? r : v - 1;
+    pB[i] = p.B + (blk.z * v + n) * Kp + 2 * dc;
+    pB2[i] = p.B + (blk.w * v + n) * Kp + 2 * dc;
+  }
+  d4p acc[2][NBJ];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j) acc[i][j] = d4p{0, 0, 0, 0};
+  const int half = (int)(Kp / 8), nst = 2 * half;
+  int st = 0;
+  auto issue = [&](int q) {   // stage st into buffer q, then on to the next (past the last: the last again)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dma16(pA[i], &sA[q][2 * wave + i][0]);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) dma16(pB[i], &sB[q][wave + 4 * i][0]);
+    if (++st == half) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) pA[i] = pA2[i];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) pB[i] = pB2[i];
+    } else if (st < nst) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) pA[i] += 8;
+#pragma unroll
+      for (int i = 0; i < NB; ++i) pB[i] += 8;
+    }
+  };
+  const int fo = fc * 8 + ((fr ^ ((fc >> 1) & 3)) * 2);   // fragment: row fc, chunk fr
+#pragma unroll
+  for (int q = 0; q < ST - 1; ++q) issue(q);
+  auto step = [&](auto buf) {
+    constexpr int q = decltype(buf)::value;
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((ST - 2) * D) : "memory");
+    issue((q + ST - 1) % ST);
+    d2p fa[2], fb[NBJ];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fa[i] = *(const d2p*)&sA[q][2 * wave + i][fo];
+#pragma unroll
+    for (int j = 0; j < NBJ; ++j) fb[j] = *(const d2p*)&sB[q][j][fo];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < NBJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i][j] = pmfma(fa[i][h], fb[j][h], acc[i][j]);
+  };
+  constexpr std::integral_constant<int, 0> b0{};
+  constexpr std::integral_constant<int, 1> b1{};
+  constexpr std::integral_constant<int, 2> b2{};
+  constexpr std::integral_constant<int, 3> b3{};
+  int s = 0;
+  for (; s + 4 <= nst; s += 4) {
+    step(b0);
+    step(b1);
+    step(b2);
+    step(b3);
+  }
+  if (s < nst) {   // nst is even
+    step(b0);
+    step(b1);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the DMA into LDS ends before the work-group does
+
+  double* C = p.C + b * vv * ldc;
+#pragma unroll
+  for (int j = 0; j < NBJ; ++j) {
+    const int64_t n = n0 + 16 * j + fc;
+    if (n >= v) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t m = m0 + 16 * (2 * wave + i) + 4 * r + fr;
+        if (m < vv) C[m * ldc + n] = acc[i][j][r];
+      }
+  }
+}
+
 }  // namespace
 
 template <typename T>
@@ -313,14 +395,24 @@ void plain_gemm(const PlainGemm<T>& p, hipStream_t s) {
   else launch_plain<T, false, false>(p, s);
 }
 
-void plain_gemm_kcat(const PlainGemm<double>& p, hipStream_t s) {
-  if (p.M == 0 || p.N == 0 || p.batch == 0) return;
-  CCX_CHECK(plain_gemm_ok(p) && p.a_kc && !p.b_nc && p.ktot == 0 && p.A2 && p.K1 > 0 && p.K1 % 16 == 0 &&
-                p.K1 < p.K && p.sw > 0 && p.sw * p.sw == p.M && p.M * p.lda < (int64_t(1) << 31) &&
-                ((uintptr_t)p.A2 % 16) == 0 && p.a2_b % 2 == 0,
-            ERR_INTERNAL, "plain_gemm_kcat layout");
-  const int64_t tiles = ceil_div(p.M, 128) * ceil_div(p.N, 128);
-  plain_gemm_kernel<double, 16, true, false, 128, true><<<dim3((unsigned)tiles, (unsigned)p.batch), 256, 0, s>>>(p);
+void kcat64(const Kcat64& p, hipStream_t s) {
+  if (p.ntri == 0 || p.v == 0) return;
+  const int64_t tm = ceil_div(p.v * p.v, 128), tn = ceil_div(p.v, 128), nbj = ceil_div(ceil_div(p.v, tn), 16);
+  CCX_CHECK(p.Kp % 8 == 0 && p.Kp > 0 && p.ldc >= p.v && ((uintptr_t)p.A | (uintptr_t)p.B) % 16 == 0,
+            ERR_INTERNAL, "kcat64 layout");
+  const int64_t blocks = tm * tn * 3 * p.ntri;
+  CCX_CHECK(blocks < (int64_t(1) << 31), ERR_ARG, "(T) GEMM grid too large");
+  const dim3 g((unsigned)blocks);
+  switch (nbj) {
+    case 1: kcat64_kernel<1><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 2: kcat64_kernel<2><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 3: kcat64_kernel<3><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 4: kcat64_kernel<4><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 5: kcat64_kernel<5><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 6: kcat64_kernel<6><<<g, 256, 0, s>>>(p, tm, tn); break;
+    case 7: kcat64_kernel<7><<<g, 256, 0, s>>>(p, tm, tn); break;
+    default: kcat64_kernel<8><<<g, 256, 0, s>>>(p, tm, tn); break;
+  }
   CCX_HIP(hipGetLastError());
 }
 

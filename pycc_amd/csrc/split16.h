@@ -33,11 +33,13 @@ struct X3Gemm {
   // split-K (set by x3_gemm): grid.y = splits K ranges of kchunk, raw partials in work[s][M][N]
   int64_t kchunk = 0;
   float* work = nullptr;
-  // x3_gemm_kcat only (interleaved operands, FP32 C): k in [K1, Kp) reads A from Ah2 (lo = Ah2 +
-  // 32) at k - K1 and row (m mod sw) sw + m / sw, the (x, y) -> (y, x) swap of a row m = x sw + y
-  // (M = sw^2); batch b of nbatch adds b sA2 to Ah2, b sB to Bh and Bl, and b sC to C.
-  const void* Ah2 = nullptr;
-  int64_t K1 = 0, sw = 0, nbatch = 1, sA2 = 0, sB = 0, sC = 0;
+  // x3_gemm_kcat only (interleaved operands, FP32 C): product b = 3 e + s of nbatch reads k < K1 from
+  // A_p, B_(q,r) and k in [K1, Kp) at k - K1 from A_p2, B_(q2,r2), the blocks of kcat_blocks(tri[e], s,
+  // nocc); A_p2's row is (m mod sw) sw + m / sw, the (x, y) -> (y, x) swap of m = x sw + y (M =
+  // sw^2). Blocks of A, B, C are sA, sB, sC elements apart.
+  const int4* tri = nullptr;
+  int nocc = 0;
+  int64_t K1 = 0, sw = 0, nbatch = 1, sA = 0, sB = 0, sC = 0;
   // ytile (x3_gemm_kcat only, = sw = N, a multiple of 8): C element (m = x sw + y, n) goes to the
   // tiled layout [x][y / 8][n / 8][n % 8][y % 8] (ldc unused), so that an 8 x 8 (y, n) block is one
   // run of 256 bytes, stored column by column: the offset is (m - m % 8) sw + 8 n + m % 8
@@ -54,8 +56,8 @@ void x3_gemm(const X3Gemm& p, hipStream_t s, Workspace* ws = nullptr);
 // nothing, when the tile grid is under one full round (the caller then runs the FP64 GEMM).
 bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s);
 
-// nbatch FP16x3 GEMMs C_b = alpha / (sa sb) [A | A2_b swapped] [B_b] with K = Kp concatenated
-// from two operands (fields Ah2 .. sC above): the connected (T) numerators, two slot products per
+// nbatch FP16x3 GEMMs C_b = alpha / (sa sb) [A_p | A_p2 swapped] [B | B2] with K = Kp concatenated
+// from two blocks of each operand (fields tri .. sC above): the connected (T) numerators, two slot products per
 // GEMM. Output tiles of 384 x 192, 256 x 256 or 256 x 192, whichever pads M x N least.
 void x3_gemm_kcat(const X3Gemm& p, hipStream_t s);
 // max |x| over n elements as x3_partials() per-block partial maxima in `part`.

@@ -421,21 +421,31 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   const int wm = wave / WGN, wn = wave % WGN;
   const int64_t tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BN - 1) / BN;
   int64_t t = xcd_remap_x3(blockIdx.x, tiles_m * tiles_n * (KCAT ? p.nbatch : 1));
-  int64_t batch = 0;
-  if constexpr (KCAT) {
-    batch = t / (tiles_m * tiles_n);
-    t -= batch * tiles_m * tiles_n;
-  }
+  int64_t batch = 0, tm, tn;
+  if constexpr (KCAT) kcat_tile(t, tiles_m, tiles_n, batch, tm, tn);
   const E* __restrict__ Ah = (const E*)p.Ah;
   const E* __restrict__ Al = (const E*)p.Al;
-  const E* __restrict__ Bh = (const E*)p.Bh + batch * p.sB;
-  const E* __restrict__ Bl = (const E*)p.Bl + batch * p.sB;
-  const E* __restrict__ Ah2 = KCAT ? (const E*)p.Ah2 + batch * p.sA2 : nullptr;
+  const E* __restrict__ Bh = (const E*)p.Bh;
+  const E* __restrict__ Bl = (const E*)p.Bl;
+  const E *__restrict__ Ah2 = nullptr, *__restrict__ Bh2 = nullptr;
+  if constexpr (KCAT) {
+    const int64_t e = batch / 3;
+    const int4 blk = kcat_blocks(p.tri[e], (int)(batch - 3 * e), p.nocc);
+    Ah2 = Ah + blk.y * p.sA;
+    Bh2 = Bh + blk.w * p.sB;
+    Ah += blk.x * p.sA;
+    Al += blk.x * p.sA;
+    Bh += blk.z * p.sB;
+    Bl += blk.z * p.sB;
+  }
   const int64_t split = blockIdx.y;
-  const int64_t group = t / (GM * tiles_n), first_m = group * GM;
-  const int64_t gsize = tiles_m - first_m < GM ? tiles_m - first_m : GM;
-  const int64_t within = t - group * GM * tiles_n;
-  const int64_t tm = first_m + within % gsize, tn = within / gsize;
+  if constexpr (!KCAT) {
+    const int64_t group = t / (GM * tiles_n), first_m = group * GM;
+    const int64_t gsize = tiles_m - first_m < GM ? tiles_m - first_m : GM;
+    const int64_t within = t - group * GM * tiles_n;
+    tm = first_m + within % gsize;
+    tn = within / gsize;
+  }
 
   int64_t gA[IPW], gB[IPB];
   int gA2[KCAT ? IPW : 1];   // M lda < 2^31 (checked by x3_gemm_kcat)
@@ -470,8 +480,10 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
       ka = q * p.ska + r;
       kb = q * p.skb + r;
     }
-    if (KCAT && k0 >= p.K1) {   // second operand of the concatenation (wave-uniform)
+    const bool second = KCAT && k0 >= p.K1;   // second block of each operand (wave-uniform)
+    if (second) {
       const int64_t ka2 = ((k0 - p.K1) >> 5) * p.ska;
+      kb = ((k0 - p.K1) >> 5) * p.skb;
 #pragma unroll
       for (int i = 0; i < IPW; ++i) {
         x3_dma16<E>(Ah2 + gA2[i] + ka2, &sA[st][0][ldso[i]]);
@@ -487,8 +499,8 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
 #pragma unroll
     for (int i = 0; i < IPB; ++i) {
       if (wave + 8 * i < NIB) {   // wave-uniform
-        x3_dma16<E>(Bh + gB[i] + kb, &sB[st][0][ldsb[i]]);
-        x3_dma16<E>(Bl + gB[i] + kb, &sB[st][1][ldsb[i]]);
+        x3_dma16<E>((second ? Bh2 : Bh) + gB[i] + kb, &sB[st][0][ldsb[i]]);
+        x3_dma16<E>((second ? Bh2 + 32 : Bl) + gB[i] + kb, &sB[st][1][ldsb[i]]);
       }
     }
   };
@@ -1149,7 +1161,7 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
 void x3_gemm_kcat(const X3Gemm& p, hipStream_t s) {
   if (p.M == 0 || p.N == 0 || p.nbatch == 0) return;
   CCX_CHECK(p.kb == BK && p.ska == 2 * BK && p.skb == 2 * BK && p.Kp % BK == 0 && p.K1 % BK == 0 && p.K1 > 0 &&
-                p.K1 < p.Kp && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.Ah2 && p.C && !p.C64 && !p.work &&
+                p.K1 < p.Kp && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.tri && p.C && !p.C64 && !p.work &&
                 p.sw > 0 && p.sw * p.sw == p.M && p.M * p.lda < (int64_t(1) << 31) && p.beta == 0.f && !p.sbn &&
                 (p.ytile == 0 || (p.ytile % 8 == 0 && p.ytile == p.sw && p.ytile == p.N &&
                                    (uintptr_t)p.C % 16 == 0 && p.sC % 4 == 0)),

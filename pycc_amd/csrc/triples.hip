@@ -2,12 +2,13 @@
 // MIXED_F16X3 mode, whose slot GEMMs are FP16x3 with FP32 output (triples_energy_x3 below).
 //
 // For every occupied triple i >= j >= k the connected numerator W[a][b][c] (cctriples.py:27-72,
-// t3c_ijk without the denominator) comes from GEMMs against A_p = [Covvv[p] | t2[p]^T] (built once
-// per call): the six slot products, each holding two of the twelve t3c_ijk terms, pair up along K
-// into three GEMMs per triple (Y1, Y2, Y3 below), batched over up to T3_KC values of k for fixed
-// (i, j). One kernel per chunk then forms W from the three blocks, orbit by orbit of 8^3 tiles, in
-// LDS (W is never stored), adds the disconnected part (t3d_ijk, cctriples.py:108-146:
-// <ij|ab> t1_kc + t2_ijab f_kc and their permutations) to form V and reduces
+// t3c_ijk without the denominator) comes from GEMMs against A_p = [Covvv[p] | t2[p]^T]: the six
+// slot products, each holding two of the twelve t3c_ijk terms, pair up along K into three GEMMs per
+// triple (Y1, Y2, Y3 below). Their operands A_p, B_(q,r) and the disconnected factors are laid out
+// once per call; the triples then run in chunks of two launches each, the GEMMs of the chunk and one
+// kernel that forms W from the three blocks, orbit by orbit of 8^3 tiles, in LDS (W is never
+// stored), adds the disconnected part (t3d_ijk, cctriples.py:108-146: <ij|ab> t1_kc + t2_ijab f_kc
+// and their permutations) to form V and reduces
 //
 //   E_ijk = sum_abc V_abc (4 W_abc + W_bca + W_cab - 2 W_acb - 2 W_bac - 2 W_cba) / D_ijk^abc,
 //   E(T)  = sum_{i>=j>=k} (2 - d_ij - d_ik - d_jk) E_ijk,
@@ -15,8 +16,9 @@
 // which is t_tjl's sum over a >= b >= c of (Y - 2Z)(W_abc + W_bca + W_cab) + (Z - 2Y)(W_acb +
 // W_bac + W_cba) + 3X with its 1/(1 + d_ab + d_ac + d_bc) weights, rewritten as a full sum over
 // a, b, c (the bracket is symmetric under permutations of abc, so each unordered abc appears
-// 6 / (1 + d_ab + d_ac + d_bc) times). The per-triple partial sums are reduced in a fixed order, so
-// the result is deterministic.
+// 6 / (1 + d_ab + d_ac + d_bc) times). The partial sums are reduced per triple, then per i, in a
+// fixed order that knows nothing of the chunks, so the result is deterministic and ranges of i add
+// up to the same bits as one call.
 #include "ccsd.h"
 #include "contract.h"
 #include "split16.h"
@@ -26,23 +28,6 @@
 namespace ccx {
 
 namespace {
-
-__device__ __forceinline__ double t3_block_sum(double x) {   // blockDim.x <= 1024, a power of two
-  __shared__ double sh[1024];
-  sh[threadIdx.x] = x;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  double r = sh[0];
-  __syncthreads();
-  return r;
-}
-
-__global__ void t3_zero_kernel(double* e) {
-  if (threadIdx.x == 0) e[0] = 0.0;
-}
 
 // A[p][(x, y)][kk] = Covvv[p][x][y][kk] for kk < v, t2[p][kk - v][x][y] for v <= kk < v + o, 0 above:
 // the two t3c_ijk products that share p as one GEMM operand with K = v + o (padded to Kp).
@@ -70,15 +55,14 @@ struct DevBuf {
   void alloc(int64_t n) {
     CCX_HIP(hipMalloc((void**)&p, (size_t)std::max<int64_t>(n, 1) * sizeof(T)));
   }
-  ~DevBuf() {
+  void release() {
     if (p) (void)hipFree(p);
+    p = nullptr;
   }
+  ~DevBuf() { release(); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
 };
-
-// k values per chunk of a fixed (i, j)
-constexpr int T3_KC = 8;
 
 // ---- slot products paired along K ----------------------------------------------------------------
 // The slot products X_pqr[x][y][z] = sum_kk A_p[(x, y)][kk] B_(q,r)[z][kk] hold the twelve t3c_ijk
@@ -89,58 +73,22 @@ constexpr int T3_KC = 8;
 //   Y1[a][b][c] = X_ijk[a][b][c] + X_jik[b][a][c] = [A_i | A_j^s](a,b) . [B_(j,k) | B_(i,k)](c)
 //   Y2[a][c][b] = X_ikj[a][c][b] + X_kij[c][a][b] = [A_i | A_k^s](a,c) . [B_(k,j) | B_(i,j)](b)
 //   Y3[b][c][a] = X_jki[b][c][a] + X_kji[c][b][a] = [A_j | A_k^s](b,c) . [B_(k,i) | B_(j,i)](a)
-// so that W[a][b][c] = Y1[a][b][c] + Y2[a][c][b] + Y3[b][c][a]: FP64 GEMMs (plain_gemm_kcat) in
-// every mode but MIXED_F16X3, whose GEMMs are FP16x3 with FP32 output, in 8 x 8 (y, z) blocks
-// when v is a multiple of 8 (x3_gemm_kcat with ytile).
+// so that W[a][b][c] = Y1[a][b][c] + Y2[a][c][b] + Y3[b][c][a]: FP64 GEMMs (kcat64) in every mode
+// but MIXED_F16X3, whose GEMMs are FP16x3 with FP32 output, in 8 x 8 (y, z) blocks when v is a
+// multiple of 8 (x3_gemm_kcat with ytile).
 //
-// B rows of the chunk (i, j, k0 .. k0 + nk): block 3 e + s (s = 0, 1, 2 for Y1, Y2, Y3 of k = k0 + e)
-// holds, for z < v, [B_(q1,r1)[z] | B_(q2,r2)[z]] (2 Kp wide) with the pairs named above.
-__global__ void t3_pack_kcat_kernel(int64_t o, int64_t v, int64_t Kp, int i, int j, int k0, int nk,
-                                    const double* __restrict__ t2, const double* __restrict__ Cooov,
-                                    double* __restrict__ B) {
-  const int64_t L = 2 * Kp, total = 3 * (int64_t)nk * v * L;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t kk2 = e % L, row = e / L, blk = row / v, z = row - blk * v;
-    const int e3 = (int)(blk / 3), sl = (int)(blk - 3 * e3), k = k0 + e3;
-    const bool h = kk2 >= Kp;
-    const int64_t kk = h ? kk2 - Kp : kk2;
-    int q, r;
-    if (sl == 0) { q = h ? i : j; r = k; }        // (j, k) | (i, k)
-    else if (sl == 1) { q = h ? i : k; r = j; }   // (k, j) | (i, j)
-    else { q = h ? j : k; r = i; }                // (k, i) | (j, i)
+// B_(q,r) for all q, r < n: [(q n + r) v + z][kk], rows of Kp (zero past v + o).
+__global__ __launch_bounds__(256) void t3_operand_b_kernel(int64_t o, int64_t v, int64_t Kp, int64_t n,
+                                                           const double* __restrict__ t2,
+                                                           const double* __restrict__ Cooov, double* __restrict__ B) {
+  const int64_t total = n * n * v * Kp;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t kk = e % Kp, row = e / Kp, qr = row / v, z = row - qr * v, q = qr / n, r = qr - q * n;
     double val = 0.0;
-    if (kk < v) val = t2[(((int64_t)r * o + q) * v + z) * v + kk];
+    if (kk < v) val = t2[((r * o + q) * v + z) * v + kk];
     else if (kk < v + o) val = -Cooov[(((kk - v) * o + q) * o + r) * v + z];
     B[e] = val;
   }
-}
-
-// MIXED_F16X3: the same B rows split straight into interleaved FP16 hi/lo (hi of k-block q of a row
-// at 64 q, lo at 64 q + 32; rows of 2 L halves) with the scale sc[0]; work-group (x, row) takes
-// 256 consecutive kk2 of the row.
-__global__ __launch_bounds__(256) void t3_pack_split_kernel(int64_t o, int64_t v, int64_t Kp, int i, int j, int k0,
-                                                           const double* __restrict__ t2,
-                                                           const double* __restrict__ Cooov,
-                                                           const float* __restrict__ sc, _Float16* __restrict__ Bhl) {
-  const int64_t L = 2 * Kp, row = blockIdx.y, blk = row / v, z = row - blk * v;
-  const int e3 = (int)(blk / 3), sl = (int)(blk - 3 * e3), k = k0 + e3;
-  const int64_t kk2 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (kk2 >= L) return;
-  const bool h = kk2 >= Kp;
-  const int64_t kk = h ? kk2 - Kp : kk2;
-  int q, r;
-  if (sl == 0) { q = h ? i : j; r = k; }        // (j, k) | (i, k)
-  else if (sl == 1) { q = h ? i : k; r = j; }   // (k, j) | (i, j)
-  else { q = h ? j : k; r = i; }                // (k, i) | (j, i)
-  double val = 0.0;
-  if (kk < v) val = t2[(((int64_t)r * o + q) * v + z) * v + kk];
-  else if (kk < v + o) val = -Cooov[(((kk - v) * o + q) * o + r) * v + z];
-  const float x = (float)(val * (double)sc[0]);
-  const _Float16 hv = (_Float16)x;
-  const int64_t at = row * 2 * L + ((kk2 >> 5) << 6) + (kk2 & 31);
-  Bhl[at] = hv;
-  Bhl[at + 32] = (_Float16)(x - (float)hv);
 }
 
 // One work-group per (orbit {A >= B >= C} of 8^3 tiles, triple k0 + blockIdx.y): W of the orbit's
@@ -188,17 +136,20 @@ __device__ __forceinline__ double t3_rcp(double x) {
   return r;
 }
 
+// index of the pair p >= q
+__device__ __forceinline__ int64_t t3_pair(int p, int q) { return (int64_t)p * (p + 1) / 2 + q; }
+
 // TY: the type of Y and of W in LDS (float in MIXED_F16X3, double in the FP64 path). FULL (float
 // only): Y in the tiled layout of x3_gemm_kcat's ytile (v a multiple of 8, every tile whole); else
 // Y is [x][y][z] with rows of ldy elements and the tiles at the edge are partial.
-// The disconnected blocks come from PB (t3_pair_blocks_kernel) and t1, F. One work-group per (orbit,
-// triple) pair t = orbit + norb e of the 1-D grid, taken in an order that gives each XCD a
+// Y holds the chunk's blocks, triple e's Y1, Y2, Y3 at 3 e v^2 ldy. The disconnected blocks come
+// from PB (t3_pair_blocks_kernel) and t1, F. One work-group per (orbit, triple) pair t = orbit +
+// norb e of the 1-D grid, taken in an order that gives each XCD a
 // contiguous range of t (consecutive orbits share tiles, so their blocks meet in that XCD's L2).
 template <typename TY, bool FULL>
 __global__ __launch_bounds__(OT_THREADS) void t3_orbit_energy_kernel(
-    int64_t o, int64_t v, int64_t ldy, int i, int j, int k0, int nk, const TY* __restrict__ Y1,
-    const TY* __restrict__ Y2, const TY* __restrict__ Y3, const int* __restrict__ orbits, int64_t norb,
-    const double* __restrict__ F, int64_t nmo, const double* __restrict__ t1, const double* __restrict__ PB,
+    int64_t o, int64_t v, int64_t ldy, const int4* __restrict__ tri, const TY* __restrict__ Y,
+    const int* __restrict__ orbits, int64_t norb, const double* __restrict__ F, int64_t nmo, const double* __restrict__ t1, const double* __restrict__ PB,
     double* __restrict__ partials) {
   static_assert(!FULL || sizeof(TY) == 4, "the tiled Y layout is FP32");
   // for the tile (P0, P1, P2) of slot x, the slots of (P1, P2, P0), (P2, P0, P1), (P0, P2, P1),
@@ -219,11 +170,12 @@ __global__ __launch_bounds__(OT_THREADS) void t3_orbit_energy_kernel(
   __shared__ double sE[3][OE];
   int64_t tw;
   {   // hardware work-group id (round-robin over the 8 XCDs) -> t
-    const int64_t n = norb * nk, q = n / 8, r = n % 8, xcd = blockIdx.x % 8, w = blockIdx.x / 8;
+    const int64_t n = gridDim.x, q = n / 8, r = n % 8, xcd = blockIdx.x % 8, w = blockIdx.x / 8;
     tw = xcd * q + (xcd < r ? xcd : r) + w;
   }
-  const int e = (int)(tw / norb), k = k0 + e;
-  const int64_t ob = tw - (int64_t)e * norb;
+  const int64_t e = tw / norb;
+  const int i = tri[e].x, j = tri[e].y, k = tri[e].z;
+  const int64_t ob = tw - e * norb;
   const int64_t nt = (v + OE - 1) / OE, vv = v * v, ys = vv * ldy;
   const int code = orbits[ob];
   const int A = (int)(code / (nt * nt)), B = (int)(code / nt % nt), C = (int)(code % nt);
@@ -244,9 +196,9 @@ __global__ __launch_bounds__(OT_THREADS) void t3_orbit_energy_kernel(
   int kept = 0;
 #pragma unroll
   for (int x = 0; x < 6; ++x) kept |= (rep[x] == x) << x;
-  const TY* y1 = Y1 + e * ys;
-  const TY* y2 = Y2 + e * ys;
-  const TY* y3 = Y3 + e * ys;
+  const TY* y1 = Y + 3 * e * ys;
+  const TY* y2 = y1 + ys;
+  const TY* y3 = y2 + ys;
   // Box loads: the threads of half hf = t / 128 take the boxes of the slots 2 p + hf; thread (x, z,
   // yg) = (t / 16 % 8, t / 2 % 8, t % 2) the four elements y = 4 yg + u, u = 0..3, of the row x and
   // column z (in the tiled layout the 16 bytes at 32 z + 16 yg of the box's 256-byte run for x).
@@ -294,9 +246,9 @@ __global__ __launch_bounds__(OT_THREADS) void t3_orbit_energy_kernel(
 #pragma unroll
   for (int rr = 0; rr < NB; ++rr) {
     const int bi = min(4 * rr + w4, 17), x = bi / 3, d = bi - 3 * x;   // wave-uniform
-    const int pp = d == 0 ? 0 : (d == 1 ? 1 + e : 1 + nk + e);
+    const int64_t pp = t3_pair(d < 2 ? i : j, d == 0 ? j : k);
     const int rt = t3_slot_tile(x, d < 2 ? 0 : 1, A, B, C), ct = t3_slot_tile(x, d == 0 ? 1 : 2, A, B, C);
-    pd[rr] = *(const d2v*)(PB + 2 * ((((int64_t)pp * nt + rt) * nt + ct) * 64 + lane));
+    pd[rr] = *(const d2v*)(PB + 2 * (((pp * nt + rt) * nt + ct) * 64 + lane));
   }
   // the vectors: row R = t / 8 < 21 (t1 of the occupied (i, j, k)[R / 3] over tile (A, B, C)[R % 3]
   // for R < 9, then the f rows for R < 18, then eps over tile R - 18), element t % 8
@@ -409,47 +361,74 @@ __global__ __launch_bounds__(OT_THREADS) void t3_orbit_energy_kernel(
   if (threadIdx.x == 0) partials[tw] = (sw4[0] + sw4[1]) + (sw4[2] + sw4[3]);
 }
 
-// PB[pp][rt][ct][r][c] = (<p q|a b>, t2_pqab) at a = 8 rt + r, b = 8 ct + c (zero past v), for the pairs
-// pp = 0: (i, j), 1 + e: (i, k0 + e), 1 + nk + e: (j, k0 + e), e < nk: the disconnected factors of a
-// chunk as contiguous 8 x 8 blocks of (integral, amplitude) pairs.
-__global__ void t3_pair_blocks_kernel(int64_t o, int64_t v, int64_t nt, int i, int j, int k0, int nk,
-                                      const double* __restrict__ Ioovv, const double* __restrict__ t2,
-                                      double* __restrict__ PB) {
-  const int64_t per = nt * nt * 64, total = (1 + 2 * (int64_t)nk) * per;
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < total; x += (int64_t)gridDim.x * blockDim.x) {
-    const int pp = (int)(x / per);
-    const int64_t rem = x - pp * per, blk = rem >> 6, rt = blk / nt, ct = blk - rt * nt;
-    const int64_t a = 8 * rt + ((rem >> 3) & 7), b = 8 * ct + (rem & 7);
-    const int p = pp <= nk ? i : j, q = pp == 0 ? j : k0 + (pp <= nk ? pp - 1 : pp - 1 - nk);
+// PB[pair(p, q)][rt][ct][r][c] = (<p q|a b>, t2_pqab) at a = 8 rt + r, b = 8 ct + c (zero past v) for
+// q <= p < n: the disconnected factors as contiguous 8 x 8 blocks of (integral, amplitude) pairs.
+// One work-group per (pair, rt) of the grid (pairs, nt).
+__global__ __launch_bounds__(256) void t3_pair_blocks_kernel(int64_t o, int64_t v, int64_t nt,
+                                                             const double* __restrict__ Ioovv,
+                                                             const double* __restrict__ t2, double* __restrict__ PB) {
+  const int64_t pp = blockIdx.x, rt = blockIdx.y;
+  int64_t p = (int64_t)((sqrt(8.0 * (double)pp + 1.0) - 1.0) * 0.5);   // the root, to within one
+  while (p * (p + 1) / 2 > pp) --p;
+  while ((p + 1) * (p + 2) / 2 <= pp) ++p;
+  const int64_t q = pp - p * (p + 1) / 2;
+  double* out = PB + 2 * (pp * nt + rt) * nt * 64;
+  for (int64_t x = threadIdx.x; x < nt * 64; x += 256) {
+    const int64_t a = 8 * rt + ((x >> 3) & 7), b = 8 * (x >> 6) + (x & 7);
     double iv = 0.0, tv = 0.0;
     if (a < v && b < v) {
-      const int64_t off = ((int64_t)p * o + q) * v * v + a * v + b;
+      const int64_t off = (p * o + q) * v * v + a * v + b;
       iv = Ioovv[off];
       tv = t2[off];
     }
-    PB[2 * x] = iv;
-    PB[2 * x + 1] = tv;
+    out[2 * x] = iv;
+    out[2 * x + 1] = tv;
   }
 }
 
-// e[0] += sum over the chunk's triples (i, j, k0 + x) of weight * sum(partials[x][0 .. norb)), in a
-// fixed order: work-group g of T3_NSUM sums the weighted partials g, g + T3_NSUM, ... into sums[g],
-// then one work-group adds sums[0 .. T3_NSUM) to e[0].
-constexpr int T3_NSUM = 256;
-__global__ __launch_bounds__(256) void t3_chunk_sums_kernel(const double* __restrict__ partials, int64_t norb, int nk,
-                                                            int i, int j, int k0, double* __restrict__ sums) {
-  const int64_t n = (int64_t)nk * norb;
+// te[t] = weight of the triple tri[t] times the sum of its norb orbit partials, a work-group per
+// triple, in an order that depends on norb alone.
+__global__ __launch_bounds__(256) void t3_triple_sums_kernel(const double* __restrict__ partials, int64_t norb,
+                                                             const int4* __restrict__ tri, double* __restrict__ te) {
+  const double* part = partials + blockIdx.x * norb;
   double s = 0.0;
-  for (int64_t t = blockIdx.x + (int64_t)T3_NSUM * threadIdx.x; t < n; t += (int64_t)T3_NSUM * blockDim.x) {
-    const int k = k0 + (int)(t / norb);
-    s += (2.0 - (double)((i == j) + (i == k) + (j == k))) * partials[t];   // cctriples.py:237
+  for (int64_t t = threadIdx.x; t < norb; t += 256) s += part[t];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  __shared__ double sw[4];
+  if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int4 c = tri[blockIdx.x];
+    te[blockIdx.x] = (2.0 - (double)((c.x == c.y) + (c.x == c.z) + (c.y == c.z))) *   // cctriples.py:237
+                     ((sw[0] + sw[1]) + (sw[2] + sw[3]));
   }
-  s = t3_block_sum(s);
-  if (threadIdx.x == 0) sums[blockIdx.x] = s;
 }
-__global__ __launch_bounds__(T3_NSUM) void t3_accumulate_chunk_kernel(const double* __restrict__ sums, double* e) {
-  const double s = t3_block_sum(sums[threadIdx.x]);
-  if (threadIdx.x == 0) e[0] += s;
+
+// e = (add ? e : 0) + E_i0 + ... + E_(i1 - 1), one after the other; E_i is the sum of the
+// (i + 1)(i + 2) / 2 energies of the triples (i, j, k), which are contiguous in te, by one wave.
+__global__ __launch_bounds__(1024) void t3_accumulate_kernel(const double* __restrict__ te, int i0, int i1, bool add,
+                                                             double* e) {
+  __shared__ double sE[1024];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t t0 = (int64_t)i0 * (i0 + 1) * (i0 + 2) / 6;
+  double acc = add ? e[0] : 0.0;
+  for (int ib = i0; ib < i1; ib += 1024) {
+    const int n = i1 - ib < 1024 ? i1 - ib : 1024;
+    for (int x = wave; x < n; x += 16) {
+      const int64_t i = ib + x, at = i * (i + 1) * (i + 2) / 6 - t0, cnt = (i + 1) * (i + 2) / 2;
+      double s = 0.0;
+      for (int64_t t = lane; t < cnt; t += 64) s += te[at + t];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+      if (lane == 0) sE[x] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int x = 0; x < n; ++x) acc += sE[x];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) e[0] = acc;
 }
 
 // orbits {A >= B >= C} of the nt^3 tiles as (A nt + B) nt + C
@@ -461,178 +440,122 @@ std::vector<int> t3_orbits(int64_t nt) {
   return out;
 }
 
-}  // namespace
+// Bytes of Y (3 v^3 elements per triple) that a chunk may hold, at least one triple: enough tiles for
+// the last, partly filled round of work-groups of a launch to cost little, yet little to allocate.
+// o = 11 v = 107 FP64: 12.6 ms at 330 MB, 12.3 at 526, 12.2 at 1 GB, 67-85 for a first call at 2.2 GB;
+// o = 24 v = 176 FP16x3: 185.5, 182.3, 180.5 ms.
+constexpr int64_t T3_Y_BYTES = int64_t(512) << 20;
+// Orbit partials held before they are summed per triple (64 MB).
+constexpr int64_t T3_PARTIALS = int64_t(1) << 23;
 
-// MIXED_F16X3: for fixed (i, j) the k values run in chunks of T3_KC; per chunk the K-concatenated
-// B rows (FP64, then split with one scale), the batched Y1, Y2, Y3 GEMMs and one orbit-energy launch.
-static void triples_energy_x3(Ctx& c, const double* F, const double* t1, const double* t2, int i0, int i1, bool accumulate,
-                              double* e_dev, hipStream_t s) {
-  const int64_t o = c.o, v = c.v, nmo = c.nmo, vv = v * v;
-  const int64_t nt = ceil_div(v, OE), KC = T3_KC;
-  const int64_t Kp = (v + o + 31) / 32 * 32, L = 2 * Kp;
-  // Y in 8 x 8 (y, z) blocks when v is a multiple of 8, else rows padded to 4 floats
-  const bool tiled = v % 8 == 0;
-  const int64_t ldy = tiled ? v : (v + 3) / 4 * 4;
-  const int64_t nA = (int64_t)i1 * vv * Kp, nBr = 3 * KC * v, np = x3_partials();
-  CCX_CHECK(vv * ldy * KC < (int64_t(1) << 40) && ceil_div(vv, 256) < (int64_t(1) << 24) && nBr < 65536, ERR_ARG,
-            "too many virtual orbitals for the (T) scratch");
-  DevBuf<f16> Ahl(nA * 2);   // A split, [i1 v^2][2 Kp]
-  DevBuf<float> sc(16 + 3 * np);   // sc[0] = scale of A, sc[1] = scale of B, then partials
-  // The entries of A over every p are exactly those of Covvv and of t2 (plus zero padding), so its
-  // scale is that of their union: the same for every range of i, whatever rows are built. Those
-  // of every chunk's B rows are entries of t2 and of -Cooov: B takes the scale of that union.
-  x3_absmax<double>(c.Covvv, o * vv * v, sc.p + 16, s);
-  x3_absmax<double>(t2, o * o * vv, sc.p + 16 + np, s);
-  x3_absmax<double>(c.Cooov, o * o * o * v, sc.p + 16 + 2 * np, s);
-  x3_scale_union(sc.p + 16, (int)(2 * np), sc.p, s);
-  x3_scale_union(sc.p + 16 + np, (int)(2 * np), sc.p + 1, s);
-  if (nA > 0) {   // A split; its FP64 form lives only until then
-    DevBuf<double> A64(nA);
-    t3_operand_a_kernel<<<(int)std::min<int64_t>(65536, ceil_div(nA, 256)), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2,
-                                                                                         A64.p);
-    CCX_HIP(hipGetLastError());
-    x3_split_rows<double>(A64.p, (int64_t)i1 * vv, Kp, Kp, sc.p, Ahl.p, Ahl.p + 32, Kp, s, true);
-    CCX_HIP(hipStreamSynchronize(s));
-  }
-  const std::vector<int> orb = t3_orbits(nt);
-  const int64_t norb = (int64_t)orb.size();
-  DevBuf<int> dorb(norb);
-  CCX_HIP(hipMemcpy(dorb.p, orb.data(), (size_t)norb * sizeof(int), hipMemcpyHostToDevice));
-  DevBuf<f16> Bhl(nBr * 2 * L);      // the K-concatenated B rows of a chunk, split: rows of 2 L halves
-  const int64_t ys = vv * ldy;          // one triple's Y block (see t3_orbit_energy_kernel)
-  DevBuf<float> Y(3 * KC * ys);        // Y1, Y2, Y3 of the chunk's triples
-  DevBuf<double> part(KC * norb + T3_NSUM);   // per (orbit, triple), then the chunk's T3_NSUM sums
-  DevBuf<double> PB((1 + 2 * KC) * nt * nt * 64 * 2);   // the chunk's disconnected blocks
-  float *Y1 = Y.p, *Y2 = Y1 + KC * ys, *Y3 = Y2 + KC * ys;
-  if (!accumulate) {
-    t3_zero_kernel<<<1, 64, 0, s>>>(e_dev);
-    CCX_HIP(hipGetLastError());
-  }
-  auto Ap = [&](int p) { return Ahl.p + (int64_t)p * vv * 2 * Kp; };
-  for (int i = i0; i < i1; ++i)
-    for (int j = 0; j <= i; ++j)
-      for (int k0 = 0; k0 <= j; k0 += (int)KC) {
-        const int nk = (int)std::min<int64_t>(KC, j + 1 - k0);
-        const int64_t nrows = 3 * (int64_t)nk * v;
-        t3_pack_split_kernel<<<dim3((unsigned)ceil_div(L, 256), (unsigned)nrows), 256, 0, s>>>(
-            o, v, Kp, i, j, k0, t2, c.Cooov, sc.p + 1, Bhl.p);
-        CCX_HIP(hipGetLastError());
-        X3Gemm g;   // C_e[m][n] = sum_kk [A | A2_e swapped][m][kk] B_e[n][kk]
-        g.M = vv; g.N = v; g.Kp = 2 * Kp; g.K1 = Kp; g.lda = 2 * Kp; g.ldb = 2 * L; g.ldc = ldy;
-        g.kb = 32; g.ska = 64; g.skb = 64; g.sw = v; g.nbatch = nk; g.ytile = tiled ? v : 0;
-        g.sa = sc.p; g.sb = sc.p + 1; g.sB = 3 * v * 2 * L; g.sC = ys;
-        // Y1 = [A_i | A_j^s] [B_(j,k) | B_(i,k)]
-        g.Ah = Ap(i); g.Al = Ap(i) + 32; g.Ah2 = Ap(j); g.sA2 = 0;
-        g.Bh = Bhl.p; g.Bl = Bhl.p + 32; g.C = Y1;
-        x3_gemm_kcat(g, s);
-        // Y2 = [A_i | A_k^s] [B_(k,j) | B_(i,j)]
-        g.Ah2 = Ap(k0); g.sA2 = vv * 2 * Kp;
-        g.Bh = Bhl.p + v * 2 * L; g.Bl = (const f16*)g.Bh + 32; g.C = Y2;
-        x3_gemm_kcat(g, s);
-        // Y3 = [A_j | A_k^s] [B_(k,i) | B_(j,i)]
-        g.Ah = Ap(j); g.Al = Ap(j) + 32;
-        g.Bh = Bhl.p + 2 * v * 2 * L; g.Bl = (const f16*)g.Bh + 32; g.C = Y3;
-        x3_gemm_kcat(g, s);
-        {
-          const int64_t nb = (1 + 2 * (int64_t)nk) * nt * nt * 64;
-          t3_pair_blocks_kernel<<<(int)std::min<int64_t>(8192, ceil_div(nb, 256)), 256, 0, s>>>(
-              o, v, nt, i, j, k0, nk, c.Ioovv, t2, PB.p);
-          CCX_HIP(hipGetLastError());
-        }
-        if (tiled)
-          t3_orbit_energy_kernel<float, true><<<(unsigned)(norb * nk), OT_THREADS, 0, s>>>(
-              o, v, ldy, i, j, k0, nk, Y1, Y2, Y3, dorb.p, norb, F, nmo, t1, PB.p, part.p);
-        else
-          t3_orbit_energy_kernel<float, false><<<(unsigned)(norb * nk), OT_THREADS, 0, s>>>(
-              o, v, ldy, i, j, k0, nk, Y1, Y2, Y3, dorb.p, norb, F, nmo, t1, PB.p, part.p);
-        CCX_HIP(hipGetLastError());
-        t3_chunk_sums_kernel<<<T3_NSUM, 256, 0, s>>>(part.p, norb, nk, i, j, k0, part.p + KC * norb);
-        CCX_HIP(hipGetLastError());
-        t3_accumulate_chunk_kernel<<<1, T3_NSUM, 0, s>>>(part.p + KC * norb, e_dev);
-        CCX_HIP(hipGetLastError());
-      }
-  CCX_HIP(hipStreamSynchronize(s));
-}
+}  // namespace
 
 void triples_energy(Ctx& c, const double* F, const double* t1, const double* t2, int i0, int i1, bool accumulate,
                     double* e_dev, hipStream_t s) {
   CCX_CHECK(c.have_ints, ERR_STATE, "triples called before the integrals were set");
   CCX_CHECK(F && t1 && t2 && e_dev, ERR_ARG, "null argument");
   CCX_CHECK(0 <= i0 && i0 <= i1 && i1 <= c.o, ERR_ARG, "triples: need 0 <= i0 <= i1 <= no");
-  const int64_t o = c.o, v = c.v, nmo = c.nmo, vv = v * v, vvv = vv * v;
+  const int64_t o = c.o, v = c.v, nmo = c.nmo, vv = v * v;
   CCX_CHECK(c.Covvv && c.Cooov && c.Ioovv, ERR_STATE, "the context holds no FP64 <ov|vv>/<oo|ov> blocks");
-  const int64_t nt8 = ceil_div(v, OE);
-  CCX_CHECK(nt8 * nt8 * nt8 < (int64_t(1) << 31) && (nt8 + 2) * (nt8 + 1) * nt8 / 6 * T3_KC < (int64_t(1) << 31),
-            ERR_ARG, "too many virtual orbitals for the (T) tiles");
+  const int64_t nt = ceil_div(v, OE);
+  CCX_CHECK(nt * nt * nt < (int64_t(1) << 31) && (nt + 2) * (nt + 1) * nt / 6 < (int64_t(1) << 28), ERR_ARG,
+            "too many virtual orbitals for the (T) tiles");
   // In MIXED_F16X3 the slot GEMMs are FP16x3 split products (interleaved hi/lo operands, K padded
-  // to 32, FP32 accumulation and output, two slot products per GEMM); every other mode runs them
-  // in FP64.
+  // to 32, FP32 accumulation and output); every other mode runs them in FP64 (K padded to 8).
   const bool x3 = c.mode == MODE_MIXED_F16X3;
-  const int64_t Kp = x3 ? (v + o + 31) / 32 * 32 : (v + o + 15) / 16 * 16;
-  const int64_t KC = T3_KC;
-  // A: only the rows p < i1 are read by this range (p is one of i >= j >= k)
-  const int64_t nA = (int64_t)i1 * vv * Kp;
-  if (x3) {
-    triples_energy_x3(c, F, t1, t2, i0, i1, accumulate, e_dev, s);
-    return;
-  }
-  // For fixed (i, j) the k values run in chunks of KC. The six slot products pair up along K into
-  // the three products Y1, Y2, Y3 of triples_energy_x3 (FP64 here); per chunk they are three
-  // batched GEMMs (plain_gemm_kcat, a batch entry per k), then the chunk's disconnected blocks and
-  // one orbit-energy launch (W formed in LDS from Y, never stored). Scratch: Y1, Y2, Y3 (KC v^3
-  // each), the chunk's B rows (3 KC v x 2 Kp), its disconnected blocks, the orbit partials and A
-  // (i1 v^2 x Kp). (every region starts on a 256-byte boundary: the GEMM loads its operands 16
-  // bytes at a time)
-  auto r32 = [](int64_t n) { return (n + 31) / 32 * 32; };
-  const int64_t ot = ceil_div(v, OE);
-  const std::vector<int> orb = t3_orbits(ot);
-  const int64_t norb = (int64_t)orb.size();
-  DevBuf<int> dorb(norb);
-  CCX_HIP(hipMemcpy(dorb.p, orb.data(), (size_t)norb * sizeof(int), hipMemcpyHostToDevice));
-  const int64_t L = 2 * Kp, nY = r32(KC * vvv), nB = r32(3 * KC * v * L), nP = r32(KC * norb + T3_NSUM);
-  const int64_t nPB = r32((1 + 2 * KC) * ot * ot * 64 * 2);
-  DevBuf<double> buf(3 * nY + nB + nP + nPB + nA);
-  double *Y1 = buf.p, *Y2 = Y1 + nY, *Y3 = Y2 + nY, *B = Y3 + nY, *part = B + nB, *PB = part + nP;
-  double* A = PB + nPB;
-  if (nA > 0) {
-    t3_operand_a_kernel<<<(int)std::min<int64_t>(65536, ceil_div(nA, 256)), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2, A);
-    CCX_HIP(hipGetLastError());
-  }
-  if (!accumulate) {
-    t3_zero_kernel<<<1, 64, 0, s>>>(e_dev);
-    CCX_HIP(hipGetLastError());
-  }
-  auto Ap = [&](int p) { return A + (int64_t)p * vv * Kp; };
+  const int64_t kpad = x3 ? 32 : 8, Kp = (v + o + kpad - 1) / kpad * kpad;
+  // FP16x3: Y in 8 x 8 (y, z) blocks when v is a multiple of 8, else rows padded to 4 floats. FP64:
+  // rows padded to 128 bytes, whole lines for the GEMM's stores (odd v = 107: 12.6 to 12.1 ms).
+  const bool tiled = x3 && v % 8 == 0;
+  const int64_t ldp = x3 ? 4 : 16, ldy = tiled ? v : (v + ldp - 1) / ldp * ldp, ys = vv * ldy;
+  std::vector<int4> tri;   // i >= j >= k, i in [i0, i1): those of one i are contiguous
   for (int i = i0; i < i1; ++i)
     for (int j = 0; j <= i; ++j)
-      for (int k0 = 0; k0 <= j; k0 += (int)KC) {
-        const int nk = (int)std::min<int64_t>(KC, j + 1 - k0);
-        const int64_t nrows = 3 * (int64_t)nk * v;
-        t3_pack_kcat_kernel<<<(int)std::min<int64_t>(4096, ceil_div(nrows * L, 256)), 256, 0, s>>>(
-            o, v, Kp, i, j, k0, nk, t2, c.Cooov, B);
-        CCX_HIP(hipGetLastError());
-        PlainGemm<double> g;   // C_e[m][n] = sum_kk [A | A2_e swapped][m][kk] B_e[n][kk]
-        g.M = vv; g.N = v; g.K = L; g.K1 = Kp; g.sw = v; g.batch = nk;
-        g.lda = Kp; g.ldb = L; g.ldc = v; g.a_kc = true; g.b_nc = false;
-        g.b_b = 3 * v * L; g.c_b = vvv;
-        g.A = Ap(i); g.A2 = Ap(j); g.a2_b = 0; g.B = B; g.C = Y1;                   // [A_i | A_j^s]
-        plain_gemm_kcat(g, s);
-        g.A2 = Ap(k0); g.a2_b = vv * Kp; g.B = B + v * L; g.C = Y2;                // [A_i | A_k^s]
-        plain_gemm_kcat(g, s);
-        g.A = Ap(j); g.B = B + 2 * v * L; g.C = Y3;                                // [A_j | A_k^s]
-        plain_gemm_kcat(g, s);
-        const int64_t npb = (1 + 2 * (int64_t)nk) * ot * ot * 64;
-        t3_pair_blocks_kernel<<<(int)std::min<int64_t>(8192, ceil_div(npb, 256)), 256, 0, s>>>(
-            o, v, ot, i, j, k0, nk, c.Ioovv, t2, PB);
-        CCX_HIP(hipGetLastError());
-        t3_orbit_energy_kernel<double, false><<<(unsigned)(norb * nk), OT_THREADS, 0, s>>>(
-            o, v, v, i, j, k0, nk, Y1, Y2, Y3, dorb.p, norb, F, nmo, t1, PB, part);
-        CCX_HIP(hipGetLastError());
-        t3_chunk_sums_kernel<<<T3_NSUM, 256, 0, s>>>(part, norb, nk, i, j, k0, part + KC * norb);
-        CCX_HIP(hipGetLastError());
-        t3_accumulate_chunk_kernel<<<1, T3_NSUM, 0, s>>>(part + KC * norb, e_dev);
-        CCX_HIP(hipGetLastError());
+      for (int k = 0; k <= j; ++k) tri.push_back(int4{i, j, k, 0});
+  const int64_t ntri = (int64_t)tri.size();
+  const std::vector<int> orb = t3_orbits(nt);
+  const int64_t norb = (int64_t)orb.size();
+  const int64_t ybytes = 3 * ys * (x3 ? 4 : 8);
+  const int64_t KC = std::max<int64_t>(1, std::min(ntri, std::min(T3_Y_BYTES / ybytes, T3_PARTIALS / norb)));
+  CCX_CHECK(KC * norb < (int64_t(1) << 31), ERR_ARG, "too many virtual orbitals for the (T) tiles");
+  const int64_t group = std::max(KC, std::min(ntri, T3_PARTIALS / norb) / KC * KC);   // triples per sum of partials
+
+  // Operands and scratch: only p, q, r < i1 are read by this range of i.
+  const int64_t nA = (int64_t)i1 * vv * Kp, nB = (int64_t)i1 * i1 * v * Kp, npair = (int64_t)i1 * (i1 + 1) / 2;
+  DevBuf<int> dorb(norb);
+  DevBuf<int4> dtri(ntri);
+  CCX_HIP(hipMemcpyAsync(dorb.p, orb.data(), (size_t)norb * sizeof(int), hipMemcpyHostToDevice, s));
+  if (ntri > 0) CCX_HIP(hipMemcpyAsync(dtri.p, tri.data(), (size_t)ntri * sizeof(int4), hipMemcpyHostToDevice, s));
+  DevBuf<double> part(group * norb + ntri), PB(npair * nt * nt * 128), A64, B64, Y64;
+  double* te = part.p + group * norb;
+  DevBuf<f16> Ahl, Bhl;
+  DevBuf<float> Y32, sc;   // sc[0] = scale of A, sc[1] = scale of B, then partial maxima
+  auto grid = [](int64_t n) { return (unsigned)std::min<int64_t>(65536, ceil_div(n, 256)); };
+  if (ntri > 0) {
+    CCX_CHECK(npair < (int64_t(1) << 31) && nt < 65536, ERR_ARG, "too many orbitals for the (T) pair blocks");
+    t3_pair_blocks_kernel<<<dim3((unsigned)npair, (unsigned)nt), 256, 0, s>>>(o, v, nt, c.Ioovv, t2, PB.p);
+    CCX_HIP(hipGetLastError());
+    A64.alloc(nA);
+    B64.alloc(nB);
+    t3_operand_a_kernel<<<grid(nA), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2, A64.p);
+    CCX_HIP(hipGetLastError());
+    t3_operand_b_kernel<<<grid(nB), 256, 0, s>>>(o, v, Kp, i1, t2, c.Cooov, B64.p);
+    CCX_HIP(hipGetLastError());
+  }
+  if (x3 && ntri > 0) {
+    // The entries of A over every p are exactly those of Covvv and of t2 (plus zero padding), so its
+    // scale is that of their union: the same for every range of i, whatever rows are built. Those
+    // of B are entries of t2 and of -Cooov: B takes the scale of that union.
+    const int64_t np = x3_partials();
+    sc.alloc(16 + 3 * np);
+    x3_absmax<double>(c.Covvv, o * vv * v, sc.p + 16, s);
+    x3_absmax<double>(t2, o * o * vv, sc.p + 16 + np, s);
+    x3_absmax<double>(c.Cooov, o * o * o * v, sc.p + 16 + 2 * np, s);
+    x3_scale_union(sc.p + 16, (int)(2 * np), sc.p, s);
+    x3_scale_union(sc.p + 16 + np, (int)(2 * np), sc.p + 1, s);
+    Ahl.alloc(nA * 2);
+    Bhl.alloc(nB * 2);
+    x3_split_rows<double>(A64.p, (int64_t)i1 * vv, Kp, Kp, sc.p, Ahl.p, Ahl.p + 32, Kp, s, true);
+    x3_split_rows<double>(B64.p, (int64_t)i1 * i1 * v, Kp, Kp, sc.p + 1, Bhl.p, Bhl.p + 32, Kp, s, true);
+    CCX_HIP(hipStreamSynchronize(s));
+    A64.release();   // their FP64 forms live only until then
+    B64.release();
+  }
+  if (x3) Y32.alloc(3 * KC * ys);
+  else Y64.alloc(3 * KC * ys);
+  for (int64_t g0 = 0; g0 < ntri; g0 += group) {
+    const int64_t ng = std::min(group, ntri - g0);
+    for (int64_t c0 = g0; c0 < g0 + ng; c0 += KC) {
+      const int64_t nc = std::min(KC, g0 + ng - c0);
+      const int4* tr = dtri.p + c0;
+      double* pt = part.p + (c0 - g0) * norb;
+      const unsigned eg = (unsigned)(norb * nc);
+      if (x3) {
+        X3Gemm g;   // C_(e, s)[m][n] = sum_kk [A | A2 swapped][m][kk] [B | B2][n][kk]
+        g.M = vv; g.N = v; g.Kp = 2 * Kp; g.K1 = Kp; g.lda = 2 * Kp; g.ldb = 2 * Kp; g.ldc = ldy;
+        g.kb = 32; g.ska = 64; g.skb = 64; g.sw = v; g.nbatch = 3 * nc; g.ytile = tiled ? v : 0;
+        g.sa = sc.p; g.sb = sc.p + 1; g.sA = vv * 2 * Kp; g.sB = v * 2 * Kp; g.sC = ys;
+        g.tri = tr; g.nocc = i1;
+        g.Ah = Ahl.p; g.Al = Ahl.p + 32; g.Bh = Bhl.p; g.Bl = Bhl.p + 32; g.C = Y32.p;
+        x3_gemm_kcat(g, s);
+        if (tiled)
+          t3_orbit_energy_kernel<float, true><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y32.p, dorb.p, norb, F, nmo, t1,
+                                                                        PB.p, pt);
+        else
+          t3_orbit_energy_kernel<float, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y32.p, dorb.p, norb, F, nmo, t1,
+                                                                         PB.p, pt);
+      } else {
+        kcat64(Kcat64{v, Kp, ldy, i1, nc, A64.p, B64.p, Y64.p, tr}, s);
+        t3_orbit_energy_kernel<double, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y64.p, dorb.p, norb, F, nmo, t1,
+                                                                        PB.p, pt);
       }
+      CCX_HIP(hipGetLastError());
+    }
+    t3_triple_sums_kernel<<<(unsigned)ng, 256, 0, s>>>(part.p, norb, dtri.p + g0, te + g0);
+    CCX_HIP(hipGetLastError());
+  }
+  t3_accumulate_kernel<<<1, 1024, 0, s>>>(te, i0, i1, accumulate, e_dev);
+  CCX_HIP(hipGetLastError());
   CCX_HIP(hipStreamSynchronize(s));
 }
 
