@@ -403,12 +403,10 @@ __device__ __forceinline__ void x3_dma16(const E* g, const E* lds) {
                :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory");
 }
 
-// BN = 192, 256 or 320 output columns per tile (320: 128 x 80 per wave, 144 KiB of LDS; B's 20 row
-// blocks of 16 go to wave q % 8, so waves 0-3 load three and 4-7 two); BT = 256 or 384 rows (384
-// with BN = 192: 192 x 48 per wave, 144 KiB). KCAT: the K-concatenated, batched form of
+// BN = 16 n up to 256, or 320, output columns per tile (320: 128 x 80 per wave, 144 KiB of LDS; B's
+// BN / 16 row blocks of 16 go to wave q % 8); BT = 256 or 384 rows. KCAT: the K-concatenated, batched form of
 // x3_gemm_kcat (interleaved operands, FP32 C, no split K).
-// WGM: waves along M (2: 2 x 4 waves; 4: 4 x 2, e.g. 96 x 96 per wave for 384 x 192 tiles, which
-// holds fewer fragment registers than 192 x 48).
+// WGM: waves along M (2: 2 x 4 waves; 8: 8 x 1, the waves of the KCAT tiles of 384 x BN, 48 x BN each).
 template <typename E, int BN, bool KCAT = false, int BT = 256, bool YT = false, int WGM = 2>
 __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   typedef typename X3<E>::v8 v8;
@@ -448,7 +446,13 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   }
 
   int64_t gA[IPW], gB[IPB];
-  int gA2[KCAT ? IPW : 1];   // M lda < 2^31 (checked by x3_gemm_kcat)
+  // KCAT: offsets in the second blocks, so that 16-byte chunk g = 4 q + c of the concatenated K (q the
+  // k-tile, c the lane's chunk) is chunk g - K1 / 8 there (M lda < 2^31, checked by x3_gemm_kcat)
+  int gA2[KCAT ? IPW : 1], gB2[KCAT ? IPB : 1];
+  const auto chunk2 = [&](int c) {
+    const int K1c = (int)(p.K1 >> 3), c2 = (c - K1c) & 3;
+    return c2 * 8 - (K1c - c + c2) / 4 * 64;
+  };
   int ldso[IPW], ldsb[IPB];
 #pragma unroll
   for (int i = 0; i < IPW; ++i) {
@@ -457,7 +461,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     int64_t m = tm * BT + row;
     m = m < p.M ? m : p.M - 1;
     gA[i] = m * p.lda + c * 8;
-    if constexpr (KCAT) gA2[i] = (int)(((m % p.sw) * p.sw + m / p.sw) * p.lda + c * 8);
+    if constexpr (KCAT) gA2[i] = (int)(((m % p.sw) * p.sw + m / p.sw) * p.lda) + chunk2(c);
     ldso[i] = R0 * 32;
   }
 #pragma unroll
@@ -468,6 +472,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     int64_t n = tn * BN + row;
     n = n < p.N ? n : p.N - 1;
     gB[i] = n * p.ldb + c * 8;
+    if constexpr (KCAT) gB2[i] = (int)(n * p.ldb) + chunk2(c);
     ldsb[i] = R0 * 32;
   }
   auto issue = [&](int st, int64_t k0) {
@@ -480,14 +485,29 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
       ka = q * p.ska + r;
       kb = q * p.skb + r;
     }
-    const bool second = KCAT && k0 >= p.K1;   // second block of each operand (wave-uniform)
-    if (second) {
-      const int64_t ka2 = ((k0 - p.K1) >> 5) * p.ska;
-      kb = ((k0 - p.K1) >> 5) * p.skb;
+    if constexpr (KCAT) {
+      const bool first = k0 + BK <= p.K1, mixed = !first && k0 < p.K1;   // wave-uniform
 #pragma unroll
       for (int i = 0; i < IPW; ++i) {
-        x3_dma16<E>(Ah2 + gA2[i] + ka2, &sA[st][0][ldso[i]]);
-        x3_dma16<E>(Ah2 + 32 + gA2[i] + ka2, &sA[st][1][ldso[i]]);
+        const E* g = (first ? Ah + gA[i] : Ah2 + gA2[i]) + ka;
+        if (mixed) {
+          const int R0 = (wave * IPW + i) * 16, row = R0 + (lane >> 2), c = (lane & 3) ^ ((row >> 1) & 3);
+          if (k0 + 8 * c < p.K1) g = Ah + gA[i] + ka;
+        }
+        x3_dma16<E>(g, &sA[st][0][ldso[i]]);
+        x3_dma16<E>(g + 32, &sA[st][1][ldso[i]]);
+      }
+#pragma unroll
+      for (int i = 0; i < IPB; ++i) {
+        if (wave + 8 * i < NIB) {   // wave-uniform
+          const E* g = (first ? Bh + gB[i] : Bh2 + gB2[i]) + kb;
+          if (mixed) {
+            const int row = (wave + 8 * i) * 16 + (lane >> 2), c = (lane & 3) ^ ((row >> 1) & 3);
+            if (k0 + 8 * c < p.K1) g = Bh + gB[i] + kb;
+          }
+          x3_dma16<E>(g, &sB[st][0][ldsb[i]]);
+          x3_dma16<E>(g + 32, &sB[st][1][ldsb[i]]);
+        }
       }
     } else {
 #pragma unroll
@@ -495,12 +515,12 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
         x3_dma16<E>(Ah + gA[i] + ka, &sA[st][0][ldso[i]]);
         x3_dma16<E>(Al + gA[i] + ka, &sA[st][1][ldso[i]]);
       }
-    }
 #pragma unroll
-    for (int i = 0; i < IPB; ++i) {
-      if (wave + 8 * i < NIB) {   // wave-uniform
-        x3_dma16<E>((second ? Bh2 : Bh) + gB[i] + kb, &sB[st][0][ldsb[i]]);
-        x3_dma16<E>((second ? Bh2 + 32 : Bl) + gB[i] + kb, &sB[st][1][ldsb[i]]);
+      for (int i = 0; i < IPB; ++i) {
+        if (wave + 8 * i < NIB) {   // wave-uniform
+          x3_dma16<E>(Bh + gB[i] + kb, &sB[st][0][ldsb[i]]);
+          x3_dma16<E>(Bl + gB[i] + kb, &sB[st][1][ldsb[i]]);
+        }
       }
     }
   };
@@ -1160,34 +1180,37 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
 
 void x3_gemm_kcat(const X3Gemm& p, hipStream_t s) {
   if (p.M == 0 || p.N == 0 || p.nbatch == 0) return;
-  CCX_CHECK(p.kb == BK && p.ska == 2 * BK && p.skb == 2 * BK && p.Kp % BK == 0 && p.K1 % BK == 0 && p.K1 > 0 &&
+  CCX_CHECK(p.kb == BK && p.ska == 2 * BK && p.skb == 2 * BK && p.Kp % BK == 0 && p.K1 % 8 == 0 && p.K1 > 0 &&
                 p.K1 < p.Kp && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.tri && p.C && !p.C64 && !p.work &&
                 p.sw > 0 && p.sw * p.sw == p.M && p.M * p.lda < (int64_t(1) << 31) && p.beta == 0.f && !p.sbn &&
                 (p.ytile == 0 || (p.ytile % 8 == 0 && p.ytile == p.sw && p.ytile == p.N &&
                                    (uintptr_t)p.C % 16 == 0 && p.sC % 4 == 0)),
             ERR_INTERNAL, "x3 K-concatenated GEMM layout");
-  // the output tile (384 x 192, 256 x 256 or 256 x 192) that pads M x N least, in that order on a
-  // tie (the 320-column tile spills registers in this form)
-  const int shapes[3][2] = {{384, 192}, {256, 256}, {256, 192}};
-  int pick = 0;
-  double best = 0.0;
-  for (int c = 0; c < 3; ++c) {
-    const double area = (double)(ceil_div(p.M, shapes[c][0]) * shapes[c][0]) *
-                        (double)(ceil_div(p.N, shapes[c][1]) * shapes[c][1]);
-    if (c == 0 || area < best) {
-      best = area;
-      pick = c;
-    }
-  }
-  const int64_t tiles = ceil_div(p.M, shapes[pick][0]) * ceil_div(p.N, shapes[pick][1]) * p.nbatch;
+  // Every column tile reads the A rows again, which costs about as much as 440 columns of products (v
+  // = 128: 384 x 128, 160, 192 tiles 485, 538, 538 us for 30 triples): as few column tiles as 256
+  // columns allow, in 384-row tiles as narrow as v leaves them (192: 634 us at v = 128, 367 to 292 at v
+  // = 107, 782 to 777 at v = 176 for 16 triples), and in 256 x 256 past 192 (v = 224: 631 us against
+  // 727 for two tiles of 112).
+  const int64_t tn = ceil_div(p.N, 256), bn = std::max<int64_t>((ceil_div(p.N, tn) + 15) / 16 * 16, 64);
+  const int BT = bn <= 192 ? 384 : 256;
+  const int64_t tiles = ceil_div(p.M, BT) * tn * p.nbatch;
   CCX_CHECK(tiles < (1ll << 31), ERR_ARG, "x3 GEMM grid too large");
-  const bool yt = p.ytile > 0;
-  if (pick == 0 && yt) x3_gemm_dma_kernel<_Float16, 192, true, 384, true, 4><<<(unsigned)tiles, 512, 0, s>>>(p);
-  else if (pick == 0) x3_gemm_dma_kernel<_Float16, 192, true, 384, false, 4><<<(unsigned)tiles, 512, 0, s>>>(p);
-  else if (pick == 1 && yt) x3_gemm_dma_kernel<_Float16, 256, true, 256, true><<<(unsigned)tiles, 512, 0, s>>>(p);
-  else if (pick == 1) x3_gemm_dma_kernel<_Float16, 256, true><<<(unsigned)tiles, 512, 0, s>>>(p);
-  else if (yt) x3_gemm_dma_kernel<_Float16, 192, true, 256, true><<<(unsigned)tiles, 512, 0, s>>>(p);
-  else x3_gemm_dma_kernel<_Float16, 192, true><<<(unsigned)tiles, 512, 0, s>>>(p);
+  auto go = [&](auto cols, auto rows, auto waves_m) {
+    constexpr int BN = decltype(cols)::value, BR = decltype(rows)::value, W = decltype(waves_m)::value;
+    if (p.ytile) x3_gemm_dma_kernel<_Float16, BN, true, BR, true, W><<<(unsigned)tiles, 512, 0, s>>>(p);
+    else x3_gemm_dma_kernel<_Float16, BN, true, BR, false, W><<<(unsigned)tiles, 512, 0, s>>>(p);
+  };
+  constexpr std::integral_constant<int, 384> r384{};
+  constexpr std::integral_constant<int, 8> w8{};
+  if (bn <= 64) go(std::integral_constant<int, 64>{}, r384, w8);
+  else if (bn <= 96) go(std::integral_constant<int, 96>{}, r384, w8);
+  else if (bn <= 112) go(std::integral_constant<int, 112>{}, r384, w8);
+  else if (bn <= 128) go(std::integral_constant<int, 128>{}, r384, w8);
+  else if (bn <= 144) go(std::integral_constant<int, 144>{}, r384, w8);
+  else if (bn <= 160) go(std::integral_constant<int, 160>{}, r384, w8);
+  else if (bn <= 176) go(std::integral_constant<int, 176>{}, r384, w8);
+  else if (bn <= 192) go(std::integral_constant<int, 192>{}, r384, w8);
+  else go(std::integral_constant<int, 256>{}, std::integral_constant<int, 256>{}, std::integral_constant<int, 2>{});
   CCX_HIP(hipGetLastError());
 }
 
