@@ -318,7 +318,7 @@ int ccx_timing_read(ccx_ctx* ctx, double* out, int n) {
 }
 
 int64_t ccx_device_bytes(const ccx_ctx* ctx) {
-  return ctx ? ctx->c.bytes + (int64_t)ctx->c.ws.size : 0;
+  return ctx ? ctx->c.bytes + (int64_t)(ctx->c.ws.size + ctx->c.t3.size) : 0;
 }
 
 int ccx_contract(const char* subscripts, double alpha, const double* A, const int64_t* a_shape,

@@ -5,6 +5,7 @@
 #include "gemm.h"
 #include "kernels.h"
 #include "split16.h"
+#include <atomic>
 #include <vector>
 
 namespace ccx {
@@ -39,6 +40,8 @@ struct Ctx {
   int mode = MODE_DP;
   bool have_ints = false;
   Workspace ws;
+  Workspace t3;                      // the (T) scratch kept between calls, held by the call that set t3_busy
+  std::atomic<bool> t3_busy{false};
   std::vector<void*> owned;          // every hipMalloc of the context, freed by destroy()
   int64_t bytes = 0;                 // device bytes held in `owned`
 

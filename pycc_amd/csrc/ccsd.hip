@@ -28,6 +28,7 @@ void Ctx::destroy() {
   for (void* p : owned) (void)hipFree(p);
   owned.clear();
   ws.release();
+  t3.release();
   if (ev_fork) (void)hipEventDestroy(ev_fork);
   if (ev_join) (void)hipEventDestroy(ev_join);
   if (side) (void)hipStreamDestroy(side);

@@ -34,6 +34,7 @@ struct Workspace {
                     std::to_string(size) + " bytes");
       if (ptr) CCX_HIP(hipFree(ptr));
       ptr = nullptr;
+      size = 0;
       CCX_HIP(hipMalloc(&ptr, bytes));
       size = bytes;
     }

@@ -29,11 +29,30 @@ namespace ccx {
 
 namespace {
 
+// Element x of an operand, as it is or (SPLIT) as the interleaved FP16 pair of x sc (hi of k-block q of a
+// row at 64 q, lo 32 after it), for rows of Kp, a multiple of 32.
+template <bool SPLIT>
+__device__ __forceinline__ void t3_put(double x, double sc, void* out, int64_t row, int64_t kk, int64_t Kp) {
+  if constexpr (SPLIT) {
+    const float f = (float)(x * sc);
+    const _Float16 hv = (_Float16)f;
+    _Float16* d = (_Float16*)out + row * 2 * Kp + ((kk >> 5) << 6) + (kk & 31);
+    d[0] = hv;
+    d[32] = (_Float16)(f - (float)hv);
+  } else {
+    ((double*)out)[row * Kp + kk] = x;
+  }
+}
+
 // A[p][(x, y)][kk] = Covvv[p][x][y][kk] for kk < v, t2[p][kk - v][x][y] for v <= kk < v + o, 0 above:
 // the two t3c_ijk products that share p as one GEMM operand with K = v + o (padded to Kp).
-__global__ void t3_operand_a_kernel(int64_t o, int64_t v, int64_t Kp, int64_t nrow_p, const double* __restrict__ Covvv,
-                                    const double* __restrict__ t2, double* __restrict__ A) {
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void t3_operand_a_kernel(int64_t o, int64_t v, int64_t Kp, int64_t nrow_p,
+                                                           const double* __restrict__ Covvv,
+                                                           const double* __restrict__ t2, const float* __restrict__ sc,
+                                                           void* __restrict__ A) {
   const int64_t total = nrow_p * v * v * Kp;   // rows p < nrow_p
+  const double scale = SPLIT ? (double)sc[0] : 1.0;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t kk = e % Kp, row = e / Kp;   // row = (p, x, y)
@@ -41,27 +60,38 @@ __global__ void t3_operand_a_kernel(int64_t o, int64_t v, int64_t Kp, int64_t nr
     double val = 0.0;
     if (kk < v) val = Covvv[row * v + kk];
     else if (kk < v + o) val = t2[(p * o + (kk - v)) * v * v + xy];
-    A[e] = val;
+    t3_put<SPLIT>(val, scale, A, row, kk, Kp);
   }
 }
 
-// Device buffer owned by one call: freed on every exit, including an exception thrown after it was
-// allocated (hipFree waits for the work queued on the device before it releases the memory).
-template <typename T>
-struct DevBuf {
-  T* p = nullptr;
-  DevBuf() = default;
-  explicit DevBuf(int64_t n) { alloc(n); }
-  void alloc(int64_t n) {
-    CCX_HIP(hipMalloc((void**)&p, (size_t)std::max<int64_t>(n, 1) * sizeof(T)));
+// Scratch of one call, one block of device memory: up to T3_KEEP bytes the context keeps it for its next
+// call (an allocation of some 100 MB costs 0.2 to 1 ms, at times 10, against 0.2 ms for all of o = 6 v
+// = 30), unless another thread's call on the context holds it; else it is the call's own. Given back
+// on every exit, after the work queued on the stream.
+constexpr int64_t T3_KEEP = int64_t(2) << 30;
+struct T3Scratch {
+  Ctx& c;
+  hipStream_t s;
+  char* own = nullptr;
+  bool leased = false;
+  T3Scratch(Ctx& ctx, hipStream_t st) : c(ctx), s(st) {}
+  char* get(int64_t bytes) {
+    if (bytes <= T3_KEEP && !c.t3_busy.exchange(true)) {
+      leased = true;
+      return (char*)c.t3.get((size_t)bytes);
+    }
+    CCX_HIP(hipMalloc((void**)&own, (size_t)bytes));
+    return own;
   }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
+  ~T3Scratch() {
+    if (leased) {
+      (void)hipStreamSynchronize(s);
+      c.t3_busy = false;
+    }
+    if (own) (void)hipFree(own);   // waits for the work queued on the device
   }
-  ~DevBuf() { release(); }
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
+  T3Scratch(const T3Scratch&) = delete;
+  T3Scratch& operator=(const T3Scratch&) = delete;
 };
 
 // ---- slot products paired along K ----------------------------------------------------------------
@@ -78,16 +108,19 @@ struct DevBuf {
 // multiple of 8 (x3_gemm_kcat with ytile).
 //
 // B_(q,r) for all q, r < n: [(q n + r) v + z][kk], rows of Kp (zero past v + o).
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void t3_operand_b_kernel(int64_t o, int64_t v, int64_t Kp, int64_t n,
                                                            const double* __restrict__ t2,
-                                                           const double* __restrict__ Cooov, double* __restrict__ B) {
+                                                           const double* __restrict__ Cooov,
+                                                           const float* __restrict__ sc, void* __restrict__ B) {
   const int64_t total = n * n * v * Kp;
+  const double scale = SPLIT ? (double)sc[0] : 1.0;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t kk = e % Kp, row = e / Kp, qr = row / v, z = row - qr * v, q = qr / n, r = qr - q * n;
     double val = 0.0;
     if (kk < v) val = t2[((r * o + q) * v + z) * v + kk];
     else if (kk < v + o) val = -Cooov[(((kk - v) * o + q) * o + r) * v + z];
-    B[e] = val;
+    t3_put<SPLIT>(val, scale, B, row, kk, Kp);
   }
 }
 
@@ -486,76 +519,76 @@ void triples_energy(Ctx& c, const double* F, const double* t1, const double* t2,
 
   // Operands and scratch: only p, q, r < i1 are read by this range of i.
   const int64_t nA = (int64_t)i1 * vv * Kp, nB = (int64_t)i1 * i1 * v * Kp, npair = (int64_t)i1 * (i1 + 1) / 2;
-  DevBuf<int> dorb(norb);
-  DevBuf<int4> dtri(ntri);
-  CCX_HIP(hipMemcpyAsync(dorb.p, orb.data(), (size_t)norb * sizeof(int), hipMemcpyHostToDevice, s));
-  if (ntri > 0) CCX_HIP(hipMemcpyAsync(dtri.p, tri.data(), (size_t)ntri * sizeof(int4), hipMemcpyHostToDevice, s));
-  DevBuf<double> part(group * norb + ntri), PB(npair * nt * nt * 128), A64, B64, Y64;
-  double* te = part.p + group * norb;
-  DevBuf<f16> Ahl, Bhl;
-  DevBuf<float> Y32, sc;   // sc[0] = scale of A, sc[1] = scale of B, then partial maxima
+  const int64_t np = x3_partials(), esz = x3 ? 2 * sizeof(f16) : sizeof(double);
+  int64_t bytes = 0;
+  auto carve = [&](int64_t n) {   // every region starts on a 256-byte boundary
+    const int64_t at = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return at;
+  };
+  const int64_t aA = carve(nA * esz), aB = carve(nB * esz), aPB = carve(npair * nt * nt * 128 * 8);
+  const int64_t aY = carve(KC * ybytes), aP = carve(group * norb * 8), aT = carve(ntri * 8);
+  const int64_t aOrb = carve(norb * sizeof(int)), aTri = carve(ntri * sizeof(int4)), aSc = carve((16 + 3 * np) * 4);
+  T3Scratch scratch(c, s);
+  char* base = scratch.get(bytes);
+  void *A = base + aA, *B = base + aB, *Y = base + aY;
+  double *PB = (double*)(base + aPB), *part = (double*)(base + aP), *te = (double*)(base + aT);
+  int* dorb = (int*)(base + aOrb);
+  int4* dtri = (int4*)(base + aTri);
+  float* sc = (float*)(base + aSc);   // sc[0] = scale of A, sc[1] = scale of B, then partial maxima
+  CCX_HIP(hipMemcpyAsync(dorb, orb.data(), (size_t)norb * sizeof(int), hipMemcpyHostToDevice, s));
+  if (ntri > 0) CCX_HIP(hipMemcpyAsync(dtri, tri.data(), (size_t)ntri * sizeof(int4), hipMemcpyHostToDevice, s));
   auto grid = [](int64_t n) { return (unsigned)std::min<int64_t>(65536, ceil_div(n, 256)); };
   if (ntri > 0) {
     CCX_CHECK(npair < (int64_t(1) << 31) && nt < 65536, ERR_ARG, "too many orbitals for the (T) pair blocks");
-    t3_pair_blocks_kernel<<<dim3((unsigned)npair, (unsigned)nt), 256, 0, s>>>(o, v, nt, c.Ioovv, t2, PB.p);
+    t3_pair_blocks_kernel<<<dim3((unsigned)npair, (unsigned)nt), 256, 0, s>>>(o, v, nt, c.Ioovv, t2, PB);
     CCX_HIP(hipGetLastError());
-    A64.alloc(nA);
-    B64.alloc(nB);
-    t3_operand_a_kernel<<<grid(nA), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2, A64.p);
-    CCX_HIP(hipGetLastError());
-    t3_operand_b_kernel<<<grid(nB), 256, 0, s>>>(o, v, Kp, i1, t2, c.Cooov, B64.p);
+    if (x3) {
+      // The entries of A over every p are exactly those of Covvv and of t2 (plus zero padding), so its
+      // scale is that of their union: the same for every range of i, whatever rows are built. Those
+      // of B are entries of t2 and of -Cooov: B takes the scale of that union.
+      x3_absmax<double>(c.Covvv, o * vv * v, sc + 16, s);
+      x3_absmax<double>(t2, o * o * vv, sc + 16 + np, s);
+      x3_absmax<double>(c.Cooov, o * o * o * v, sc + 16 + 2 * np, s);
+      x3_scale_union(sc + 16, (int)(2 * np), sc, s);
+      x3_scale_union(sc + 16 + np, (int)(2 * np), sc + 1, s);
+      t3_operand_a_kernel<true><<<grid(nA), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2, sc, A);
+      t3_operand_b_kernel<true><<<grid(nB), 256, 0, s>>>(o, v, Kp, i1, t2, c.Cooov, sc + 1, B);
+    } else {
+      t3_operand_a_kernel<false><<<grid(nA), 256, 0, s>>>(o, v, Kp, i1, c.Covvv, t2, nullptr, A);
+      t3_operand_b_kernel<false><<<grid(nB), 256, 0, s>>>(o, v, Kp, i1, t2, c.Cooov, nullptr, B);
+    }
     CCX_HIP(hipGetLastError());
   }
-  if (x3 && ntri > 0) {
-    // The entries of A over every p are exactly those of Covvv and of t2 (plus zero padding), so its
-    // scale is that of their union: the same for every range of i, whatever rows are built. Those
-    // of B are entries of t2 and of -Cooov: B takes the scale of that union.
-    const int64_t np = x3_partials();
-    sc.alloc(16 + 3 * np);
-    x3_absmax<double>(c.Covvv, o * vv * v, sc.p + 16, s);
-    x3_absmax<double>(t2, o * o * vv, sc.p + 16 + np, s);
-    x3_absmax<double>(c.Cooov, o * o * o * v, sc.p + 16 + 2 * np, s);
-    x3_scale_union(sc.p + 16, (int)(2 * np), sc.p, s);
-    x3_scale_union(sc.p + 16 + np, (int)(2 * np), sc.p + 1, s);
-    Ahl.alloc(nA * 2);
-    Bhl.alloc(nB * 2);
-    x3_split_rows<double>(A64.p, (int64_t)i1 * vv, Kp, Kp, sc.p, Ahl.p, Ahl.p + 32, Kp, s, true);
-    x3_split_rows<double>(B64.p, (int64_t)i1 * i1 * v, Kp, Kp, sc.p + 1, Bhl.p, Bhl.p + 32, Kp, s, true);
-    CCX_HIP(hipStreamSynchronize(s));
-    A64.release();   // their FP64 forms live only until then
-    B64.release();
-  }
-  if (x3) Y32.alloc(3 * KC * ys);
-  else Y64.alloc(3 * KC * ys);
   for (int64_t g0 = 0; g0 < ntri; g0 += group) {
     const int64_t ng = std::min(group, ntri - g0);
     for (int64_t c0 = g0; c0 < g0 + ng; c0 += KC) {
       const int64_t nc = std::min(KC, g0 + ng - c0);
-      const int4* tr = dtri.p + c0;
-      double* pt = part.p + (c0 - g0) * norb;
+      const int4* tr = dtri + c0;
+      double* pt = part + (c0 - g0) * norb;
       const unsigned eg = (unsigned)(norb * nc);
       if (x3) {
         X3Gemm g;   // C_(e, s)[m][n] = sum_kk [A | A2 swapped][m][kk] [B | B2][n][kk]
         g.M = vv; g.N = v; g.Kp = (2 * K1 + 31) / 32 * 32; g.K1 = K1; g.lda = 2 * Kp; g.ldb = 2 * Kp; g.ldc = ldy;
         g.kb = 32; g.ska = 64; g.skb = 64; g.sw = v; g.nbatch = 3 * nc; g.ytile = tiled ? v : 0;
-        g.sa = sc.p; g.sb = sc.p + 1; g.sA = vv * 2 * Kp; g.sB = v * 2 * Kp; g.sC = ys;
+        g.sa = sc; g.sb = sc + 1; g.sA = vv * 2 * Kp; g.sB = v * 2 * Kp; g.sC = ys;
         g.tri = tr; g.nocc = i1;
-        g.Ah = Ahl.p; g.Al = Ahl.p + 32; g.Bh = Bhl.p; g.Bl = Bhl.p + 32; g.C = Y32.p;
+        g.Ah = A; g.Al = (f16*)A + 32; g.Bh = B; g.Bl = (f16*)B + 32; g.C = (float*)Y;
         x3_gemm_kcat(g, s);
         if (tiled)
-          t3_orbit_energy_kernel<float, true><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y32.p, dorb.p, norb, F, nmo, t1,
-                                                                        PB.p, pt);
+          t3_orbit_energy_kernel<float, true><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, (const float*)Y, dorb, norb, F,
+                                                                        nmo, t1, PB, pt);
         else
-          t3_orbit_energy_kernel<float, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y32.p, dorb.p, norb, F, nmo, t1,
-                                                                         PB.p, pt);
+          t3_orbit_energy_kernel<float, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, (const float*)Y, dorb, norb, F,
+                                                                         nmo, t1, PB, pt);
       } else {
-        kcat64(Kcat64{v, Kp, ldy, i1, nc, A64.p, B64.p, Y64.p, tr}, s);
-        t3_orbit_energy_kernel<double, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, Y64.p, dorb.p, norb, F, nmo, t1,
-                                                                        PB.p, pt);
+        kcat64(Kcat64{v, Kp, ldy, i1, nc, (const double*)A, (const double*)B, (double*)Y, tr}, s);
+        t3_orbit_energy_kernel<double, false><<<eg, OT_THREADS, 0, s>>>(o, v, ldy, tr, (const double*)Y, dorb, norb, F,
+                                                                        nmo, t1, PB, pt);
       }
       CCX_HIP(hipGetLastError());
     }
-    t3_triple_sums_kernel<<<(unsigned)ng, 256, 0, s>>>(part.p, norb, dtri.p + g0, te + g0);
+    t3_triple_sums_kernel<<<(unsigned)ng, 256, 0, s>>>(part, norb, dtri + g0, te + g0);
     CCX_HIP(hipGetLastError());
   }
   t3_accumulate_kernel<<<1, 1024, 0, s>>>(te, i0, i1, accumulate, e_dev);
