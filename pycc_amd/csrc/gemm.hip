@@ -275,6 +275,34 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
     for (int j = 0; j < NBJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
   const int fr = lane >> 4, fc = lane & 15;
   const bool m_in = m0 + BM <= p.M, n_in = n0 + BN <= p.N;
+  // This wave's 16 x 16 blocks: rows r0 + 16 i, columns c0 + 16 j, i < ni, j < nj. A 64 x 64 tile computes only the
+  // blocks that hold outputs, and where a side has at most two of them the four waves share them out: an o-wide
+  // side (o = 9, 13) would otherwise spend 4 to 16 times its flops (Lambda at o=13 v=101: 2.26 to 2.11 ms).
+  int r0 = wm * WM, c0 = wn * WN, ni = NBI, nj = NBJ;
+  if constexpr (BM == 64 && BN == 64) {
+    const int rb = m_in ? 4 : (p.M - m0 + 15) >> 4, cb = n_in ? 4 : (p.N - n0 + 15) >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    if (rb <= 2 && cb > 2) {
+      r0 = 0;
+      c0 = 16 * w;
+      ni = rb;
+      nj = w < cb;
+    } else if (cb <= 2 && rb > 2) {
+      r0 = 16 * w;
+      c0 = 0;
+      ni = w < rb;
+      nj = cb;
+    } else if (rb <= 2) {
+      r0 = 16 * (w >> 1);
+      c0 = 16 * (w & 1);
+      ni = (w >> 1) < rb;
+      nj = (w & 1) < cb;
+    } else {
+      ni = min(2, rb - 2 * (w >> 1));
+      nj = min(2, cb - 2 * (w & 1));
+    }
+  }
+  const bool all = ni == NBI && nj == NBJ;
 
   if (kt < kt_end) {
     typename decltype(la)::Load va;
@@ -308,26 +336,27 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
     auto body = [&](int buf) {
       next();
       load();
-      // small wave tiles read the whole k-tile's fragments first; large ones have no registers for that, and more
-      // waves to fill the gaps
-      constexpr int KG = WM * WN <= 1024 ? BK : 8;
 #pragma unroll
-      for (int kg = 0; kg < BK; kg += KG) {
-        T a[KG / 8][2][NBI], b[KG / 8][2][NBJ];
-#pragma unroll
-        for (int g = 0; g < KG / 8; ++g) {
-          As[buf].frags(a[g], wm * WM, kg + 8 * g, fr, fc);
-          Bs[buf].frags(b[g], wn * WN, kg + 8 * g, fr, fc);
-        }
-        if (KG == BK) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int g = 0; g < KG / 8; ++g)
+      for (int kg = 0; kg < BK; kg += 8) {
+        T a[2][NBI], b[2][NBJ];
+        As[buf].frags(a, r0, kg, fr, fc);
+        Bs[buf].frags(b, c0, kg, fr, fc);
+        auto products = [&](int bi, int bj) {
 #pragma unroll
           for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < NBI; ++i)
+            for (int i = 0; i < bi; ++i)
 #pragma unroll
-              for (int j = 0; j < NBJ; ++j) acc[i][j] = mfma16(a[g][h][i], b[g][h][j], acc[i][j]);
+              for (int j = 0; j < bj; ++j) acc[i][j] = mfma16(a[h][i], b[h][j], acc[i][j]);
+        };
+        if constexpr (BM == 64 && BN == 64) {
+          if (all) products(NBI, NBJ);
+          else if (ni == 2 && nj == 1) products(2, 1);
+          else if (ni == 1 && nj == 2) products(1, 2);
+          else if (ni == 1 && nj == 1) products(1, 1);
+        } else {
+          products(NBI, NBJ);
+        }
       }
       la.store(va, As[buf ^ 1]);
       lb.store(vb, Bs[buf ^ 1]);
@@ -342,7 +371,7 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
   }
 
   // output row of register r within a 16x16 block (see the layout note at the top)
-  auto row = [&](int i, int r) { return m0 + wm * WM + i * 16 + (sizeof(T) == 8 ? 4 * r + fr : 4 * fr + r); };
+  auto row = [&](int i, int r) { return m0 + r0 + i * 16 + (sizeof(T) == 8 ? 4 * r + fr : 4 * fr + r); };
   if (p.splits == 1) {
     T* C = p.C + bidx * p.c_b;
 #pragma unroll
@@ -350,12 +379,12 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = row(i, r);
-        if (m >= p.M) continue;
+        if (i >= ni || m >= p.M) continue;
         T* Cm = C + off2(p.cm, (uint32_t)m);
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) {
-          const int n = n0 + wn * WN + j * 16 + fc;
-          if (n >= p.N) continue;
+          const int n = n0 + c0 + j * 16 + fc;
+          if (j >= nj || n >= p.N) continue;
           T* dst = Cm + off2(p.cn, (uint32_t)n);
           T v = p.alpha * acc[i][j][r];
           if (p.beta != T(0)) v += p.beta * *dst;
@@ -369,11 +398,11 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = row(i, r);
-        if (m >= p.M) continue;
+        if (i >= ni || m >= p.M) continue;
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) {
-          const int n = n0 + wn * WN + j * 16 + fc;
-          if (n < p.N) W[(int64_t)m * p.N + n] = acc[i][j][r];
+          const int n = n0 + c0 + j * 16 + fc;
+          if (j < nj && n < p.N) W[(int64_t)m * p.N + n] = acc[i][j][r];
         }
       }
   }
@@ -655,22 +684,26 @@ static bool as_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
 struct Plan {
   int tile = 128, splits = 1, chunk = 0;
 };
-static Plan plan_f64(const GemmParams<double>& p, size_t limit, int cus = 256, bool only64 = false) {
+// CU time of a contraction on 64 x 64 tiles, of which only the 16 x 16 blocks that hold outputs are computed
+static double tile64_us(const GemmParams<double>& p) {
+  const double blocks = (double)ceil_div(p.M, 16) * (double)ceil_div(p.N, 16) * (double)p.batch;
+  return blocks * (double)std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx) * (2.0 * 16 * 16 * 16 / 0.24e6);
+}
+static Plan plan_f64(const GemmParams<double>& p, size_t limit) {
   static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128, 192, 256};
   const int64_t ntk = std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx);
   Plan best;
   double t_best = 0.0;
   for (int tile : {128, 64}) {
-    if (only64 && tile != 64) continue;
     const int64_t tiles = ceil_div(p.M, tile) * ceil_div(p.N, tile) * p.batch;
-    const double t_ktile = 2.0 * tile * tile * 16 / 0.24e6;
+    const double t_ktile = tile == 64 ? tile64_us(p) / (double)(tiles * ntk) : 2.0 * tile * tile * 16 / 0.24e6;
     const int per_cu = tile == 128 ? 2 : 4;   // resident work-groups (LDS)
     for (int want : counts) {
       const int64_t chunk = ceil_div(ntk, want), splits = ceil_div(ntk, chunk);
       if (want > 1 && (chunk < 4 || splits * p.batch > 65535)) break;
       const double bytes = 8.0 * (double)splits * (double)p.batch * (double)p.M * (double)p.N;
       if (want > 1 && bytes > (double)limit) break;
-      const int64_t on_cu = ceil_div(tiles * splits, cus);
+      const int64_t on_cu = ceil_div(tiles * splits, 256);
       double t = 6.0 + (double)chunk * (0.25 * (double)ceil_div(on_cu, per_cu) + (double)on_cu * t_ktile);
       if (splits > 1) t += 5.0 + 2.0 * bytes / 4.0e6;
       if (t_best == 0.0 || t < t_best) {
@@ -713,15 +746,34 @@ static Plan plan_fixed(const GemmParams<T>& p, size_t limit) {
   return r;
 }
 static Plan plan(const GemmParams<float>& p, const Workspace& ws) { return plan_fixed(p, ws.limit); }
-static Plan plan(const GemmParams<double>& p, const Workspace& ws, int cus = 256, bool only64 = false) {
+// Splits of a member of a group whose work is `group_us` over the whole chip: chains of k-tiles of half that time (1.4
+// us a k-tile with two work-groups on the CU), so that the blocks of all members pack, but no shorter than 4 us, and
+// partial sums that move (4 TB/s) in a third of it. A 549 x 549 x 549 product among small ones then splits in 3:
+// 53 to 39 us for that launch (each member planned for an equal share of the chip left it unsplit).
+static Plan plan_member(const GemmParams<double>& p, size_t limit, double group_us) {
+  Plan r;
+  r.tile = 64;
+  const int64_t ntk = std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx);
+  const double one = 8.0 * (double)p.batch * (double)p.M * (double)p.N;
+  const double target = std::max(8.0, group_us);
+  const int64_t room = std::min<int64_t>((int64_t)((double)limit / one), 65535 / p.batch);
+  const int64_t cheap = (int64_t)(target / 3 * 4.0e6 / (2.0 * one));
+  int64_t splits = ceil_div(ntk, std::max<int64_t>(4, (int64_t)(target / 2.8)));
+  splits = std::max<int64_t>(1, std::min({splits, room, std::max<int64_t>(cheap, 1), (int64_t)256}));
+  r.chunk = (int)ceil_div(ntk, splits);
+  r.splits = (int)ceil_div(ntk, r.chunk);
+  return r;
+}
+// group_us: the work of the group that it is launched in, 0 for a launch of its own
+static Plan plan(const GemmParams<double>& p, const Workspace& ws, double group_us = 0.0) {
   if (ws.fixed_k) {
     Plan f = plan_fixed(p, ws.limit);
     if (f.splits <= FIXED_K_SPLITS) {   // the tile is free
-      if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch * f.splits < 512 || only64) f.tile = 64;
+      if (ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch * f.splits < 512 || group_us > 0) f.tile = 64;
       return f;
     }
   }
-  return plan_f64(p, ws.limit, cus, only64);
+  return group_us > 0 ? plan_member(p, ws.limit, group_us) : plan_f64(p, ws.limit);
 }
 
 // How a contraction is loaded: which operands are k-fast, lane offsets in 32 bits, pairs.
@@ -912,9 +964,9 @@ void GemmQueue::flush() {
       tc_gemm<double>(todo[at].p, ws, s);
       return;
     }
-    // planned for their share of the chip, the longest first
     const size_t left = std::min<size_t>(todo.size() - at, GROUP);
-    const int cus = std::max<int>(32, 256 / (int)left);
+    double work_us = 0.0;   // of the group, spread over the chip
+    for (size_t i = at; i < at + left; ++i) work_us += tile64_us(todo[i].p) / 256;
     struct Item {
       const Op* o;
       Plan pl;
@@ -923,7 +975,7 @@ void GemmQueue::flush() {
     size_t bytes = 0;
     for (; items.size() < left; ++at) {
       const GemmParams<double>& p = todo[at].p;
-      const Plan pl = plan(p, ws, cus, true);
+      const Plan pl = plan(p, ws, work_us);
       const size_t w = pl.splits > 1 ? (size_t)pl.splits * p.batch * p.M * p.N * sizeof(double) : 0;
       if (!items.empty() && bytes + w > ws.limit) break;
       bytes += w;
