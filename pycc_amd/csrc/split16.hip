@@ -1139,7 +1139,9 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
   const bool direct = p.cn.s2 == 1 && p.cn.n2 >= N && p.cm.n2 >= M && p.cm.s2 >= N && tiles >= 512 &&
                       (double)(float)p.beta == p.beta;   // the epilogue applies beta in FP32
   auto r256 = [](int64_t b) { return (b + 255) / 256 * 256; };
-  constexpr int PB = 256;   // partial maxima per operand (a 16 x 16 grid of the absmax pass)
+  // The largest-magnitude pass takes up to 64 x 64 work-groups: it is bound by its loads, one 64 x 64 tile's in
+  // flight per work-group (8192 x 8192, 537 MB: 530 us with 16 x 16 of them).
+  constexpr int PB = 4096;   // partial maxima per operand
   const int64_t bA = r256(M * 2 * Kp * 2), bB = r256(N * 2 * Kp * 2), bC = direct ? 0 : r256(M * N * 4);
   char* base = (char*)ws.get((size_t)(bA + bB + bC + 2 * PB * 4 + 256));
   f16* Ahl = (f16*)base;
@@ -1147,12 +1149,12 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
   float* S = (float*)(base + bA + bB);
   float* part = (float*)(base + bA + bB + bC);
   float* sc = part + 2 * PB;   // sc[0] scale of A, sc[1] scale of B
-  const dim3 gmax(16, 16);
   auto split = [&](const double* src, int64_t R, Idx2 dr, Idx2 dk, float* pmax, float* scl, f16* hl) {
     const bool rfast = dr.s2 == 1 && dk.s2 != 1;
+    const dim3 gmax((unsigned)std::min<int64_t>(ceil_div(Kp, 64), 64), (unsigned)std::min<int64_t>(ceil_div(R, 64), 64));
     view_split_kernel<<<gmax, 256, 0, s>>>(src, R, K, Kp, dr, dk, rfast, nullptr, pmax, nullptr);
     CCX_HIP(hipGetLastError());
-    x3_scale_kernel<<<1, 256, 0, s>>>(pmax, PB, 1.f, pmax, 0, 0.f, scl);
+    x3_scale_kernel<<<1, 256, 0, s>>>(pmax, (int)(gmax.x * gmax.y), 1.f, pmax, 0, 0.f, scl);
     CCX_HIP(hipGetLastError());
     const dim3 g((unsigned)std::min<int64_t>(ceil_div(Kp, 64), 1024), (unsigned)std::min<int64_t>(ceil_div(R, 64), 65535));
     view_split_kernel<<<g, 256, 0, s>>>(src, R, K, Kp, dr, dk, rfast, scl, nullptr, hl);
