@@ -71,20 +71,23 @@ struct PLoader {
   static constexpr int SEGS = KC ? BK / VEC : R / VEC;  // vectors per stored row
   uint4 v[NV];
   int row[NV], seg[NV];                                 // stored-row index and vector index
+  int from[NV];                                         // the row that load_fast reads into it
 
-  __device__ __forceinline__ void init(int tid) {
+  // nrows: valid rows; a k-contiguous tile's rows past them read the last one (their results are not stored)
+  __device__ __forceinline__ void init(int tid, int64_t nrows) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       int q = tid + 256 * i;
       row[i] = q / SEGS;
       seg[i] = q % SEGS;
+      from[i] = KC && row[i] >= nrows ? (int)nrows - 1 : row[i];
     }
   }
   // base points at the tile origin (row 0, k = k0); ld = leading dimension in elements
   __device__ __forceinline__ void load_fast(const T* __restrict__ base, int64_t ld) {
 #pragma unroll
     for (int i = 0; i < NV; ++i)
-      v[i] = *(const uint4*)(base + (int64_t)row[i] * ld + seg[i] * VEC);
+      v[i] = *(const uint4*)(base + (int64_t)from[i] * ld + seg[i] * VEC);
   }
   // guarded: rows beyond nrows / k beyond nk are zero (nrows, nk relative to the tile origin)
   __device__ __forceinline__ void load_safe(const T* __restrict__ base, int64_t ld, int64_t nrows, int64_t nk) {
@@ -142,24 +145,29 @@ __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(Plai
   auto a_at = [&](int64_t k) { return A_KC ? A + m0 * p.lda + k : A + k * p.lda + m0; };
   auto b_at = [&](int64_t k) { return B_NC ? B + k * p.ldb + n0 : B + n0 * p.ldb + k; };
   const int64_t a_rows = p.M - m0, b_rows = p.N - n0;   // valid tile rows (m / n)
-  const bool interior = a_rows >= BM && b_rows >= BN;
+  // every load of a whole k-tile is a vector inside the operand
+  const bool inside = (a_rows >= BM || A_KC) && (b_rows >= BN || !B_NC);
+  // 16-row blocks of this wave that hold outputs
+  const int wrows = (int)(a_rows < BM ? a_rows : BM) - wm * WM;
+  const int nbi = __builtin_amdgcn_readfirstlane(wrows <= 0 ? 0 : wrows >= WM ? NBI : (wrows + 15) / 16);
 
   PLoader<T, BM, BK, A_KC> la;
   PLoader<T, BN, BK, !B_NC> lb;
-  la.init(tid);
-  lb.init(tid);
+  la.init(tid, a_rows);
+  lb.init(tid, b_rows);
   acc_t acc[NBI][NBJ];
 #pragma unroll
   for (int i = 0; i < NBI; ++i)
 #pragma unroll
     for (int j = 0; j < NBJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
-  // The k loop, compiled twice: FAST (an interior tile and K a multiple of BK, so every load is a
-  // full in-bounds vector) and checked. Keeping the checked loads out of the FAST loop lets the
+  // The k loop, compiled three times: FAST (K a multiple of BK, every load a full in-bounds vector), with all
+  // of the tile's rows or (!WHOLE) only the 16-row blocks that hold outputs, and checked. A ladder of 528 pair
+  // rows ends in a tile of 16: with checked loads and all products it cost as much as two whole ones. Keeping the checked loads out of the FAST loop lets the
   // prefetch of tile k + 1 stay in flight while tile k is multiplied (a shared loop forces a full
   // wait on the loads at the join of the two load paths).
-  auto kloop = [&](auto fast_tag) {
-    constexpr bool FAST = decltype(fast_tag)::value;
+  auto kloop = [&](auto fast_tag, auto whole_tag) {
+    constexpr bool FAST = decltype(fast_tag)::value, WHOLE = decltype(whole_tag)::value;
     auto load = [&](int64_t k0) {
       const int64_t nk = Kb - k0;
       if constexpr (FAST) {
@@ -188,9 +196,11 @@ __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(Plai
         for (int j = 0; j < NBJ; ++j)
           b[j] = B_NC ? Bs[buf].d[ks + fr][wn * WN + j * 16 + fc] : Bs[buf].d[wn * WN + j * 16 + fc][ks + fr];
 #pragma unroll
-        for (int i = 0; i < NBI; ++i)
+        for (int i = 0; i < NBI; ++i) {
+          if (!WHOLE && i >= nbi) break;
 #pragma unroll
           for (int j = 0; j < NBJ; ++j) acc[i][j] = pmfma(a[i], b[j], acc[i][j]);
+        }
       }
       if (has_next) {
         la.store(As[buf ^ 1]);
@@ -201,8 +211,9 @@ __global__ __launch_bounds__(256, BT == 128 ? 2 : 1) void plain_gemm_kernel(Plai
     }
   };
   if (Kb > 0) {
-    if (interior && Kb % BK == 0) kloop(std::true_type{});
-    else kloop(std::false_type{});
+    if (inside && Kb % BK == 0 && a_rows >= BM) kloop(std::true_type{}, std::true_type{});
+    else if (inside && Kb % BK == 0) kloop(std::true_type{}, std::false_type{});
+    else kloop(std::false_type{}, std::true_type{});
   }
 
 #pragma unroll
