@@ -56,7 +56,7 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t w, int64_t ntiles) {
 // one to issue: 8 waves of 64 x 32 per 128 x 128 work-group, two work-groups per CU (4 waves per SIMD, 128 registers).
 // Measured at 8192^3: 59-62 TF; 70-74 TF with the global loads and LDS writes left out, each of which costs the
 // matrix cores about 10% however early it is issued (a third LDS stage, two k-tiles in flight and 32-wide k-tiles
-// changed nothing), so loads and LDS writes are 16 bytes wherever pairs are contiguous (57 TF with 8-byte ones). Addresses
+// changed nothing), so loads and LDS writes are pairs wherever those are contiguous (57 TF with 8-byte ones). Addresses
 // come from an odometer per k-tile, so any strides, odd extents and remainders run the same loop: 2793^3 with odd
 // leading dimensions takes 0.76 ms (0.99 with guarded 8-byte loads). Rows past M or N read row M - 1 or N - 1
 // (their outputs are not stored); k past its end reads a valid k and is zeroed on its way into LDS.
@@ -98,12 +98,13 @@ struct TileGemm {
   T* work;   // [split][batch][M][N] partial sums when splits > 1
 };
 
-// two doubles in LDS
-struct alignas(16) Two {
-  double x, y;
+// two neighbouring elements, aligned as one: read from memory by one load, written to LDS by one instruction
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) Two {
+  T x, y;
 };
-// two neighbouring doubles in memory: 8-byte aligned, read by one 16-byte load
-struct __attribute__((packed, aligned(8))) TwoIn {
+// a pair of doubles in LDS, where rows are 16-byte aligned
+struct alignas(16) Two16 {
   double x, y;
 };
 
@@ -128,7 +129,7 @@ struct GTile {
 // offset in bytes (Off: 32 bits where the operand spans less than 4 GiB), k by an odometer over its (n2, s1, s2):
 // a k-tile costs a lane one step of it and an add per load. Where a whole wave holds one k (row-fast, V R >= 64
 // lanes) that k stays in scalar registers.
-// V = 2 reads 16 bytes at a time. It needs the inner index contiguous and pairs that do not straddle its blocks: an
+// V = 2 reads two elements at a time. It needs the inner index contiguous and pairs that do not straddle its blocks: an
 // even n2 or a single level. An odd extent ends in a pair that starts one early (`late`: its second half counts).
 template <typename T, int R, int BK, bool KF, int NT, typename Off, int V>
 struct GLoader {
@@ -186,7 +187,7 @@ struct GLoader {
   }
   static __device__ __forceinline__ void get(T (&v)[V], const char* p) {
     if constexpr (V == 2) {
-      const TwoIn q = *(const TwoIn*)p;
+      const Two<T> q = *(const Two<T>*)p;
       v[0] = q.x;
       v[1] = q.y;
     } else {
@@ -219,7 +220,8 @@ struct GLoader {
   }
   __device__ __forceinline__ void put(const T (&x)[V], int i, GTile<T, R, BK, KF>& t) {
     T* dst = KF ? &t.at(rl + i * STEP, kl) : &t.at(rl, kl + i * STEP);
-    if constexpr (V == 2) *(Two*)dst = Two{x[0], x[1]};
+    if constexpr (V == 2 && sizeof(T) == 8) *(Two16*)dst = Two16{x[0], x[1]};
+    else if constexpr (V == 2) *(Two<T>*)dst = Two<T>{x[0], x[1]};
     else *dst = x[0];
   }
   __device__ __forceinline__ void store(const Load& l, GTile<T, R, BK, KF>& t) {
@@ -745,7 +747,13 @@ static Plan plan_fixed(const GemmParams<T>& p, size_t limit) {
   r.chunk = (int)kchunk;
   return r;
 }
-static Plan plan(const GemmParams<float>& p, const Workspace& ws) { return plan_fixed(p, ws.limit); }
+static Plan plan(const GemmParams<float>& p, const Workspace& ws) {
+  Plan f = plan_fixed(p, ws.limit);
+  // the tile is free: 128 x 128 reach 100 TF of padded work at 2793^3, 64 x 64 93, so these where they pad 7% less (190
+  // x 13671 x 10878: 862 to 615 us; 549^3: 22 to 17)
+  if (f.tile == 128 && 25 * ceil_div(p.M, 64) * ceil_div(p.N, 64) < 93 * ceil_div(p.M, 128) * ceil_div(p.N, 128)) f.tile = 64;
+  return f;
+}
 // Splits of a member of a group whose work is `group_us` over the whole chip: chains of k-tiles of half that time (1.4
 // us a k-tile with two work-groups on the CU), so that the blocks of all members pack, but no shorter than 4 us, and
 // partial sums that move (4 TB/s) in a third of it. A 549 x 549 x 549 product among small ones then splits in 3:
@@ -796,7 +804,7 @@ static Form form_of(const GemmParams<T>& p, int tile) {
   f.off32 = narrow(p.am, p.M, p.ak, f.akf) && narrow(p.bn, p.N, p.bk, f.bkf);
   // pairs along the contiguous index of both operands
   auto pairs = [](const Idx2& d, int64_t n) { return d.s2 == 1 && n >= 2 && (d.n2 % 2 == 0 || n <= d.n2); };
-  f.two = sizeof(T) == 8 && f.off32 &&
+  f.two = f.off32 &&
           (tile == 128 || (narrow(p.am, p.M, p.ak, true) && narrow(p.bn, p.N, p.bk, true))) &&
           pairs(f.akf ? p.ak : p.am, f.akf ? p.K : p.M) && pairs(f.bkf ? p.bk : p.bn, f.bkf ? p.K : p.N);
   return f;
@@ -858,14 +866,9 @@ void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
   if (std::getenv("CCX_TRACE"))
     std::fprintf(stderr, "[ccx]   -> tile %d%s%s batch %lld splits %d\n", pl.tile, f.akf ? " Ak" : " Am",
                  f.bkf ? " Bk" : " Bn", (long long)p.batch, pl.splits);
-  if constexpr (sizeof(T) == 8) {
-    if (f.two) launch_tile<T, uint32_t, 2>(pl.tile, g, p.batch, f.akf, f.bkf, s);
-    else if (f.off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
-    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
-  } else {
-    if (f.off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
-    else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
-  }
+  if (f.two) launch_tile<T, uint32_t, 2>(pl.tile, g, p.batch, f.akf, f.bkf, s);
+  else if (f.off32) launch_tile<T, uint32_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
+  else launch_tile<T, int64_t, 1>(pl.tile, g, p.batch, f.akf, f.bkf, s);
   if (pl.splits > 1) splitk_reduce<T>(p, g.work, pl.splits, s);
 }
 
