@@ -75,3 +75,19 @@ def test_rows_more_than_4_gib_apart(contract):
     for sub, B in (("ak,kb->ab", b), ("ak,bk->ab", b.t().contiguous())):
         out = contract(sub, A, B.cuda()).cpu()
         assert float((out - a @ b).abs().max()) <= 2 * (k + 4) * 2.2e-16 * float((a.abs() @ b.abs()).max())
+
+
+# every count of 16-row and 16-column blocks that a 64 x 64 tile can hold, alone and after a whole tile
+@pytest.mark.parametrize("m", [7, 17, 40, 64, 78, 91, 107])
+@pytest.mark.parametrize("n", [13, 30, 45, 61, 80, 100, 115])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_blocks_of_a_tile(contract, m, n, dtype):
+    _check(contract, "ak,kb->ab", {"a": m, "b": n, "k": 53}, dtype, beta=0.5)
+
+
+# aligned matrices of many tiles whose last tile row is short
+@pytest.mark.parametrize("sub", ["ak,kb->ab", "ak,bk->ab", "ka,kb->ab"])
+@pytest.mark.parametrize("m", [514, 528, 612, 640])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_short_last_tile_row(contract, sub, m, dtype):
+    _check(contract, sub, {"a": m, "b": 8192, "k": 64}, dtype, beta=0.5)
