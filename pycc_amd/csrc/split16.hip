@@ -407,6 +407,12 @@ __device__ __forceinline__ void x3_dma16(const E* g, const E* lds) {
 // BN / 16 row blocks of 16 go to wave q % 8); BT = 256 or 384 rows. KCAT: the K-concatenated, batched form of
 // x3_gemm_kcat (interleaved operands, FP32 C, no split K).
 // WGM: waves along M (2: 2 x 4 waves; 8: 8 x 1, the waves of the KCAT tiles of 384 x BN, 48 x BN each).
+// A last tile row of at most BT / 2 rows (not KCAT) loads and computes only the 16-row blocks that hold outputs, shared
+// out over the waves along M, and its tiles are dispatched last, into the CUs that the last round of whole tiles leaves:
+// the packed ladder of 32 occupied orbitals has 528 pair rows, 528 x 32896 x 32896 4.90 to 4.23 ms (a tile of 16 rows
+// still takes 1.75 ms, a load latency per k-tile, against 2.45 for a whole one; its operands straight from global
+// memory into registers, two k-tiles ahead: 4.86). The wave index is scalar: 8 registers fewer ((T) at o=24 v=176 180.2
+// to 174.7 ms).
 template <typename E, int BN, bool KCAT = false, int BT = 256, bool YT = false, int WGM = 2>
 __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   typedef typename X3<E>::v8 v8;
@@ -415,10 +421,13 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   constexpr int NIB = BN / 16, IPB = (NIB + 7) / 8;   // B row blocks, per wave (rounded up)
   __shared__ __attribute__((aligned(1024))) E sA[2][2][BT * 32];   // [stage][hi/lo]
   __shared__ __attribute__((aligned(1024))) E sB[2][2][BN * 32];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   const int64_t tiles_m = (p.M + BT - 1) / BT, tiles_n = (p.N + BN - 1) / BN;
-  int64_t t = xcd_remap_x3(blockIdx.x, tiles_m * tiles_n * (KCAT ? p.nbatch : 1));
+  const int last_rows = (int)(p.M - (tiles_m - 1) * BT);
+  const int64_t whole = !KCAT && last_rows <= BT / 2 ? tiles_m - 1 : tiles_m;   // tile rows that come first
+  const bool brief = !KCAT && blockIdx.x >= whole * tiles_n;                    // a tile of the short last row
+  int64_t t = brief ? 0 : xcd_remap_x3(blockIdx.x, whole * tiles_n * (KCAT ? p.nbatch : 1));
   int64_t batch = 0, tm, tn;
   if constexpr (KCAT) kcat_tile(t, tiles_m, tiles_n, batch, tm, tn);
   const E* __restrict__ Ah = (const E*)p.Ah;
@@ -439,11 +448,12 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   const int64_t split = blockIdx.y;
   if constexpr (!KCAT) {
     const int64_t group = t / (GM * tiles_n), first_m = group * GM;
-    const int64_t gsize = tiles_m - first_m < GM ? tiles_m - first_m : GM;
+    const int64_t gsize = whole - first_m < GM ? whole - first_m : GM;
     const int64_t within = t - group * GM * tiles_n;
-    tm = first_m + within % gsize;
-    tn = within / gsize;
+    tm = brief ? whole : first_m + within % gsize;
+    tn = brief ? blockIdx.x - whole * tiles_n : within / gsize;
   }
+  const int blocks = brief ? (last_rows + 15) >> 4 : BT / 16;   // 16-row blocks of A that are loaded
 
   int64_t gA[IPW], gB[IPB];
   // KCAT: offsets in the second blocks, so that 16-byte chunk g = 4 q + c of the concatenated K (q the
@@ -475,7 +485,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     if constexpr (KCAT) gB2[i] = (int)(n * p.ldb) + chunk2(c);
     ldsb[i] = R0 * 32;
   }
-  auto issue = [&](int st, int64_t k0) {
+  auto issue = [&](int st, int64_t k0, auto short_row) {
     int64_t ka = k0, kb = k0;
     if (p.kb == BK) {   // interleaved operands and other 32-blocked layouts
       ka = (k0 >> 5) * p.ska;
@@ -512,6 +522,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     } else {
 #pragma unroll
       for (int i = 0; i < IPW; ++i) {
+        if (decltype(short_row)::value && wave * IPW + i >= blocks) continue;   // wave-uniform
         x3_dma16<E>(Ah + gA[i] + ka, &sA[st][0][ldso[i]]);
         x3_dma16<E>(Al + gA[i] + ka, &sA[st][1][ldso[i]]);
       }
@@ -525,9 +536,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     }
   };
   const int fr = lane >> 4, fc = lane & 15;
-  int ra[NBM], rb[NBN];
-#pragma unroll
-  for (int i = 0; i < NBM; ++i) ra[i] = x3_swz(wm * WTM + i * 16 + fc, fr);
+  int rb[NBN];
 #pragma unroll
   for (int j = 0; j < NBN; ++j) rb[j] = x3_swz(wn * WTN + j * 16 + fc, fr);
   f4 acc[NBM][NBN];
@@ -538,37 +547,56 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
 
   const int64_t kbeg = p.work ? split * p.kchunk : 0;
   const int64_t kend = p.work ? (kbeg + p.kchunk < p.Kp ? kbeg + p.kchunk : p.Kp) : p.Kp;
-  issue(0, kbeg);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  int buf = 0;
-  for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
-    if (k0 + BK < kend) issue(buf ^ 1, k0 + BK);
-    v8 a[NBM], b[NBN];
-    // lo(A) x hi(B), hi(A) x hi(B), hi(A) x lo(B)
+  // this wave's rows: NI blocks of 16 from wm 16 NI
+  int wrow = wm * WTM, ni = NBM;
+  auto run = [&](auto nblocks, auto short_row) {
+    constexpr int NI = decltype(nblocks)::value;
+    int ra[NI];
 #pragma unroll
-    for (int i = 0; i < NBM; ++i) a[i] = *(const v8*)&sA[buf][1][ra[i]];
+    for (int i = 0; i < NI; ++i) ra[i] = x3_swz(wm * 16 * NI + i * 16 + fc, fr);
+    issue(0, kbeg, short_row);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
+      if (k0 + BK < kend) issue(buf ^ 1, k0 + BK, short_row);
+      v8 a[NI], b[NBN];
+      // lo(A) x hi(B), hi(A) x hi(B), hi(A) x lo(B)
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) b[j] = *(const v8*)&sB[buf][0][rb[j]];
+      for (int i = 0; i < NI; ++i) a[i] = *(const v8*)&sA[buf][1][ra[i]];
 #pragma unroll
-    for (int i = 0; i < NBM; ++i)
+      for (int j = 0; j < NBN; ++j) b[j] = *(const v8*)&sB[buf][0][rb[j]];
 #pragma unroll
-      for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int i = 0; i < NBM; ++i) a[i] = *(const v8*)&sA[buf][0][ra[i]];
+        for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
 #pragma unroll
-    for (int i = 0; i < NBM; ++i)
+      for (int i = 0; i < NI; ++i) a[i] = *(const v8*)&sA[buf][0][ra[i]];
 #pragma unroll
-      for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) b[j] = *(const v8*)&sB[buf][1][rb[j]];
+        for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
 #pragma unroll
-    for (int i = 0; i < NBM; ++i)
+      for (int j = 0; j < NBN; ++j) b[j] = *(const v8*)&sB[buf][1][rb[j]];
 #pragma unroll
-      for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's loads of the next k-tile
-    __syncthreads();                                    // everyone's loads landed, reads of buf done
-    buf ^= 1;
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) acc[i][j] = X3<E>::mfma(a[i], b[j], acc[i][j]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's loads of the next k-tile
+      __syncthreads();                                    // everyone's loads landed, reads of buf done
+      buf ^= 1;
+    }
+  };
+  typedef std::integral_constant<int, NBM> whole_tile;
+  if constexpr (KCAT) {
+    run(whole_tile{}, std::false_type{});
+  } else if (brief) {   // uniform in the work-group
+    ni = blocks <= WGM ? 1 : NBM / 2;
+    wrow = wm * 16 * ni;
+    if (ni == 1) run(std::integral_constant<int, 1>{}, std::true_type{});
+    else run(std::integral_constant<int, NBM / 2>{}, std::true_type{});
+  } else {
+    run(whole_tile{}, std::false_type{});
   }
 
   if (p.work) {   // split-K: raw partial sums
@@ -581,8 +609,8 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
       for (int i = 0; i < NBM; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int64_t m = tm * BT + wm * WTM + i * 16 + fr * 4 + r;
-          if (m < p.M) Wb[m * p.N + n] = acc[i][j][r];
+          const int64_t m = tm * BT + wrow + i * 16 + fr * 4 + r;
+          if (i < ni && m < p.M) Wb[m * p.N + n] = acc[i][j][r];
         }
     }
     return;
@@ -624,8 +652,8 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     for (int i = 0; i < NBM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t m = tm * BT + wm * WTM + i * 16 + fr * 4 + r;
-        if (m < p.M) {
+        const int64_t m = tm * BT + wrow + i * 16 + fr * 4 + r;
+        if (i < ni && m < p.M) {
           if (p.C64) {   // FP64 destination without split K
             const int64_t at = m * p.ldc + n;
             double val = (double)(f * acc[i][j][r]);
