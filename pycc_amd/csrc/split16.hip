@@ -1149,6 +1149,60 @@ __global__ __launch_bounds__(256) void scatter_add_kernel(const float* __restric
   }
 }
 
+// scatter_add_kernel where C runs along another index than S: S[f sf + n + q0 s0 + q1 s1] to C[f + n cn + q0 c0 + q1 c1],
+// in 64 x 64 (n, f) tiles through LDS, so that S is read along n and C is read and written along f.
+// Bound by HBM: 67 M elements (1024 x 65536, n outer contiguous in C) of the Lambda residual at o=32 v=256 take 258 us, 1936
+// in scatter_add_kernel, whose lanes then touch a line of C each.
+struct ScatterT {
+  int64_t nf, nn, n0, n1;   // extents of f, n, q0, q1
+  int64_t sf, s0, s1, cn, c0, c1;
+};
+__global__ __launch_bounds__(256) void scatter_add_t_kernel(const float* __restrict__ S, ScatterT d, double beta,
+                                                            double* __restrict__ C) {
+  __shared__ float tile[64][65];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t n0 = blockIdx.x * (int64_t)64, f0 = blockIdx.y * (int64_t)64;
+  for (int64_t q = blockIdx.z; q < d.n0 * d.n1; q += gridDim.z) {
+    const int64_t q0 = q / d.n1, q1 = q - q0 * d.n1;
+    const float* Sq = S + q0 * d.s0 + q1 * d.s1;
+    double* Cq = C + q0 * d.c0 + q1 * d.c1;
+    __syncthreads();   // the previous tile is no longer read
+    for (int j = ty; j < 64; j += 4)
+      if (f0 + j < d.nf && n0 + tx < d.nn) tile[j][tx] = Sq[(f0 + j) * d.sf + n0 + tx];
+    __syncthreads();
+    for (int j = ty; j < 64; j += 4)
+      if (f0 + tx < d.nf && n0 + j < d.nn) {
+        double* c = Cq + (n0 + j) * d.cn + f0 + tx;
+        const double val = (double)tile[tx][j];
+        *c = beta == 0.0 ? val : beta * *c + val;
+      }
+  }
+}
+
+void scatter_add(const float* S, int64_t M, int64_t N, const Idx2& cm, const Idx2& cn, double beta, double* C,
+                 hipStream_t s) {
+  // C's four indices (m outer, m inner, n outer, n inner) with their strides in S and in C
+  struct Dim {
+    int64_t ext, ss, sc;
+  };
+  const int64_t m2 = std::min(cm.n2, M), n2 = std::min(cn.n2, N);
+  const Dim d[4] = {{M / m2, m2 * N, cm.s1}, {m2, N, cm.s2}, {N / n2, n2, cn.s1}, {n2, 1, cn.s2}};
+  // The transposed form where C's contiguous index is not S's and both are wide enough to fill most of a tile's rows
+  int f = -1;
+  for (int i = 0; i < 3; ++i)
+    if (d[i].ext >= 32 && d[i].sc == 1) f = i;
+  if (f >= 0 && cn.s2 != 1 && n2 >= 32 && M % m2 == 0 && N % n2 == 0 && ceil_div(d[f].ext, 64) < 65536) {
+    const Dim &a = d[f == 0 ? 1 : 0], &b = d[f == 2 ? 1 : 2];
+    const ScatterT t{d[f].ext, n2, a.ext, b.ext, d[f].ss, a.ss, b.ss, cn.s2, a.sc, b.sc};
+    const dim3 g((unsigned)ceil_div(n2, 64), (unsigned)ceil_div(t.nf, 64), (unsigned)std::min<int64_t>(a.ext * b.ext, 65535));
+    scatter_add_t_kernel<<<g, 256, 0, s>>>(S, t, beta, C);
+  } else {
+    const dim3 g((unsigned)std::min<int64_t>(ceil_div(N, 256), 64), (unsigned)std::min<int64_t>(M, 65535));
+    scatter_add_kernel<<<g, 256, 0, s>>>(S, M, N, cm, cn, beta, C);
+  }
+  CCX_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
@@ -1201,9 +1255,7 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
   } else {
     g.C = S; g.ldc = N; g.beta = 0.f;
     x3_gemm<_Float16>(g, s);
-    const dim3 gs((unsigned)std::min<int64_t>(ceil_div(N, 256), 64), (unsigned)std::min<int64_t>(M, 65535));
-    scatter_add_kernel<<<gs, 256, 0, s>>>(S, M, N, p.cm, p.cn, p.beta, p.C);
-    CCX_HIP(hipGetLastError());
+    scatter_add(S, M, N, p.cm, p.cn, p.beta, p.C, s);
   }
   return true;
 }
