@@ -13,8 +13,10 @@
 //              row = 4 * r + (l / 16)   for v_mfma_f64_16x16x4f64
 #include "common.h"
 #include "gemm.h"
+#include "tile_blocks.h"
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 namespace ccx {
 
@@ -277,32 +279,15 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
     for (int j = 0; j < NBJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
   const int fr = lane >> 4, fc = lane & 15;
   const bool m_in = m0 + BM <= p.M, n_in = n0 + BN <= p.N;
-  // This wave's 16 x 16 blocks: rows r0 + 16 i, columns c0 + 16 j, i < ni, j < nj. A 64 x 64 tile computes only the
-  // blocks that hold outputs, and where a side has at most two of them the four waves share them out: an o-wide
-  // side (o = 9, 13) would otherwise spend 4 to 16 times its flops (Lambda at o=13 v=101: 2.26 to 2.11 ms).
+  // This wave's 16 x 16 blocks: rows r0 + 16 i, columns c0 + 16 j, i < ni, j < nj
   int r0 = wm * WM, c0 = wn * WN, ni = NBI, nj = NBJ;
   if constexpr (BM == 64 && BN == 64) {
-    const int rb = m_in ? 4 : (p.M - m0 + 15) >> 4, cb = n_in ? 4 : (p.N - n0 + 15) >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(wave);
-    if (rb <= 2 && cb > 2) {
-      r0 = 0;
-      c0 = 16 * w;
-      ni = rb;
-      nj = w < cb;
-    } else if (cb <= 2 && rb > 2) {
-      r0 = 16 * w;
-      c0 = 0;
-      ni = w < rb;
-      nj = cb;
-    } else if (rb <= 2) {
-      r0 = 16 * (w >> 1);
-      c0 = 16 * (w & 1);
-      ni = (w >> 1) < rb;
-      nj = (w & 1) < cb;
-    } else {
-      ni = min(2, rb - 2 * (w >> 1));
-      nj = min(2, cb - 2 * (w & 1));
-    }
+    const WaveBlocks b = wave_blocks(m_in ? 4 : (p.M - m0 + 15) >> 4, n_in ? 4 : (p.N - n0 + 15) >> 4,
+                                     __builtin_amdgcn_readfirstlane(wave));
+    r0 = b.r0;
+    c0 = b.c0;
+    ni = b.ni;
+    nj = b.nj;
   }
   const bool all = ni == NBI && nj == NBJ;
 
@@ -340,24 +325,28 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
       load();
 #pragma unroll
       for (int kg = 0; kg < BK; kg += 8) {
-        T a[2][NBI], b[2][NBJ];
-        As[buf].frags(a, r0, kg, fr, fc);
-        Bs[buf].frags(b, c0, kg, fr, fc);
-        auto products = [&](int bi, int bj) {
+        // BI x BJ blocks: only rows that the wave owns are read (r0 and c0 go up to 48, so that a second block's rows
+        // may lie past the tile, in the buffer that is being written or past the work-group's LDS)
+        auto products = [&](auto bi, auto bj) {
+          constexpr int BI = decltype(bi)::value, BJ = decltype(bj)::value;
+          T a[2][BI], b[2][BJ];
+          As[buf].frags(a, r0, kg, fr, fc);
+          Bs[buf].frags(b, c0, kg, fr, fc);
 #pragma unroll
           for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < bi; ++i)
+            for (int i = 0; i < BI; ++i)
 #pragma unroll
-              for (int j = 0; j < bj; ++j) acc[i][j] = mfma16(a[h][i], b[h][j], acc[i][j]);
+              for (int j = 0; j < BJ; ++j) acc[i][j] = mfma16(a[h][i], b[h][j], acc[i][j]);
         };
+        constexpr std::integral_constant<int, 1> one{};
         if constexpr (BM == 64 && BN == 64) {
-          if (all) products(NBI, NBJ);
-          else if (ni == 2 && nj == 1) products(2, 1);
-          else if (ni == 1 && nj == 2) products(1, 2);
-          else if (ni == 1 && nj == 1) products(1, 1);
+          if (all) products(std::integral_constant<int, NBI>{}, std::integral_constant<int, NBJ>{});
+          else if (ni == 2 && nj == 1) products(std::integral_constant<int, 2>{}, one);
+          else if (ni == 1 && nj == 2) products(one, std::integral_constant<int, 2>{});
+          else if (ni == 1 && nj == 1) products(one, one);
         } else {
-          products(NBI, NBJ);
+          products(std::integral_constant<int, NBI>{}, std::integral_constant<int, NBJ>{});
         }
       }
       la.store(va, As[buf ^ 1]);
