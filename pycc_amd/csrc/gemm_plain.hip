@@ -262,11 +262,15 @@ void launch_plain(const PlainGemm<T>& p, hipStream_t s) {
 
 typedef double d2p __attribute__((ext_vector_type(2)));
 
-// 16 bytes per lane from global memory into LDS at lds + 16 lane, no register in between
+// 16 bytes per lane from global memory into LDS at lds + 16 lane, no register in between. The load takes the LDS address
+// from m0, which it sees one wait state after a scalar write: the s_nop is that state, which the compiler cannot add here.
 __device__ __forceinline__ void dma16(const double* g, const double* lds) {
   const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const double*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory");
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved, named all the same
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory", "m0");
+#pragma clang diagnostic pop
 }
 
 // The (T) products (kcat64): 128 x 16 NBJ tiles, 4 waves of 32 rows by all 16 NBJ columns. A stage is

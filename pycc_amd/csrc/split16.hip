@@ -393,14 +393,18 @@ __global__ __launch_bounds__(256) void x3_skinny_kernel(X3Gemm p) {
 // chunk c ^ ((r >> 1) & 3), which keeps both the DMA writes and the fragment reads free of bank
 // conflicts. An LDS-DMA instruction writes 16 bytes per lane at M0 + 16 lane, so lane l of an
 // instruction covering rows R0 .. R0 + 15 loads row R0 + l / 4, chunk (l % 4) ^ ((row >> 1) & 3).
-// Rows past M / N load a valid row (their results are not stored).
+// Rows past M / N load a valid row (their results are not stored). The load sees m0 one wait state after its scalar
+// write: the s_nop, which the compiler cannot add inside an asm block.
 __device__ __forceinline__ int x3_swz(int r, int c) { return r * 32 + ((c ^ ((r >> 1) & 3)) * 8); }
 
 template <typename E>
 __device__ __forceinline__ void x3_dma16(const E* g, const E* lds) {
   const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const E*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory");
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is reserved, named all the same
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g) : "memory", "m0");
+#pragma clang diagnostic pop
 }
 
 // BN = 16 n up to 256, or 320, output columns per tile (320: 128 x 80 per wave, 144 KiB of LDS; B's
