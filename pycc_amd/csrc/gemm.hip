@@ -835,8 +835,22 @@ static void check_extents(const GemmParams<T>& p) {
   CCX_CHECK(p.batch < 65536, ERR_ARG, "gemm batch too large");
 }
 
+// p as the planner and the kernels take it: an empty sum (K = 0: C = beta C) has any index of extent one, which the
+// empty loop over k never reads, so that nobody divides by an extent of zero.
 template <typename T>
-void tc_gemm(const GemmParams<T>& p, Workspace& ws, hipStream_t s) {
+static GemmParams<T> summable(GemmParams<T> p) {
+  if (p.K == 0 || p.kx == 0) {
+    p.K = 0;
+    p.kx = 1;
+    p.a_x = p.b_x = 0;
+    p.ak = p.bk = Idx2{1, 0, 0};
+  }
+  return p;
+}
+
+template <typename T>
+void tc_gemm(const GemmParams<T>& given, Workspace& ws, hipStream_t s) {
+  const GemmParams<T> p = summable(given);
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
   {
     // enough 128 x 128 tiles to fill the 256 CUs: the plain-matrix kernel
@@ -915,7 +929,8 @@ void GemmQueue::axpby(const EltOp& e, int64_t n) {
   elts.push_back(x);
 }
 
-void GemmQueue::gemm(const GemmParams<double>& p, int part) {
+void GemmQueue::gemm(const GemmParams<double>& given, int part) {
+  const GemmParams<double> p = summable(given);
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
   check_extents(p);
   Op o{p, Range{}, Range{}, range_of(p.C, p.cm, p.M, p.cn, p.N, 1, 0, p.batch, p.c_b), part};
