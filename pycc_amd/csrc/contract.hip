@@ -212,7 +212,8 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   }
   if (gb.size() > 1) { loop_over(smallest(ob)); return; }
   // Three K classes: the third is the GEMM's outer K level -- the one of the smallest extent that is not
-  // contiguous in an operand. (The sliced form stays where a slice alone is an FP16x3 product.)
+  // contiguous in an operand. (The sliced form stays where a slice alone is an FP16x3 product, and where the kernel
+  // cannot count all of K in 31 bits.)
   Lab kx{0, 1, {0, 0, 0}};
   if (gk.size() == 3) {
     size_t x = 3;
@@ -222,7 +223,7 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
     std::vector<Lab> in = gk;
     in.erase(in.begin() + x);
     const double slice = 2.0 * (double)extent(gm) * (double)extent(gn) * (double)extent(in);
-    if (!(std::is_same<T, double>::value && split16 && slice >= X3_ROUTE_FLOPS)) {
+    if (extent(gk) < (1ll << 31) && !(std::is_same<T, double>::value && split16 && slice >= X3_ROUTE_FLOPS)) {
       kx = gk[x];
       gk = in;
     }
