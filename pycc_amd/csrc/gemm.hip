@@ -90,7 +90,8 @@ __device__ __forceinline__ int64_t off2(const FastIdx& d, uint32_t i) {
 
 template <typename T>
 struct TileGemm {
-  int M, N, K, kx, splits, chunk;   // chunk: k-tiles per split, counted over x and k
+  uint32_t M, N, K;         // under 2^31: rows, columns and k's of a tile that reaches past them stay under 2^32
+  int kx, splits, chunk;    // chunk: k-tiles per split, counted over x and k
   FastIdx am, ak, bk, bn, cm, cn;
   int64_t a_x, b_x, a_b, b_b, c_b;
   T alpha, beta;
@@ -149,29 +150,29 @@ struct GLoader {
     uint32_t ok;   // bit i: piece i's k is inside
     bool late, whole;
   };
-  __device__ __forceinline__ void init(const FastIdx& rix, int row0, int nrows, int tid) {
+  __device__ __forceinline__ void init(const FastIdx& rix, uint32_t row0, uint32_t nrows, int tid) {
     const int along = tid % LANES * V, across = tid / LANES;
     kl = KF ? along : UK ? __builtin_amdgcn_readfirstlane(across) : across;
     rl = KF ? across : along;
     row_late = false;
 #pragma unroll
     for (int i = 0; i < (KF ? NE : 1); ++i) {
-      int r = row0 + rl + i * STEP;
+      uint32_t r = row0 + rl + i * STEP;
       if (!KF && V == 2) row_late = r == nrows - 1;
       r = r < nrows - (KF ? 1 : V) ? r : nrows - (KF ? 1 : V);
-      roff[i] = (Off)(off2(rix, (uint32_t)r) * (int64_t)sizeof(T));
+      roff[i] = (Off)(off2(rix, r) * (int64_t)sizeof(T));
     }
   }
-  __device__ __forceinline__ void seek(const FastIdx& kix, int k0) {
+  __device__ __forceinline__ void seek(const FastIdx& kix, uint32_t k0) {
     if (UK) return;
 #pragma unroll
     for (int i = 0; i < NO; ++i) {
-      const uint32_t k = (uint32_t)(k0 + kl + i * STEP), q = (__umulhi(k, kix.mul) + k) >> kix.sh;
+      const uint32_t k = k0 + kl + i * STEP, q = (__umulhi(k, kix.mul) + k) >> kix.sh;
       kr[i] = k - q * kix.n2;
       koff[i] = (Off)(((int64_t)q * kix.s1 + (int64_t)kr[i] * kix.s2) * (int64_t)sizeof(T));
     }
   }
-  __device__ __forceinline__ void step(const FastIdx& kix, int k0) {   // BK further, to the tile at k0
+  __device__ __forceinline__ void step(const FastIdx& kix, uint32_t k0) {   // BK further, to the tile at k0
     if (UK) return;
     if (kix.n2 < (uint32_t)BK) {
       seek(kix, k0);
@@ -197,13 +198,13 @@ struct GLoader {
     }
   }
   // rows_in: every row of the tile is inside
-  __device__ __forceinline__ void load(Load& l, const T* __restrict__ base, const FastIdx& kix, int k0, int K,
+  __device__ __forceinline__ void load(Load& l, const T* __restrict__ base, const FastIdx& kix, uint32_t k0, uint32_t K,
                                        bool rows_in) {
     l.ok = 0;
     l.late = row_late;
     l.whole = rows_in && k0 + BK <= K;
     if constexpr (KF) {
-      const int k = k0 + kl;
+      const uint32_t k = k0 + kl;
       Off ko = koff[0];
       if (V == 2) l.late = k == K - 1;
       if (k > K - V) ko = V == 2 && k < K ? ko - (Off)sizeof(T) : 0;
@@ -213,9 +214,9 @@ struct GLoader {
     } else {
 #pragma unroll
       for (int i = 0; i < NE; ++i) {
-        const int k = k0 + kl + i * STEP;
+        const uint32_t k = k0 + kl + i * STEP;
         if (k < K) l.ok |= 1u << i;
-        if constexpr (UK) get(l.v[i], (const char*)(base + off2(kix, (uint32_t)(k < K ? k : K - 1))) + roff[0]);
+        if constexpr (UK) get(l.v[i], (const char*)(base + off2(kix, k < K ? k : K - 1)) + roff[0]);
         else get(l.v[i], (const char*)base + (Off)(roff[0] + (k < K ? koff[i] : (Off)0)));
       }
     }
@@ -257,13 +258,13 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
   const int64_t group = t / (8 * tiles_n);
   const int first_m = (int)group * 8, gsize = tiles_m - first_m < 8 ? tiles_m - first_m : 8;
   const int within = (int)(t - group * 8 * tiles_n);
-  const int m0 = (first_m + within % gsize) * BM, n0 = within / gsize * BN;
+  const uint32_t m0 = (uint32_t)(first_m + within % gsize) * BM, n0 = (uint32_t)(within / gsize) * BN;
 
   const int ntk = (p.K + BK - 1) / BK;   // k-tiles of one x
   int kt = sidx * p.chunk;               // first and end k-tile of this split, over x and k
   const int kt_end = kt + p.chunk < ntk * p.kx ? kt + p.chunk : ntk * p.kx;
   const int x0 = ntk ? kt / ntk : 0;
-  int k0 = (kt - x0 * ntk) * BK;
+  uint32_t k0 = (uint32_t)(kt - x0 * ntk) * BK;
   const T* __restrict__ A = p.A + bidx * p.a_b + x0 * p.a_x;
   const T* __restrict__ B = p.B + bidx * p.b_b + x0 * p.b_x;
 
@@ -369,14 +370,14 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = row(i, r);
+        const uint32_t m = row(i, r);
         if (i >= ni || m >= p.M) continue;
-        T* Cm = C + off2(p.cm, (uint32_t)m);
+        T* Cm = C + off2(p.cm, m);
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) {
-          const int n = n0 + c0 + j * 16 + fc;
+          const uint32_t n = n0 + c0 + j * 16 + fc;
           if (j >= nj || n >= p.N) continue;
-          T* dst = Cm + off2(p.cn, (uint32_t)n);
+          T* dst = Cm + off2(p.cn, n);
           T v = p.alpha * acc[i][j][r];
           if (p.beta != T(0)) v += p.beta * *dst;
           *dst = v;
@@ -388,11 +389,11 @@ __device__ __forceinline__ void tile_body(const TileGemm<T>& p, int64_t t, int b
     for (int i = 0; i < NBI; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = row(i, r);
+        const uint32_t m = row(i, r);
         if (i >= ni || m >= p.M) continue;
 #pragma unroll
         for (int j = 0; j < NBJ; ++j) {
-          const int n = n0 + c0 + j * 16 + fc;
+          const uint32_t n = n0 + c0 + j * 16 + fc;
           if (j < nj && n < p.N) W[(int64_t)m * p.N + n] = acc[i][j][r];
         }
       }
@@ -404,7 +405,9 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 4) void tile_gemm_kerne
   __shared__ GTile<T, BM, BK, AKF> As[2];
   __shared__ GTile<T, BN, BK, BKF> Bs[2];
   const int64_t tiles = (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-  tile_body<T, BM, BN, WM, WN, BK, AKF, BKF, Off, V>(p, xcd_remap(blockIdx.x, tiles), blockIdx.y / p.splits,
+  const int64_t t = blockIdx.x + (int64_t)gridDim.x * blockIdx.z;
+  if (t >= tiles) return;
+  tile_body<T, BM, BN, WM, WN, BK, AKF, BKF, Off, V>(p, xcd_remap(t, tiles), blockIdx.y / p.splits,
                                                      blockIdx.y % p.splits, gridDim.y / p.splits, As, Bs);
 }
 
@@ -423,7 +426,7 @@ template <bool AKF, bool BKF, int V>
 __device__ __forceinline__ void group_body(const TileGemm<double>& p, int nbatch, int local, char* lds) {
   typedef GTile<double, 64, 16, AKF> TA;
   typedef GTile<double, 64, 16, BKF> TB;
-  const int tiles = ((p.M + 63) / 64) * ((p.N + 63) / 64), y = local / tiles;
+  const int tiles = (int)((p.M + 63) / 64) * (int)((p.N + 63) / 64), y = local / tiles;
   tile_body<double, 64, 64, 32, 32, 16, AKF, BKF, uint32_t, V>(p, local - y * tiles, y / p.splits, y % p.splits, nbatch,
                                                                (TA*)lds, (TB*)(lds + 2 * sizeof(TA)));
 }
@@ -484,9 +487,9 @@ __global__ __launch_bounds__(256) void sum_group_kernel(const SumGroup a) {
     s = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
   }
   if (e >= total) return;
-  const uint32_t mn = (uint32_t)p.M * (uint32_t)p.N, b = (uint32_t)(e / mn), r = (uint32_t)(e - (int64_t)b * mn);
-  const uint32_t m = r / (uint32_t)p.N;
-  double* dst = p.C + b * p.c_b + off2(p.cm, m) + off2(p.cn, r - m * (uint32_t)p.N);
+  const uint32_t mn = p.M * p.N, b = (uint32_t)(e / mn), r = (uint32_t)(e - (int64_t)b * mn);
+  const uint32_t m = r / p.N;
+  double* dst = p.C + b * p.c_b + off2(p.cm, m) + off2(p.cn, r - m * p.N);
   double v = p.alpha * s;
   if (p.beta != 0.0) v += p.beta * *dst;
   *dst = v;
@@ -495,7 +498,9 @@ __global__ __launch_bounds__(256) void sum_group_kernel(const SumGroup a) {
 template <typename T, int BM, int BN, int WM, int WN, typename Off, int V>
 static void launch_tile(const TileGemm<T>& p, int64_t batch, bool akf, bool bkf, hipStream_t s) {
   constexpr int BK = 16, NT = 64 * (BM / WM) * (BN / WN);
-  const dim3 grid((unsigned)(ceil_div(p.M, BM) * ceil_div(p.N, BN)), (unsigned)(batch * p.splits));
+  // a launch has under 2^32 threads along x (outputs of a row or two with 2^30 columns have more): z takes the rest
+  const int64_t tiles = ceil_div(p.M, BM) * ceil_div(p.N, BN), gx = std::min<int64_t>(tiles, ((1ll << 32) - 1) / NT);
+  const dim3 grid((unsigned)gx, (unsigned)(batch * p.splits), (unsigned)ceil_div(tiles, gx));
   if (akf && bkf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, true, true, Off, V><<<grid, NT, 0, s>>>(p);
   else if (akf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, true, false, Off, V><<<grid, NT, 0, s>>>(p);
   else if (bkf) tile_gemm_kernel<T, BM, BN, WM, WN, BK, false, true, Off, V><<<grid, NT, 0, s>>>(p);
@@ -802,9 +807,9 @@ static Form form_of(const GemmParams<T>& p, int tile) {
 template <typename T>
 static TileGemm<T> describe(const GemmParams<T>& p, const Plan& pl) {
   TileGemm<T> g;
-  g.M = (int)p.M;
-  g.N = (int)p.N;
-  g.K = (int)p.K;
+  g.M = (uint32_t)p.M;
+  g.N = (uint32_t)p.N;
+  g.K = (uint32_t)p.K;
   g.kx = (int)p.kx;
   g.splits = pl.splits;
   g.chunk = pl.chunk;

@@ -61,3 +61,39 @@ def test_three_summed_indices_past_2_31():
     for i in range(k):
         want += float((torch.as_strided(A, (l, m), sa[1:], i * sa[0]) * torch.as_strided(B, (l, m), sb[1:], i * sb[0])).sum())
     assert float(C) == want
+
+
+# one row of outputs as wide as an index goes, B row-fast and k-fast; past 2^30 columns a launch of 64-wide tiles has
+# more threads than its x extent holds
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,n", [(torch.float32, (1 << 31) - 1), (torch.float64, (1 << 30) + 77)])
+@pytest.mark.parametrize("step", [1, 5])
+def test_one_row_of_very_many_columns(dtype, n, step):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    K = 3
+    B = _whole(n + step * K, dtype, 3)
+    a = torch.tensor([1.0, -2.0, 3.0], dtype=dtype, device="cuda")
+    C = torch.empty(n, dtype=dtype, device="cuda")
+    assert _call("k,kn->n", dtype, [(a.data_ptr(), (K,), (1,)), (B.data_ptr(), (K, n), (step, 1)), (C.data_ptr(), (n,), (1,))]) == 0
+    for k, x in enumerate((1.0, -2.0, 3.0)):
+        C.sub_(B[k * step:k * step + n], alpha=x)
+    assert int(torch.count_nonzero(C)) == 0
+
+
+# a sum as long as an index goes: of equal ones (no stride), and of a buffer that holds ones only at both ends
+@pytest.mark.gpu
+def test_a_sum_of_very_many_products():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    k = (1 << 31) - 1
+    one = torch.ones(1, dtype=torch.float64, device="cuda")
+    out = torch.empty(1, dtype=torch.float64, device="cuda")
+    assert _call("k,k->", torch.float64, [(one.data_ptr(), (k,), (0,))] * 2 + [(out.data_ptr(), (), ())]) == 0
+    assert float(out) == k
+    x = torch.zeros(k, dtype=torch.float32, device="cuda")
+    x[:3] = 1.0
+    x[-20:] = 2.0
+    out = torch.empty(1, dtype=torch.float32, device="cuda")
+    assert _call("k,k->", torch.float32, [(x.data_ptr(), (k,), (1,))] * 2 + [(out.data_ptr(), (), ())]) == 0
+    assert float(out) == 3.0 + 20 * 4.0
