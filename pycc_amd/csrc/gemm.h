@@ -17,8 +17,9 @@ struct Workspace {
   size_t limit = size_t(1) << 30;
   bool fixed = false;
   // FP64 sums over K in up to FIXED_K_SPLITS parts are partitioned by the shape alone, and the parts added in order: a
-  // context whose FP64 results become FP32 or split FP16 operands then rounds the same operands however a
-  // launch is planned.
+  // context whose FP64 results become FP32 or split FP16 operands then rounds the same operands whatever else is queued
+  // beside them. (Two rules: one of the tile kernel and one of the plain-matrix kernel, whose contractions are never
+  // grouped in such a context. Sums in more parts, of few outputs, follow the launch that they are in.)
   bool fixed_k = false;
   static Workspace wrap(void* p, size_t bytes) {
     Workspace w;

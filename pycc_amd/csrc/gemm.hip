@@ -672,6 +672,12 @@ static bool as_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
   return plain_gemm_ok(q);
 }
 
+// Whether p runs on the plain-matrix kernel: enough 128 x 128 tiles to fill the 256 CUs
+template <typename T>
+static bool takes_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
+  return p.kx == 1 && ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q);
+}
+
 // Tile and split count of an FP64 contraction: the cheapest of both tiles and a few split counts under a model of
 // the launch fitted to M x N x 1313 products of 1, 2 and 3 tiles per CU (64 x 64: 68, 115, 158 us) and to 8192^3
 // (128 x 128: 18 ms): a k-tile costs 0.25 us a round of resident work-groups plus its flops at 0.24 TF a CU,
@@ -857,13 +863,10 @@ template <typename T>
 void tc_gemm(const GemmParams<T>& given, Workspace& ws, hipStream_t s) {
   const GemmParams<T> p = summable(given);
   if (p.M == 0 || p.N == 0 || p.batch == 0) return;
-  {
-    // enough 128 x 128 tiles to fill the 256 CUs: the plain-matrix kernel
-    PlainGemm<T> q;
-    if (p.kx == 1 && ceil_div(p.M, 128) * ceil_div(p.N, 128) * p.batch >= 240 && as_plain(p, q)) {
-      plain_dispatch<T>(q, ws, s);
-      return;
-    }
+  PlainGemm<T> q;
+  if (takes_plain(p, q)) {
+    plain_dispatch<T>(q, ws, s);
+    return;
   }
   check_extents(p);
   const Plan pl = plan(p, ws);
@@ -951,7 +954,11 @@ void GemmQueue::gemm(const GemmParams<double>& given, int part) {
     }
   }
   const int64_t tiles = ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batch;
-  if (tiles > GROUP_TILES || 2.0 * p.M * p.N * p.K * p.kx * p.batch > GROUP_FLOPS || !form_of(p, 64).off32) {
+  // With fixed_k, the plain kernel's too: it has a partition of K of its own, so that whether such a contraction takes
+  // it must not depend on what else is queued.
+  PlainGemm<double> plain;
+  if (tiles > GROUP_TILES || 2.0 * p.M * p.N * p.K * p.kx * p.batch > GROUP_FLOPS || !form_of(p, 64).off32 ||
+      (ws.fixed_k && takes_plain(p, plain))) {
     // it fills the chip by itself: now, before the queued ones, which it does not meet
     bool clash = false;
     for (auto& e : elts) clash = clash || o.a.meets(e.c) || o.b.meets(e.c) || o.c.meets(e.c) || o.c.meets(e.a);
