@@ -58,7 +58,7 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s);
 
 // nbatch FP16x3 GEMMs C_b = alpha / (sa sb) [A_p | A_p2 swapped] [B | B2] with K = Kp concatenated
 // from two blocks of each operand (fields tri .. sC above): the connected (T) numerators, two slot products per
-// GEMM. K1 is a multiple of 8 with K1 % 32 != 24, Kp the next multiple of 32 from 2 K1; B is zero past its K.
+// GEMM. K1 and Kp are multiples of 32.
 void x3_gemm_kcat(const X3Gemm& p, hipStream_t s);
 // max |x| over n elements as x3_partials() per-block partial maxima in `part`.
 template <typename T>

@@ -460,13 +460,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
   const int blocks = brief ? (last_rows + 15) >> 4 : BT / 16;   // 16-row blocks of A that are loaded
 
   int64_t gA[IPW], gB[IPB];
-  // KCAT: offsets in the second blocks, so that 16-byte chunk g = 4 q + c of the concatenated K (q the
-  // k-tile, c the lane's chunk) is chunk g - K1 / 8 there (M lda < 2^31, checked by x3_gemm_kcat)
-  int gA2[KCAT ? IPW : 1], gB2[KCAT ? IPB : 1];
-  const auto chunk2 = [&](int c) {
-    const int K1c = (int)(p.K1 >> 3), c2 = (c - K1c) & 3;
-    return c2 * 8 - (K1c - c + c2) / 4 * 64;
-  };
+  int gA2[KCAT ? IPW : 1];   // KCAT: offsets in the second block of A (M lda < 2^31, checked by x3_gemm_kcat)
   int ldso[IPW], ldsb[IPB];
 #pragma unroll
   for (int i = 0; i < IPW; ++i) {
@@ -475,7 +469,7 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     int64_t m = tm * BT + row;
     m = m < p.M ? m : p.M - 1;
     gA[i] = m * p.lda + c * 8;
-    if constexpr (KCAT) gA2[i] = (int)(((m % p.sw) * p.sw + m / p.sw) * p.lda) + chunk2(c);
+    if constexpr (KCAT) gA2[i] = (int)(((m % p.sw) * p.sw + m / p.sw) * p.lda + c * 8);
     ldso[i] = R0 * 32;
   }
 #pragma unroll
@@ -486,7 +480,6 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     int64_t n = tn * BN + row;
     n = n < p.N ? n : p.N - 1;
     gB[i] = n * p.ldb + c * 8;
-    if constexpr (KCAT) gB2[i] = (int)(n * p.ldb) + chunk2(c);
     ldsb[i] = R0 * 32;
   }
   auto issue = [&](int st, int64_t k0, auto short_row) {
@@ -500,29 +493,26 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
       kb = q * p.skb + r;
     }
     if constexpr (KCAT) {
-      const bool first = k0 + BK <= p.K1, mixed = !first && k0 < p.K1;   // wave-uniform
+      // The second blocks start at a k-tile of their own, so that a row's 32 k of a tile are one 128-byte line. Joined
+      // within a tile (at a multiple of 8, one k-tile less) every tile of the second half reads halves of two
+      // lines: E(T) at o=24 v=176 179 ms against 163, o=16 v=340 699 against 645, o=48 v=384 20.4 s in all.
+      auto load = [&](const E* a, const auto& oa, const E* b, int64_t k) {
+        const int64_t kq = (k >> 5) * 64;
 #pragma unroll
-      for (int i = 0; i < IPW; ++i) {
-        const E* g = (first ? Ah + gA[i] : Ah2 + gA2[i]) + ka;
-        if (mixed) {
-          const int R0 = (wave * IPW + i) * 16, row = R0 + (lane >> 2), c = (lane & 3) ^ ((row >> 1) & 3);
-          if (k0 + 8 * c < p.K1) g = Ah + gA[i] + ka;
+        for (int i = 0; i < IPW; ++i) {
+          x3_dma16<E>(a + oa[i] + kq, &sA[st][0][ldso[i]]);
+          x3_dma16<E>(a + 32 + oa[i] + kq, &sA[st][1][ldso[i]]);
         }
-        x3_dma16<E>(g, &sA[st][0][ldso[i]]);
-        x3_dma16<E>(g + 32, &sA[st][1][ldso[i]]);
-      }
 #pragma unroll
-      for (int i = 0; i < IPB; ++i) {
-        if (wave + 8 * i < NIB) {   // wave-uniform
-          const E* g = (first ? Bh + gB[i] : Bh2 + gB2[i]) + kb;
-          if (mixed) {
-            const int row = (wave + 8 * i) * 16 + (lane >> 2), c = (lane & 3) ^ ((row >> 1) & 3);
-            if (k0 + 8 * c < p.K1) g = Bh + gB[i] + kb;
+        for (int i = 0; i < IPB; ++i) {
+          if (wave + 8 * i < NIB) {   // wave-uniform
+            x3_dma16<E>(b + gB[i] + kq, &sB[st][0][ldsb[i]]);
+            x3_dma16<E>(b + 32 + gB[i] + kq, &sB[st][1][ldsb[i]]);
           }
-          x3_dma16<E>(g, &sB[st][0][ldsb[i]]);
-          x3_dma16<E>(g + 32, &sB[st][1][ldsb[i]]);
         }
-      }
+      };
+      if (k0 >= p.K1) load(Ah2, gA2, Bh2, k0 - p.K1);   // wave-uniform
+      else load(Ah, gA, Bh, k0);
     } else {
 #pragma unroll
       for (int i = 0; i < IPW; ++i) {
@@ -1266,7 +1256,7 @@ bool x3_contract(const GemmParams<double>& p, Workspace& ws, hipStream_t s) {
 
 void x3_gemm_kcat(const X3Gemm& p, hipStream_t s) {
   if (p.M == 0 || p.N == 0 || p.nbatch == 0) return;
-  CCX_CHECK(p.kb == BK && p.ska == 2 * BK && p.skb == 2 * BK && p.Kp % BK == 0 && p.K1 % 8 == 0 && p.K1 > 0 &&
+  CCX_CHECK(p.kb == BK && p.ska == 2 * BK && p.skb == 2 * BK && p.Kp % BK == 0 && p.K1 % BK == 0 && p.K1 > 0 &&
                 p.K1 < p.Kp && p.lda % 8 == 0 && p.ldb % 8 == 0 && p.tri && p.C && !p.C64 && !p.work &&
                 p.sw > 0 && p.sw * p.sw == p.M && p.M * p.lda < (int64_t(1) << 31) && p.beta == 0.f && !p.sbn &&
                 (p.ytile == 0 || (p.ytile % 8 == 0 && p.ytile == p.sw && p.ytile == p.N &&

@@ -496,11 +496,7 @@ void triples_energy(Ctx& c, const double* F, const double* t1, const double* t2,
   // In MIXED_F16X3 the slot GEMMs are FP16x3 split products (interleaved hi/lo operands, K padded
   // to 32, FP32 accumulation and output); every other mode runs them in FP64 (K padded to 8).
   const bool x3 = c.mode == MODE_MIXED_F16X3;
-  // FP16x3: the halves of the concatenated K end at K1, a multiple of 8, and the whole at the next
-  // multiple of 32, in the zeros that pad a row of B and whatever pads that of A.
   const int64_t kpad = x3 ? 32 : 8, Kp = (v + o + kpad - 1) / kpad * kpad;
-  int64_t K1 = (v + o + 7) / 8 * 8;
-  if (x3 && K1 % 32 == 24) K1 += 8;
   // FP16x3: Y in 8 x 8 (y, z) blocks when v is a multiple of 8, else rows padded to 4 floats. FP64:
   // rows padded to 128 bytes, whole lines for the GEMM's stores (odd v = 107: 12.6 to 12.1 ms).
   const bool tiled = x3 && v % 8 == 0;
@@ -569,7 +565,7 @@ void triples_energy(Ctx& c, const double* F, const double* t1, const double* t2,
       const unsigned eg = (unsigned)(norb * nc);
       if (x3) {
         X3Gemm g;   // C_(e, s)[m][n] = sum_kk [A | A2 swapped][m][kk] [B | B2][n][kk]
-        g.M = vv; g.N = v; g.Kp = (2 * K1 + 31) / 32 * 32; g.K1 = K1; g.lda = 2 * Kp; g.ldb = 2 * Kp; g.ldc = ldy;
+        g.M = vv; g.N = v; g.Kp = 2 * Kp; g.K1 = Kp; g.lda = 2 * Kp; g.ldb = 2 * Kp; g.ldc = ldy;
         g.kb = 32; g.ska = 64; g.skb = 64; g.sw = v; g.nbatch = 3 * nc; g.ytile = tiled ? v : 0;
         g.sa = sc; g.sb = sc + 1; g.sA = vv * 2 * Kp; g.sB = v * 2 * Kp; g.sC = ys;
         g.tri = tr; g.nocc = i1;
