@@ -494,8 +494,8 @@ __global__ __launch_bounds__(512) void x3_gemm_dma_kernel(X3Gemm p) {
     }
     if constexpr (KCAT) {
       // The second blocks start at a k-tile of their own, so that a row's 32 k of a tile are one 128-byte line. Joined
-      // within a tile (at a multiple of 8, one k-tile less) every tile of the second half reads halves of two
-      // lines: E(T) at o=24 v=176 179 ms against 163, o=16 v=340 699 against 645, o=48 v=384 20.4 s in all.
+      // within a k-tile (at a multiple of 8, for one k-tile less) the second half read halves of two lines: E(T) at o=24
+      // v=176 179 ms against 162, o=16 v=340 689 against 639, triples of i = 22 to 25 at o=48 v=384 1304 against 1199.
       auto load = [&](const E* a, const auto& oa, const E* b, int64_t k) {
         const int64_t kq = (k >> 5) * 64;
 #pragma unroll

@@ -473,11 +473,13 @@ std::vector<int> t3_orbits(int64_t nt) {
   return out;
 }
 
-// Bytes of Y (3 v^3 elements per triple) that a chunk may hold, at least one triple: enough tiles for
-// the last, partly filled round of work-groups of a launch to cost little, yet little to allocate.
-// o = 11 v = 107 FP64: 12.6 ms at 330 MB, 12.3 at 526, 12.2 at 1 GB, 67-85 for a first call at 2.2 GB;
-// o = 24 v = 176 FP16x3: 185.5, 182.3, 180.5 ms.
-constexpr int64_t T3_Y_BYTES = int64_t(512) << 20;
+// Y (3 v^3 elements per triple) of a chunk: 512 MB of it, enough tiles for the last, partly filled round
+// of work-groups of a launch to cost little, yet little to allocate (o = 11 v = 107 FP64: 12.6 ms at 330 MB,
+// 12.3 at 526, 12.2 at 1 GB, 67-85 for a first call at 2.2 GB); and eight triples where they take more, up to
+// 16 GB: by bytes alone a chunk is one triple from v = 224 in FP64, whose launches of 2400 tiles end in a round of
+// their own. One to four triples, then eight: FP64 o = 20 v = 224, i = 10 to 19, 838 and 769 ms, o = 16 v = 182 238 and
+// 230; FP16x3 o = 24 v = 300, i = 14 to 19, 497 and 481, o = 48 v = 384, i = 22 to 25, 1196 and 1173.
+constexpr int64_t T3_Y_BYTES = int64_t(512) << 20, T3_Y_MOST = int64_t(16) << 30, T3_TRIPLES = 8;
 // Orbit partials held before they are summed per triple (64 MB).
 constexpr int64_t T3_PARTIALS = int64_t(1) << 23;
 
@@ -509,7 +511,8 @@ void triples_energy(Ctx& c, const double* F, const double* t1, const double* t2,
   const std::vector<int> orb = t3_orbits(nt);
   const int64_t norb = (int64_t)orb.size();
   const int64_t ybytes = 3 * ys * (x3 ? 4 : 8);
-  const int64_t KC = std::max<int64_t>(1, std::min(ntri, std::min(T3_Y_BYTES / ybytes, T3_PARTIALS / norb)));
+  const int64_t room = std::max(T3_Y_BYTES / ybytes, std::min(T3_TRIPLES, T3_Y_MOST / ybytes));
+  const int64_t KC = std::max<int64_t>(1, std::min({ntri, room, T3_PARTIALS / norb}));
   CCX_CHECK(KC * norb < (int64_t(1) << 31), ERR_ARG, "too many virtual orbitals for the (T) tiles");
   const int64_t group = std::max(KC, std::min(ntri, T3_PARTIALS / norb) / KC * KC);   // triples per sum of partials
 
