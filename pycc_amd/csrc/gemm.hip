@@ -680,16 +680,18 @@ static bool takes_plain(const GemmParams<T>& p, PlainGemm<T>& q) {
 }
 
 // Tile and split count of an FP64 contraction: the cheapest of both tiles and a few split counts under a model of the
-// launch. It is fitted to the times of every tile and split count of 120 contractions from 5 x 5 x 1805 to 5632^3 (plain
-// and compound, thin and square, K from 13 to 410571); the plan that it takes is 0.7% from the best of them in the mean
-// and 7% at most (1024^3: 128 x 128 in 4, 57 us; 64 x 64 unsplit 77; 1313^3 125 to 130 against 158; 3072^3 1042
-// against 1129). A launch costs 9 us, a k-tile 0.32 us a round of resident work-groups plus its flops at 0.22 (64 x 64)
-// or 0.26 TF (128 x 128) a CU, partial sums, which mostly stay in the caches, move at 9.7 TB/s behind a launch of 4 us.
+// launch. It is fitted to the times of every tile and split count of 150 contractions from 5 x 5 x 1805 to 5632^3 (plain
+// and compound, one row to square, K from 13 to 410571); the plan that it takes is 0.8% from the best of them in the
+// mean and 7% at most (1024^3: 128 x 128 in 4, 57 us; 64 x 64 unsplit 77; 1313^3 125 to 130 against 158; 3072^3 1042
+// against 1129; 1 x 40000 x 2400: 64 x 64 in 4, 154 us, in 30 187, unsplit 198). A launch costs 5 us; a k-tile takes 0.26
+// (64 x 64) or 0.49 us (128 x 128) a round of resident work-groups plus its flops at 0.205 or 0.252 TF a CU, and at least
+// the latency of its loads, 1.05 us a round; the operands come at 5.7 TB/s beside it; partial sums, which mostly stay in
+// the caches, move at 7.4 TB/s behind a launch that gains its 8 us (4 to 9 fit alike; with 4 products of 10 us were split).
 //
 // Where an operand is not contiguous along either index that its lanes could walk (two summed indices, each contiguous in
 // another operand), every lane reads a line of its own, which later k-tiles have to find in cache. Past two 64 x 64
-// tiles a CU that fails for these, whose panels are read twice as often (5120^3 of o=32 v=160: 20.1 ms, 128 x 128 6.0 to
-// 6.6), and it fails the sooner the longer the work-groups that share a panel run apart: 4% per doubling of a split's
+// work-groups a CU that fails for these, whose panels are read twice as often (5120^3 of o=32 v=160: 20.1 ms, 128 x 128 6.0
+// to 6.6; 576 x 576 x 22500 1.5 and 0.96), and it fails the sooner the longer the work-groups that share a panel run apart: 4% per doubling of a split's
 // k-tiles over 40, which gives 2048^3 two parts and 4960^3 five (8.8 ms unsplit, in 4 8.0, in 8 7.6).
 struct Plan {
   int tile = 128, splits = 1, chunk = 0;
@@ -704,22 +706,25 @@ static Plan plan_f64(const GemmParams<double>& p, size_t limit) {
   const int64_t ntk = std::max<int64_t>(1, ceil_div(p.K, 16) * p.kx);
   // lanes walk k wherever rows are not contiguous (form_of)
   const bool strided = (p.am.s2 != 1 && p.ak.s2 != 1) || (p.bn.s2 != 1 && p.bk.s2 != 1);
-  const bool cached = strided && p.M > 64 && p.N > 64 && ceil_div(p.M, 64) * ceil_div(p.N, 64) * p.batch > 512;
+  const bool cached = strided && p.M > 64 && p.N > 64;
+  const double t_load = 8.0 * (double)p.batch * ((double)(p.K * p.kx) * (double)(p.M + p.N) + (double)p.M * (double)p.N) / 5.7e6;
   Plan best;
   double t_best = 0.0;
   for (int tile : {128, 64}) {
-    if (tile == 64 && cached) continue;
     const int64_t tiles = ceil_div(p.M, tile) * ceil_div(p.N, tile) * p.batch;
-    const double t_ktile = tile == 64 ? 1.09 * tile64_us(p) / (double)(tiles * ntk) : 2.0 * tile * tile * 16 / 0.26e6;
+    const double t_ktile = tile == 64 ? 1.17 * tile64_us(p) / (double)(tiles * ntk) : 2.0 * tile * tile * 16 / 0.252e6;
     const int per_cu = tile == 128 ? 2 : 4;   // resident work-groups (LDS)
     for (int want : counts) {
       const int64_t chunk = ceil_div(ntk, want), splits = ceil_div(ntk, chunk);
       if (want > 1 && (chunk < 4 || splits * p.batch > 65535)) break;
       const double bytes = 8.0 * (double)splits * (double)p.batch * (double)p.M * (double)p.N;
       if (want > 1 && bytes > (double)limit) break;
+      if (cached && tile == 64 && tiles * splits > 512) break;
       const int64_t on_cu = ceil_div(tiles * splits, 256);
-      double t = 9.0 + (double)chunk * (0.32 * (double)ceil_div(on_cu, per_cu) + (double)on_cu * t_ktile);
-      if (splits > 1) t += 4.0 + 2.0 * bytes / 9.7e6;
+      const double rounds = (double)ceil_div(on_cu, per_cu), busy = (double)on_cu * t_ktile;
+      const double work = (double)chunk * (tile == 64 ? std::max(1.05 * rounds, 0.26 * rounds + busy) : 0.49 * rounds + busy);
+      double t = 5.0 + std::max(work, t_load) + 0.05 * std::min(work, t_load);
+      if (splits > 1) t += 8.0 + 2.0 * bytes / 7.4e6;
       if (cached && chunk > 40) t *= 1.0 + 0.04 * std::log2((double)chunk / 40.0);
       if (t_best == 0.0 || t < t_best) {
         t_best = t;
