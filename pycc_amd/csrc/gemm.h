@@ -79,7 +79,6 @@ class GemmQueue {
   void gemm(const GemmParams<double>& p, int part = 0);
   void axpby(const EltOp& e, int64_t n);
   void flush();
-  bool empty() const;
 
  private:
   struct Op;

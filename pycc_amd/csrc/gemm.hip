@@ -1,9 +1,9 @@
 // MFMA tensor-contraction GEMM for gfx950.
 //
-// One kernel serves every contraction of the CCSD residual: each GEMM dimension (M, N, K) is a
-// 2-level index (two tensor indices with independent strides) and there is one batch index, so
-// e.g. 'jnfb,mnef->mbej' runs without materialising permuted copies. Operands are staged through
-// LDS in k-major tiles; each of the 4 waves owns a (BM/2) x (BN/2) block of 16x16 MFMA tiles.
+// The tile kernel serves every contraction that is not a plain matrix product of many tiles (gemm_plain.hip): M and N
+// are 2-level indices (two tensor indices with independent strides), K has a third, outer level, and there is one
+// batch index, so e.g. 'jnfb,mnef->mbej' runs without materialising permuted copies. It comes as 128 x 128 tiles of 8
+// waves (64 x 32 each) and 64 x 64 tiles of 4, alone or several contractions to a launch (GemmQueue).
 //
 // Lane layout of the 16x16x4 MFMAs used here (measured on gfx950):
 //   A (16x4):  lane l holds A[l % 16][l / 16]
@@ -935,8 +935,6 @@ struct GemmQueue::Elt {
 
 GemmQueue::GemmQueue(Workspace& w, hipStream_t st) : ws(w), s(st) {}
 GemmQueue::~GemmQueue() {}
-
-bool GemmQueue::empty() const { return ops.empty() && elts.empty(); }
 
 void GemmQueue::axpby(const EltOp& e, int64_t n) {
   if (n == 0) return;
