@@ -169,16 +169,21 @@ int ccx_density_energy(ccx_ctx* ctx, const double* t1, const double* t2, const d
  * the orbital-energy denominators from the diagonal of `fock`. FP64, except in CCX_MODE_MIXED_F16X3,
  * whose slot products are FP16x3 split products with FP32 accumulation and output (E(T) within
  * ~1e-9 relative of FP64 for tens of virtuals and more, ~5e-8 for two or three). Synchronises
- * `stream`. Device scratch for the duration of the call:
- * o v^2 (v + o) + 24 v^3 doubles in FP64; in CCX_MODE_MIXED_F16X3 o v^2 (v + o) doubles while the
- * operand is split (half that afterwards, as FP16 hi/lo) + 12 v^3 + 34 v^2 doubles. */
+ * `stream`. Device scratch, one block of
+ *   A   o v^2 (v + o)        B   o^2 v (v + o)        pair blocks   o (o + 1) v^2
+ *   Y   3 v^3 for each of eight triples, but no more than 16 GB (one triple at least), or for as many as 512 MB hold
+ * doubles (v + o rounded up to 8, v to 8 in the pair blocks and to 16 once in Y) and up to 64 MB of partial sums; in
+ * CCX_MODE_MIXED_F16X3 an element of A, B and Y takes 4 bytes (FP16 hi/lo, FP32) and v + o is rounded up to 32. 0.7 GB
+ * at o=11 v=107 and 41 GB at o=48 v=384 in FP64, 23 GB in CCX_MODE_MIXED_F16X3. A block of up to 2 GB stays with the context
+ * for its next call (ccx_device_bytes counts it) and is freed with it; a larger one, and that of a second thread's
+ * call on the context at the same time, is freed before the call returns. */
 int ccx_triples(ccx_ctx* ctx, const double* fock, const double* t1, const double* t2, double* e_dev,
                 void* stream);
 
 /* e_dev[0] += the part of ccx_triples' E(T) from the occupied triples i >= j >= k with
  * i0 <= i < i1 (0 <= i0 <= i1 <= no). Zeroing e_dev[0] and calling it over consecutive ranges that
  * cover [0, no) in ascending order gives ccx_triples' value bit for bit. A long (T) can then report
- * progress, or stop and resume, between ranges. Same modes, scratch and synchronisation as
+ * progress, or stop and resume, between ranges. Same modes, scratch (with i1 for o) and synchronisation as
  * ccx_triples; no counterpart in the reference, whose t_tjl is one call (pycc/cctriples.py:177). */
 int ccx_triples_range(ccx_ctx* ctx, const double* fock, const double* t1, const double* t2, int i0, int i1,
                       double* e_dev, void* stream);
@@ -199,7 +204,9 @@ int ccx_t3_denominator(const double* fock, int64_t nmo, int p, int q, int r, int
  * the ring GEMMs and each whole residual.
  * ccx_timing_start clears and starts recording; ccx_timing_read synchronises, writes
  * out[3*p + {0,1,2}] = {launches, milliseconds, algorithmic flops} for p = 0 (ladder GEMMs),
- * 1 (ring GEMMs), 2 (whole residuals), n <= 9 entries, and stops recording. */
+ * 1 (ring GEMMs), 2 (whole residuals), n <= 9 entries, and stops recording. In FP64 contexts of up to (ov)^2 = 2^22 the
+ * ladder and ring GEMMs otherwise share launches with other terms; while recording they get launches of their own, so
+ * that they can be timed, and a residual takes longer and rounds in another order than one that is not recorded. */
 int ccx_timing_start(ccx_ctx* ctx);
 int ccx_timing_read(ccx_ctx* ctx, double* out, int n);
 

@@ -334,7 +334,8 @@ void ladder_x3(Ctx& c, const double* t1, const double* t2, hipStream_t s);      
 // they read -- amplitudes and integrals, then the intermediates, then G and Hm -- and sums of several terms are taken as
 // partial sums (PartSum), which are independent of each other. One by one the terms of o=5 v=19 are 67 launches of 5 to
 // 10 us; together they are about 25. Where a sum is rounded to FP32 or FP16 operands afterwards (Wmnij and W in the mixed
-// modes, Fae in MIXED_F16X3) its terms are added in the same order in every form.
+// modes, Fae in MIXED_F16X3) its terms are added in the same order in every form. While phases are timed (c.timing) the
+// ladder and ring products keep launches of their own, between their events.
 template <typename T>
 static void residual_t(Ctx& c, const double* F, const double* t1, const double* t2, double* r1,
                        double* r2, hipStream_t s) {
