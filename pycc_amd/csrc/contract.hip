@@ -159,6 +159,16 @@ void contract(T alpha, const TV& A_, const TV& B_, T beta, const TV& C, Workspac
   for (char c : B.lab)
     CCX_CHECK(A.find(c) >= 0 || C.find(c) >= 0, ERR_ARG, std::string("index summed in one operand only: ") + c);
 
+  // No output: nothing to do. An empty sum: one index of extent 0, however many there are and whatever their strides
+  // (below, a class of too many indices is sliced over one that has values).
+  for (const std::vector<Lab>* g : {&gm, &gn, &gb})
+    for (const Lab& l : *g)
+      if (l.ext == 0) return;
+  for (const Lab& l : gk)
+    if (l.ext == 0) {
+      gk = {Lab{l.c, 0, {0, 0, 0}}};
+      break;
+    }
   const std::vector<Lab> om = gm, on = gn, ok = gk, ob = gb;   // before fusion
   fuse(gm, 1 | 4);
   fuse(gn, 2 | 4);

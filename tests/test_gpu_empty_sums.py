@@ -129,3 +129,22 @@ def test_derivatives_with_one_virtual(no, stored):
     j1, j2 = ccsd_jacobian(ref, oh, x1, x2, t2=t2)
     g1, g2 = cc.jvp(_dev(t1), _dev(t2), _dev(x1), _dev(x2), store_vvvv=stored)
     assert _err(g1, j1) < 1e-12 and _err(g2, j2 + j2.transpose(1, 0, 3, 2)) < 1e-12
+
+
+def test_empty_indices_of_any_strides():
+    """Several empty indices whose strides do not nest: an empty output is nothing to do, an empty sum comes as far as its
+    launch."""
+    if torch.cuda.is_available():
+        pytest.skip("a GPU is present")
+    lib, buf = _library(), (ctypes.c_double * 64)()
+    p = ctypes.c_void_p(ctypes.addressof(buf))
+
+    def call(sub, *views):
+        args = [x for shape, strides in views for x in (p, _i64(shape), _i64(strides))]
+        return lib.ccx_contract(sub.encode(), 1.0, *args[:6], 0.5, *args[6:], None)
+
+    assert call("ab,ba->ab", ((0, 0), (5, 1)), ((0, 0), (3, 1)), ((0, 0), (2, 1))) == 0
+    assert call("xab,xba->xab", ((3, 0, 0), (9, 5, 1)), ((3, 0, 0), (8, 3, 1)), ((3, 0, 0), (7, 2, 1))) == 0
+    assert call("abcd,d->cab", ((0, 0, 0, 3), (9, 5, 3, 1)), ((3,), (1,)), ((0, 0, 0), (7, 2, 1))) == 0
+    assert call("abc,cba->", ((0, 0, 0), (5, 3, 1)), ((0, 0, 0), (7, 2, 1)), ((), ())) == -2
+    assert call("abcd,dcba->", ((0, 0, 0, 0), (9, 5, 3, 1)), ((0, 0, 0, 0), (11, 7, 2, 1)), ((), ())) == -2
